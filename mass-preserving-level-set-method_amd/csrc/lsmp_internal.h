@@ -33,13 +33,13 @@ constexpr int RNT = 640;
 static_assert(REX * REY <= RNT, "reinit tile needs one thread per ring cell");
 
 // 3D reinitialisation tile: R3X x R3Y interior cells, one thread each (a
-// 4-wave workgroup); RKC planes per workgroup in z.
+// 4-wave workgroup); at most RKC planes per workgroup in z.
 #ifndef LSMP_R3Y
 #define LSMP_R3Y 8
 #endif
 constexpr int R3X = 32, R3Y = LSMP_R3Y;
 constexpr int P3X = R3X + 8, P3Y = R3Y + 8;
-constexpr int RKC = 32;
+constexpr int RKC = 16;
 // the narrow band's workgroups march RKC_NB planes: a workgroup without a tube
 // cell is skipped, and an active one's march is the kernel's critical path
 constexpr int RKC_NB = 8;

@@ -14,7 +14,7 @@
 // and s3 are zero, so the box sums take band cells only.
 //
 // k_redis3d: a workgroup of R3X*R3Y threads owns an interior tile in (i, j),
-// one cell per thread, and marches over KC planes in k.  Each thread keeps
+// one cell per thread, and marches over kc planes in k.  Each thread keeps
 // its column phi(k-3..k+3) in registers; the current plane, with a 4-cell
 // halo for the x and y stencils, goes to LDS.  The WENO-HJ correction terms
 // of D+ at m and of D- at m+1 are built from the same four second
@@ -33,6 +33,8 @@
 // phi2 = 3/4 phi0 + 1/4 (phi1 - dtau l(phi1)); phi3 = 1/3 phi0 + 2/3 (phi2 - dtau l(phi2)).
 // Stage 3 also reduces max |phi3 - phi0| (:46-62).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "lsmp_device.h"
 #include "lsmp_internal.h"
@@ -88,12 +90,12 @@ template <typename T> LSMP_DEV T load_at(const T *plane_base, unsigned byte_off)
 
 }  // namespace
 
-template <typename T, int STAGE, int BTN, int KC>
+template <typename T, int STAGE, int BTN>
 __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__restrict__ phi_out,
                                                 const T *__restrict__ phi0, const T *__restrict__ S0, RedisArgs ra,
                                                 unsigned long long *ctl, const unsigned char *__restrict__ tiles,
                                                 T *__restrict__ bgr, unsigned *__restrict__ blist,
-                                                unsigned *__restrict__ bcount)
+                                                unsigned *__restrict__ bcount, int kc)
 {
     __shared__ T sphi[P3Y][P3X];
     // D- terms of the x and y faces: column tx (row ty) holds the one of cell tx (ty)
@@ -101,9 +103,9 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     __shared__ T mys[R3Y + 1][R3X];
     static_assert(R3X + R3Y <= 64, "the first faces in one wave");
     // the workgroup's band cells, (plane - k0) * NT + thread, and their count
-    __shared__ unsigned short lcell[BTN == 1 ? KC * NT : 1];
+    __shared__ unsigned short lcell[BTN == 1 ? RKC * NT : 1];
     __shared__ unsigned lcount, lbase;
-    static_assert(KC * NT <= 65536, "local band-cell index in 16 bits");
+    static_assert(RKC * NT <= 65536, "local band-cell index in 16 bits");
     if (ctl[1]) return;   // the pseudo-time loop has stopped (k_redis_ctl)
     const int nx = ra.nx, ny = ra.ny, nz = ra.nz;
     // tiles in x-fastest order, renumbered so that each XCD takes a contiguous
@@ -120,15 +122,15 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         const int ci = bx * R3X + (int)threadIdx.x % R3X, cj = by * R3Y + (int)threadIdx.x / R3X;
         if (ci >= nx || cj >= ny) return;
         const size_t c0 = (size_t)cj * nx + ci, pl = (size_t)nx * ny;
-        for (int k = bz * KC; k < min((bz + 1) * KC, nz); ++k)
+        for (int k = bz * kc; k < min((bz + 1) * kc, nz); ++k)
             phi_out[(size_t)k * pl + c0] = phi[(size_t)k * pl + c0];
         return;
     }
     const T inv12dx = (T)ra.inv12dx, inv12dy = (T)ra.inv12dy, inv12dz = (T)ra.inv12dz;
     const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt, c3 = (T)ra.three;
     const int t = threadIdx.x;
-    const int i0 = bx * R3X, j0 = by * R3Y, k0 = bz * KC;
-    const int k1 = min(k0 + KC, nz);
+    const int i0 = bx * R3X, j0 = by * R3Y, k0 = bz * kc;
+    const int k1 = min(k0 + kc, nz);
     const int tx = t % R3X, ty = t / R3X;
     // cells past the domain edge hold the boundary cell (zero-gradient ghosts)
     const int gi = min(i0 + tx, nx - 1), gj = min(j0 + ty, ny - 1);
@@ -421,31 +423,45 @@ static inline unsigned nb_of(int n, int b) { return (unsigned)((n + b - 1) / b);
 // cell (65536 cells a pass; a longer list takes more passes)
 constexpr unsigned BAND_GRID = 1024;
 
+// Planes a workgroup of the stage kernel marches, for `tiles` (x, y) tiles and
+// nz planes.  A workgroup's march is a serial chain (1.1 us a plane with one
+// workgroup on a CU, 2.6 us with four), so a grid that leaves the device
+// idle is cut into shorter ones: the shortest that still fit one round of
+// resident workgroups (1,024, four per CU).  Per pseudo-step, FP64 (FP32),
+// with 32 planes always and with this rule: 32^3 161 -> 48 us (137 -> 36),
+// 96^3 167 -> 78 (140 -> 57), 128^3 176 -> 109 (150 -> 77), 131x77x101
+// 161 -> 83 (137 -> 65).  Grids of several rounds take 8 planes where the
+// tail of the last round counts (192^3: 238 us, 246 with 16, 274 with 32) and
+// 16 from three rounds of 16 (256^3: 534 us, 550 with 8, 536 with 32), beyond
+// which the three planes of run-up per march cost less than they save.
+static int stage_planes(unsigned tiles, int nz)
+{
+    constexpr int ROUND = 1024;
+    const int blocks = std::max(1, ROUND / (int)tiles);   // blocks in z that fit one round
+    const int one = std::max(1, (nz + blocks - 1) / blocks);
+    if (one <= 8) return one;
+    return (size_t)tiles * nb_of(nz, RKC) >= (size_t)3 * ROUND ? RKC : 8;
+}
+
 template <typename T>
 void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
                     const RedisArgs &ra, unsigned long long *ctl, const unsigned char *tiles, const RedisBand<T> &bd,
                     bool band)
 {
     // the narrow band (tiles) marches RKC_NB planes per workgroup
-    const int kc = tiles ? RKC_NB : RKC;
+    const int kc = tiles ? RKC_NB : stage_planes(nb_of(ra.nx, R3X) * nb_of(ra.ny, R3Y), ra.nz);
     const dim3 g(nb_of(ra.nx, R3X), nb_of(ra.ny, R3Y), nb_of(ra.nz, kc));
-#define LSMP_R3(S, B, KCV)                                                                                     \
+#define LSMP_R3(S, B)                                                                                          \
     do {                                                                                                       \
         if (!band)                                                                                             \
-            hipLaunchKernelGGL((k_redis3d<T, S, B, KCV>), g, dim3(NT), 0, st, phi, phi_out, phi0, S0, ra, ctl, \
-                               tiles, bd.gr, bd.list, bd.count);                                               \
+            hipLaunchKernelGGL((k_redis3d<T, S, B>), g, dim3(NT), 0, st, phi, phi_out, phi0, S0, ra, ctl,      \
+                               tiles, bd.gr, bd.list, bd.count, kc);                                           \
         else if (B == 1)                                                                                       \
             hipLaunchKernelGGL((k_redis3d_band<T, S>), dim3(BAND_GRID), dim3(NT), 0, st, phi, phi_out, phi0,   \
                                S0, ra, ctl, bd.gr, bd.list, bd.count, bd.next);                                \
     } while (0)
-#define LSMP_R3K(S, B)                                                                                         \
-    do {                                                                                                       \
-        if (tiles) LSMP_R3(S, B, RKC_NB);                                                                      \
-        else LSMP_R3(S, B, RKC);                                                                               \
-    } while (0)
-    if (btn) { if (stage == 1) LSMP_R3K(1, 1); else if (stage == 2) LSMP_R3K(2, 1); else LSMP_R3K(3, 1); }
-    else { if (stage == 1) LSMP_R3K(1, 0); else if (stage == 2) LSMP_R3K(2, 0); else LSMP_R3K(3, 0); }
-#undef LSMP_R3K
+    if (btn) { if (stage == 1) LSMP_R3(1, 1); else if (stage == 2) LSMP_R3(2, 1); else LSMP_R3(3, 1); }
+    else { if (stage == 1) LSMP_R3(1, 0); else if (stage == 2) LSMP_R3(2, 0); else LSMP_R3(3, 0); }
 #undef LSMP_R3
 }
 
