@@ -255,53 +255,50 @@ template <typename T> LSMP_DEV T phyn_fast(T a, T b, T c, T d, T sbc, T scd)
     return fma(t0, a - T(2) * b + c, t2 * (b - T(2) * c + d));
 }
 
-// Face m+1/2 of a line with second differences sa = s(m-1), sb = s(m),
-// sc = s(m+1), sd = s(m+2): plus = 12 phyn(sd, sc, sb, sa) (the term of D+
-// at m) and minus = 12 phyn(sa, sb, sc, sd) (the term of D- at m+1), each as
-// phyn_fast evaluates it up to rounding; the factor 12 joins the one of the
-// central part, so that both scale by 1 / (12 dx).  IS0 of one is IS2 of the other,
-// IS1 is common, and so are the products of their squares and the two
-// third differences the terms weigh.  The indicators are the expanded
-// quadratic forms 13 (a - b)^2 + 3 (a - 3b)^2 = 4 (4a^2 - 11ab + 10b^2) and
-// 13 (a - b)^2 + 3 (a + b)^2 = 4 (4a^2 - 5ab + 4b^2) over shared squares,
-// each formed as 4 IS + eps = 40b^2 + (a (16a - 44b) + eps) (and
-// 16a^2 + (b (16b - 20a) + eps)).  With the weights' denominators Dp and
-// Dm, plus = (4 pJB e1 + 6 pAJ e2) / Dp - e2 and minus the same with the
-// roles of the two products and third differences exchanged.
-// FP64 takes both reciprocals from one (the product of the two denominators
-// stays within [1e-48, 1e28]).  three: 3.0.
-template <typename T> LSMP_DEV void weno_hj_face(T sa, T sb, T sc, T sd, T three, T &plus, T &minus)
+// WENO-HJ on a line with second differences s_m = phi(m+1) - 2 phi(m) + phi(m-1)
+// (level_set_rk3_redis.f90:290-315, 456-471), everything times 6 dx:
+//   6 dx D+(m) = b(m) + P(m+1/2),          b(m) = 6 (phi(m+1) - phi(m)) - s(m+1) - 2 s(m),
+//   6 dx D-(m) = b(m) + e(m) - Q(m-1/2),   e(m) = s(m+1) - 2 s(m) + s(m-1),
+// where the central part and the constant -1/2 of the weights are merged into
+// b and b + e (each of third order, one-sided), and P, Q are the weighted third
+// differences of a face, formed together: the indicators of P at m+1/2 and of
+// Q there are those of s(m-1..m+2) in reversed roles.  An indicator plus eps
+// is a sum of two squares,
+//   13 (a - b)^2 + 3 (a - 3b)^2 = 16 ((a - 1.375 b)^2 + 0.609375 b^2),
+//   13 (b - c)^2 + 3 (b + c)^2 = 16 ((b - 0.625 c)^2 + 0.609375 c^2),
+// so that h(s) = 0.609375 s^2 + eps / 16 of the two middle differences serves
+// all three of a face (hj_h; the common factor 16 drops out of the weights).
+template <typename T> LSMP_DEV T hj_h(T s) { return fma(T(0.609375) * s, s, T(1.0e-6 / 16.0)); }
+
+// P and Q of face m+1/2: sa..sd = s(m-1..m+2), hb = hj_h(sb), hc = hj_h(sc),
+// e1 = e(m+1) = sd - 2 sc + sb, e2 = e(m) = sc - 2 sb + sa.  With q the squares of
+// the indicators, P = (2 qJ qB e1 + 3 qA qJ e2) / Dp, Dp = qJ qB + 3 qA qJ +
+// 6 qA qB, and Q the same with A and B, e1 and e2 exchanged.  FP64 takes both
+// reciprocals from one (the product of the two denominators stays within
+// [1e-58, 1e28]); FP32 denominators stay within [1e-28, 1e13].
+template <typename T> LSMP_DEV void weno_hj_face(T sa, T sb, T sc, T sd, T hb, T hc, T e1, T e2, T &P, T &Q)
 {
-    const T eps = T(1.0e-6);
-    const T bb = sb * sb, cc = sc * sc;
-    const T fA = fma(T(40), cc, fma(sd, fma(T(16), sd, T(-44) * sc), eps));   // IS0 of plus, IS2 of minus
-    const T fJ = fma(T(16), bb, fma(sc, fma(T(16), sc, T(-20) * sb), eps));   // IS1 of both
-    const T fB = fma(T(40), bb, fma(sa, fma(T(16), sa, T(-44) * sb), eps));   // IS2 of plus, IS0 of minus
-    const T qA = sq(fA), qJ = sq(fJ), qB = sq(fB);
+    const T tA = fma(T(-1.375), sc, sd), tJ = fma(T(-0.625), sc, sb), tB = fma(T(-1.375), sb, sa);
+    const T qA = sq(fma(tA, tA, hc)), qJ = sq(fma(tJ, tJ, hc)), qB = sq(fma(tB, tB, hb));
     const T pJB = qJ * qB, pAJ = qA * qJ, pAB = qA * qB;
-    // plus: q0 = qA, q1 = qJ, q2 = qB; minus: q0 = qB, q1 = qJ, q2 = qA
-    const T dp = fma(three, fma(T(2), pAB, pAJ), pJB), dm = fma(three, fma(T(2), pAB, pJB), pAJ);
-    T rp, rm;
+    const T w = fma(T(6), pAB, pAJ + pJB);
+    const T dp = fma(T(2), pAJ, w), dm = fma(T(2), pJB, w);
+    const T u1 = pJB * e1, u2 = pAJ * e2, t = u1 + u2;
+    const T yp = fma(T(2), t, u2), ym = fma(T(2), t, u1);
     if constexpr (sizeof(T) == 8) {
         const T r = rcp_w(dp * dm);
-        rp = dm * r;
-        rm = dp * r;
+        P = (dm * r) * yp;
+        Q = (dp * r) * ym;
     } else {
-        rp = rcp_w(dp);
-        rm = rcp_w(dm);
+        P = rcp_w(dp) * yp;
+        Q = rcp_w(dm) * ym;
     }
-    const T e1 = sd - T(2) * sc + sb, e2 = sc - T(2) * sb + sa;
-    const T u1 = pJB * e1, u2 = pAJ * e2;
-    plus = fma(rp, fma(T(4), u1, T(6) * u2), -e2);
-    minus = fma(rm, fma(T(4), u2, T(6) * u1), -e1);
 }
 
-// The central part of the WENO-HJ derivatives times 12 dx,
-// -(m1 - m2) + 7 (c - m1) + 7 (p1 - c) - (p2 - p1), which is
-// (m2 - p2) + 8 (p1 - m1): c drops out.
-template <typename T> LSMP_DEV T central12(T m2, T m1, T p1, T p2)
+// b(m) from phi(m), phi(m+1), s(m), s(m+1)
+template <typename T> LSMP_DEV T hj_base(T c, T p1, T s0, T s1)
 {
-    return fma(T(8), p1 - m1, m2 - p2);
+    return fma(T(-2), s0, fma(T(6), p1 - c, -s1));
 }
 
 // D+ and D- from the five second differences s_m = phi(m+1) - 2 phi(m) + phi(m-1),

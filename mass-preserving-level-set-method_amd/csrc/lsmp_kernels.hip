@@ -732,8 +732,8 @@ template <typename T> LSMP_DEV bool in_band(T x)
 // 2D stage: one tile, no marching (Disk/ and Vortex2D/ forms: |grad| without
 // z, lambda box 3x3 with centre weight 17, Disk/...redis.f90:357-361, 434-438).
 // The tile's RTX x RTY cells and the ring around them (the lambda box) need
-// D+ and D- in x and y.  Each WENO-HJ face m+1/2 gives the D+ term of cell m
-// and the D- term of cell m+1 (weno_hj_face), so the workgroup forms every
+// D+ and D- in x and y.  Each WENO-HJ face m+1/2 gives the P term of cell m
+// and the Q term of cell m+1 (weno_hj_face), so the workgroup forms every
 // face once -- x faces i+1/2 for i = i0-2 .. i0+RTX on the REY ring rows, y
 // faces j+1/2 for j = j0-2 .. j0+RTY on the REX ring columns, two faces a
 // thread -- into LDS, and each cell of the tile and ring reads its four terms
@@ -748,13 +748,13 @@ __global__ __launch_bounds__(RNT) void k_redis_stage2d(const T *__restrict__ phi
                                                        RedisArgs ra, unsigned long long *ctl)
 {
     __shared__ T sphi[RPY][RPX];
-    __shared__ T fplus[R2F], fminus[R2F];   // the faces' D+ and D- terms, times 12
+    __shared__ T fplus[R2F], fminus[R2F];   // P and Q of the faces
     __shared__ T ss2[REY][REX];
     __shared__ T ss3[REY][REX];
     if (ctl[1]) return;   // the pseudo-time loop has stopped (k_redis_ctl)
     const int nx = ra.nx, ny = ra.ny;
-    const T inv12dx = (T)ra.inv12dx, inv12dy = (T)ra.inv12dy;
-    const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt, c3 = (T)ra.three;
+    const T kx = (T)(2.0 * ra.inv12dx), ky = (T)(2.0 * ra.inv12dy);
+    const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt;
     const int t = threadIdx.x;
     const int i0 = blockIdx.x * RTX, j0 = blockIdx.y * RTY;
     const bool ext = t < REX * REY;
@@ -784,11 +784,12 @@ __global__ __launch_bounds__(RNT) void k_redis_stage2d(const T *__restrict__ phi
             const int st = fx ? 1 : RPX;
             const T *v = &sphi[r][c];
             const T vm2 = v[-2 * st], vm1 = v[-st], v0 = v[0], vp1 = v[st], vp2 = v[2 * st], vp3 = v[3 * st];
-            T plus, minus;
-            weno_hj_face(vm2 - T(2) * vm1 + v0, vm1 - T(2) * v0 + vp1, v0 - T(2) * vp1 + vp2,
-                         vp1 - T(2) * vp2 + vp3, c3, plus, minus);
-            fplus[f] = plus;
-            fminus[f] = minus;
+            const T sa = vm2 - T(2) * vm1 + v0, sb = vm1 - T(2) * v0 + vp1, sc = v0 - T(2) * vp1 + vp2,
+                    sd = vp1 - T(2) * vp2 + vp3;
+            T P, Q;
+            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, sc - T(2) * sb + sa, P, Q);
+            fplus[f] = P;
+            fminus[f] = Q;
         }
     }
     __syncthreads();
@@ -806,10 +807,17 @@ __global__ __launch_bounds__(RNT) void k_redis_stage2d(const T *__restrict__ phi
         // cy (RTX + 3) + cx (+ 1), its y faces j -/+ 1/2 y faces cy REX + cx (+ REX)
         const int cx = gi - i0 + 1, cy = gj - j0 + 1;
         const int fxm = cy * (RTX + 3) + cx, fym = R2FX + cy * REX + cx;
-        const T ax = inv12dx * central12(sphi[pr][pc - 2], sphi[pr][pc - 1], sphi[pr][pc + 1], sphi[pr][pc + 2]);
-        const T ay = inv12dy * central12(sphi[pr - 2][pc], sphi[pr - 1][pc], sphi[pr + 1][pc], sphi[pr + 2][pc]);
-        const T xs1 = ax + inv12dx * fplus[fxm + 1], xs2 = ax - inv12dx * fminus[fxm];
-        const T ys1 = ay + inv12dy * fplus[fym + REX], ys2 = ay - inv12dy * fminus[fym];
+        auto slopes = [&](int st, T k, T P, T Q, T &dp, T &dm) {
+            const T *v = &sphi[pr][pc];
+            const T sa = v[-2 * st] - T(2) * v[-st] + c0, sb = v[-st] - T(2) * c0 + v[st],
+                    sc = c0 - T(2) * v[st] + v[2 * st];
+            const T b6 = hj_base(c0, v[st], sb, sc);
+            dp = k * (b6 + P);
+            dm = k * ((b6 + (sc - T(2) * sb + sa)) - Q);
+        };
+        T xs1, xs2, ys1, ys2;
+        slopes(1, kx, fplus[fxm + 1], fminus[fxm], xs1, xs2);
+        slopes(RPX, ky, fplus[fym + REX], fminus[fym], ys1, ys2);
         grad_p = godunov<T, 2>(xs1, xs2, ys1, ys2, T(0), T(0), s0_p);
         phi_p = c0;
         if (BTN == 1) {

@@ -15,18 +15,22 @@
 //
 // k_redis3d: a workgroup of R3X*R3Y threads owns an interior tile in (i, j),
 // one cell per thread, and marches over kc planes in k.  Each thread keeps
-// its column phi(k-3..k+3) in registers; the current plane, with a 4-cell
-// halo for the x and y stencils, goes to LDS.  The WENO-HJ correction terms
-// of D+ at m and of D- at m+1 are built from the same four second
-// differences s(m-1..m+2) and share their smoothness indicators, their
-// squares and the pairwise products of those (in reversed roles), so each
-// direction evaluates one face m+1/2 per cell.  z: each plane evaluates face
-// p+1/2 and carries its D- term and the second differences to the next
-// plane.  x and y: each thread evaluates the faces i+1/2 and j+1/2 of its
-// cell and hands the D- terms to its neighbours through LDS; one wave (a
-// different one from tile to tile) also evaluates the tile's first faces
-// i0-1/2 and j0-1/2.  Two barriers per
-// plane: the plane is in LDS, the D- terms are.
+// its column phi(k..k+3) in registers; the current plane, with a 4-cell
+// halo for the x and y stencils, goes to LDS.  The weighted third differences
+// of D+ at m (P) and of D- at m+1 (Q) are built from the same four second
+// differences s(m-1..m+2) (weno_hj_face), so each direction evaluates one
+// face m+1/2 per cell.  z: each plane evaluates face p+1/2 and carries its Q,
+// the second and fourth differences and h(s) to the next plane.  x and y:
+// each thread evaluates the faces i+1/2 and j+1/2 of its cell and hands the Q
+// terms to its neighbours through LDS; one wave (a different one from tile to
+// tile) also evaluates the tile's first faces i0-1/2 and j0-1/2.  Two barriers
+// per plane: the plane is in LDS, the Q terms are.
+//
+// Bound by VALU issue and HBM together: 210 VALU instructions per plane and
+// thread, 158 of them FP64 (233 and 186 with the indicators as expanded
+// quadratic forms and a central part beside the face terms).  256^3, per
+// pseudo-step of three stages and band passes: FP64 534 -> 506 us, FP32 302 ->
+// 271 us (79 VGPRs instead of 89: six waves per SIMD instead of five).
 //
 // The RK stage is written in Shu-Osher form, algebraically identical to the
 // reference's increments: phi1 = phi0 - dtau l(phi0);
@@ -63,15 +67,18 @@ template <typename T> LSMP_DEV bool in_band_x(T x)
     return !(x > T(1) - T(1.0e-12)) && !(x < T(-1) + T(1.0e-12));
 }
 
-// Godunov |grad phi| (level_set_rk3_redis.f90:341-360): with sigma the sign of
+// Godunov |grad phi| (level_set_rk3_redis.f90:341-360) from the one-sided
+// slopes times 6 dx, 6 dy, 6 dz; k = 1 / (6 dx), ...: with sigma the sign of
 // S0, max(-min(D+, 0), max(D-, 0)) is max(-sigma D+, sigma D-, 0) per direction
-// (and max(max(D+, 0), -min(D-, 0)) the same with sigma = -1).
-template <typename T> LSMP_DEV T godunov_sig(T xp, T xm, T yp, T ym, T zp, T zm, T s0)
+// (and max(max(D+, 0), -min(D-, 0)) the same with sigma = -1).  Where S0 is a
+// zero of either sign the pseudo-time right-hand side S0 (|grad| - 1) is zero.
+template <typename T>
+LSMP_DEV T godunov_sig(T xp, T xm, T yp, T ym, T zp, T zm, T s0, T kx, T ky, T kz)
 {
-    const T sg = s0 >= T(0) ? T(1) : T(-1);
-    const T gx = fmax(fmax(-(sg * xp), sg * xm), T(0));
-    const T gy = fmax(fmax(-(sg * yp), sg * ym), T(0));
-    const T gz = fmax(fmax(-(sg * zp), sg * zm), T(0));
+    const T sx = copysign(kx, s0), sy = copysign(ky, s0), sz = copysign(kz, s0);
+    const T gx = fmax(fmax(-(sx * xp), sx * xm), T(0));
+    const T gy = fmax(fmax(-(sy * yp), sy * ym), T(0));
+    const T gz = fmax(fmax(-(sz * zp), sz * zm), T(0));
     return sqrt_w(sq(gx) + sq(gy) + sq(gz));
 }
 
@@ -98,7 +105,7 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
                                                 unsigned *__restrict__ bcount, int kc)
 {
     __shared__ T sphi[P3Y][P3X];
-    // D- terms of the x and y faces: column tx (row ty) holds the one of cell tx (ty)
+    // Q of the x and y faces: column tx (row ty) holds the one of cell tx (ty)
     __shared__ T mxs[R3Y][R3X + 1];
     __shared__ T mys[R3Y + 1][R3X];
     static_assert(R3X + R3Y <= 64, "the first faces in one wave");
@@ -126,8 +133,8 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
             phi_out[(size_t)k * pl + c0] = phi[(size_t)k * pl + c0];
         return;
     }
-    const T inv12dx = (T)ra.inv12dx, inv12dy = (T)ra.inv12dy, inv12dz = (T)ra.inv12dz;
-    const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt, c3 = (T)ra.three;
+    const T kx = (T)(2.0 * ra.inv12dx), ky = (T)(2.0 * ra.inv12dy), kz = (T)(2.0 * ra.inv12dz);
+    const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt;
     const int t = threadIdx.x;
     const int i0 = bx * R3X, j0 = by * R3Y, k0 = bz * kc;
     const int k1 = min(k0 + kc, nz);
@@ -160,20 +167,27 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     const int f_off = first_x ? (fu + 4) * P3X + 1 : (first_y ? P3X + 4 + (fu - R3Y) : 0);
     const int f_str = first_x ? 1 : P3X;
 
-    T w[7];   // phi(p-3 .. p+3) of this cell's column
-#pragma unroll
-    for (int d = 0; d < 7; ++d) w[d] = load_at(base(phi, k0 - 3 + d), col);
-    // z: second differences s(k0-1), s(k0), s(k0+1) and the D- term of the
-    // first plane (its face k0 - 1/2)
-    T za = w[0] - T(2) * w[1] + w[2];   // s(k0 - 2)
-    T zb = w[1] - T(2) * w[2] + w[3];   // s(k0 - 1)
-    T zc = w[2] - T(2) * w[3] + w[4];   // s(k0)
-    T zminus;
+    T w0, w1, w2, w3;   // phi(p .. p+3) of this cell's column
+    // z: second differences s(p-1), s(p), s(p+1), h(s(p)), e(p) and Q of face
+    // p - 1/2, carried from plane to plane
+    T za, zb, zc, zhb, ze, zq;
     {
+        T v[7];   // phi(k0-3 .. k0+3)
+#pragma unroll
+        for (int d = 0; d < 7; ++d) v[d] = load_at(base(phi, k0 - 3 + d), col);
+        const T s2 = v[0] - T(2) * v[1] + v[2], s1 = v[1] - T(2) * v[2] + v[3];   // s(k0-2), s(k0-1)
+        const T s0 = v[2] - T(2) * v[3] + v[4], sp = v[3] - T(2) * v[4] + v[5];   // s(k0), s(k0+1)
+        za = s1;
+        zb = s0;
+        zc = sp;
+        zhb = hj_h(zb);
+        ze = zc - T(2) * zb + za;
         T unused;
-        const T zd = w[3] - T(2) * w[4] + w[5];   // s(k0 + 1)
-        weno_hj_face(za, zb, zc, zd, c3, unused, zminus);
-        za = zb; zb = zc; zc = zd;
+        weno_hj_face(s2, s1, s0, sp, hj_h(s1), zhb, ze, s0 - T(2) * s1 + s2, unused, zq);
+        w0 = v[3];
+        w1 = v[4];
+        w2 = v[5];
+        w3 = v[6];
     }
     T halo_cur = halo ? load_at(base(phi, k0), hcol) : T(0);
     T halo2_cur = halo2 ? load_at(base(phi, k0), hcol2) : T(0);
@@ -191,58 +205,64 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         const T p0_cur = STAGE > 1 ? load_at(base(phi0, p), col) : T(0);
 
         // the previous plane's readers have passed its second barrier
-        sphi[ty + 4][tx + 4] = w[3];
+        sphi[ty + 4][tx + 4] = w0;
         if (halo) sphi[hr][hc] = halo_cur;
         if (halo2) sphi[hr2][hc2] = halo2_cur;
 
-        // z face p + 1/2: its D+ term is this plane's, its D- term the next one's
-        const T zs_new = w[4] - T(2) * w[5] + w[6];   // s(p + 2)
-        T zplus, zminus_next;
-        weno_hj_face(za, zb, zc, zs_new, c3, zplus, zminus_next);
-        const T az = inv12dz * central12(w[1], w[2], w[4], w[5]);
-        const T zs1 = az + inv12dz * zplus, zs2 = az - inv12dz * zminus;
+        // z face p + 1/2: P is this plane's, Q the next one's
+        const T zs_new = w1 - T(2) * w2 + w3;   // s(p + 2)
+        const T zhc = hj_h(zc), ze_next = zs_new - T(2) * zc + zb;
+        T zp, zq_next;
+        weno_hj_face(za, zb, zc, zs_new, zhb, zhc, ze_next, ze, zp, zq_next);
+        const T bz6 = hj_base(w0, w1, zb, zc);
+        const T zs1 = bz6 + zp, zs2 = (bz6 + ze) - zq;
         __syncthreads();
-        // x face i+1/2: D+ term of this cell, D- term of cell i+1
-        T xs1, ax, ys1, ay;
+        // x face i+1/2: P of this cell, Q of cell i+1
+        T xs1, xs2, ys1, ys2;
         {
             const T *r = &sphi[ty + 4][tx + 4];
-            const T m2 = r[-2], m1 = r[-1], c = w[3], p1 = r[1], p2 = r[2], p3 = r[3];
-            ax = inv12dx * central12(m2, m1, p1, p2);
-            T plus, minus;
-            weno_hj_face(m2 - T(2) * m1 + c, m1 - T(2) * c + p1, c - T(2) * p1 + p2, p1 - T(2) * p2 + p3, c3,
-                         plus, minus);
-            xs1 = ax + inv12dx * plus;
-            mxs[ty][tx + 1] = minus;
+            const T m2 = r[-2], m1 = r[-1], c = w0, p1 = r[1], p2 = r[2], p3 = r[3];
+            const T sa = m2 - T(2) * m1 + c, sb = m1 - T(2) * c + p1, sc = c - T(2) * p1 + p2, sd = p1 - T(2) * p2 + p3;
+            const T e2 = sc - T(2) * sb + sa;
+            T P, Q;
+            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
+            mxs[ty][tx + 1] = Q;
+            const T b6 = hj_base(c, p1, sb, sc);
+            xs1 = b6 + P;
+            xs2 = b6 + e2;
         }
         // y face j+1/2
         {
             const T *r = &sphi[ty + 4][tx + 4];
-            const T m2 = r[-2 * P3X], m1 = r[-P3X], c = w[3], p1 = r[P3X], p2 = r[2 * P3X], p3 = r[3 * P3X];
-            ay = inv12dy * central12(m2, m1, p1, p2);
-            T plus, minus;
-            weno_hj_face(m2 - T(2) * m1 + c, m1 - T(2) * c + p1, c - T(2) * p1 + p2, p1 - T(2) * p2 + p3, c3,
-                         plus, minus);
-            ys1 = ay + inv12dy * plus;
-            mys[ty + 1][tx] = minus;
+            const T m2 = r[-2 * P3X], m1 = r[-P3X], c = w0, p1 = r[P3X], p2 = r[2 * P3X], p3 = r[3 * P3X];
+            const T sa = m2 - T(2) * m1 + c, sb = m1 - T(2) * c + p1, sc = c - T(2) * p1 + p2, sd = p1 - T(2) * p2 + p3;
+            const T e2 = sc - T(2) * sb + sa;
+            T P, Q;
+            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
+            mys[ty + 1][tx] = Q;
+            const T b6 = hj_base(c, p1, sb, sc);
+            ys1 = b6 + P;
+            ys2 = b6 + e2;
         }
         if (first_x || first_y) {
             const T *f = &sphi[0][0] + f_off;
             const T v0 = f[0], v1 = f[f_str], v2 = f[2 * f_str], v3 = f[3 * f_str], v4 = f[4 * f_str],
                     v5 = f[5 * f_str];
-            T plus, minus;
-            weno_hj_face(v0 - T(2) * v1 + v2, v1 - T(2) * v2 + v3, v2 - T(2) * v3 + v4, v3 - T(2) * v4 + v5, c3,
-                         plus, minus);
-            if (first_x) mxs[fu][0] = minus;
-            else mys[0][fu - R3Y] = minus;
+            const T sa = v0 - T(2) * v1 + v2, sb = v1 - T(2) * v2 + v3, sc = v2 - T(2) * v3 + v4,
+                    sd = v3 - T(2) * v4 + v5;
+            T P, Q;
+            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, sc - T(2) * sb + sa, P, Q);
+            if (first_x) mxs[fu][0] = Q;
+            else mys[0][fu - R3Y] = Q;
         }
         __syncthreads();
-        const T xs2 = ax - inv12dx * mxs[ty][tx];
-        const T ys2 = ay - inv12dy * mys[ty][tx];
-        const T grad = godunov_sig(xs1, xs2, ys1, ys2, zs1, zs2, s0_cur);
+        xs2 = xs2 - mxs[ty][tx];
+        ys2 = ys2 - mys[ty][tx];
+        const T grad = godunov_sig(xs1, xs2, ys1, ys2, zs1, zs2, s0_cur, kx, ky, kz);
         // lambda = 0: final off the band, replaced by k_redis3d_band on it
         const T l = s0_cur * grad - s0_cur;
-        const T pn = rk_stage<T, STAGE>(w[3], p0_cur, l, rdt);
-        const bool band = BTN == 1 && inner && in_band_x(w[3] * inv_w);
+        const T pn = rk_stage<T, STAGE>(w0, p0_cur, l, rdt);
+        const bool band = BTN == 1 && inner && in_band_x(w0 * inv_w);
         if (inner) {
             const size_t off = (size_t)p * plane;
             *reinterpret_cast<T *>(reinterpret_cast<char *>(phi_out + off) + col) = pn;
@@ -265,11 +285,16 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
                         (unsigned short)((p - k0) * NT + t);
             }
         }
-#pragma unroll
-        for (int d = 0; d < 6; ++d) w[d] = w[d + 1];
-        w[6] = w_next;
-        za = zb; zb = zc; zc = zs_new;
-        zminus = zminus_next;
+        w0 = w1;
+        w1 = w2;
+        w2 = w3;
+        w3 = w_next;
+        za = zb;
+        zb = zc;
+        zc = zs_new;
+        zhb = zhc;
+        ze = ze_next;
+        zq = zq_next;
         halo_cur = halo_next;
         halo2_cur = halo2_next;
     }
