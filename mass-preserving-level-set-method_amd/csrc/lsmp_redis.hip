@@ -26,11 +26,20 @@
 // tile) also evaluates the tile's first faces i0-1/2 and j0-1/2.  Two barriers
 // per plane: the plane is in LDS, the Q terms are.
 //
-// Bound by VALU issue and HBM together: 210 VALU instructions per plane and
-// thread, 158 of them FP64 (233 and 186 with the indicators as expanded
-// quadratic forms and a central part beside the face terms).  256^3, per
-// pseudo-step of three stages and band passes: FP64 534 -> 506 us, FP32 302 ->
-// 271 us (79 VGPRs instead of 89: six waves per SIMD instead of five).
+// Bound by FP64 issue: 205 VALU instructions per plane and thread, 158 of them
+// FP64, are 100 us of the 143 us a 256^3 stage takes (2.05 ns per FP64
+// instruction and SIMD measured alone; reading S0 as two bits a cell, a
+// quarter of the traffic, changes nothing).  256^3, per pseudo-step of three
+// stages and band passes, FP64 (FP32):
+//   534 us (302)  indicators as expanded quadratic forms, a central part beside
+//                 the face terms
+//   506 us (271)  the forms of weno_hj_face
+//   494 us (269)  no plane waits for its own loads or the last plane's stores
+//                 (one wait a plane, before its stores)
+//   480 us (250)  plane addresses in scalar registers, the LDS arrays on one row
+//                 length, four planes a loop trip (no register moves): 106
+//                 VGPRs instead of 122 (FP32 60 instead of 78: eight waves per
+//                 SIMD).  A fifth FP64 wave per SIMD spills and runs slower.
 //
 // The RK stage is written in Shu-Osher form, algebraically identical to the
 // reference's increments: phi1 = phi0 - dtau l(phi0);
@@ -90,10 +99,27 @@ template <typename T, int STAGE> LSMP_DEV T rk_stage(T phi_c, T p0, T l, T rdt)
     return p0 * T(1.0 / 3.0) + T(2.0 / 3.0) * (phi_c - rdt * l);
 }
 
+// Element of a plane at a byte offset: the plane's address, the same in every
+// lane, stays in scalar registers and the offset in one vector register (the
+// empty statements, here and on the offsets in the plane loop, keep the
+// compiler from adding the two into a vector pair per field: two registers
+// and an addition per access).
+template <typename T> using global_ptr = __attribute__((address_space(1))) T *;
 template <typename T> LSMP_DEV T load_at(const T *plane_base, unsigned byte_off)
 {
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(plane_base) + byte_off);
+    unsigned long long b = (unsigned long long)plane_base;
+    asm("" : "+s"(b));
+    return *(global_ptr<const T>)((global_ptr<const char>)b + byte_off);
 }
+template <typename T> LSMP_DEV void store_at(T *plane_base, unsigned byte_off, T v)
+{
+    unsigned long long b = (unsigned long long)plane_base;
+    asm("" : "+s"(b));
+    *(global_ptr<T>)((global_ptr<char>)b + byte_off) = v;
+}
+
+// s_waitcnt vmcnt(0): the wave's loads and stores issued so far are done
+LSMP_DEV void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 }  // namespace
 
@@ -104,10 +130,11 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
                                                 T *__restrict__ bgr, unsigned *__restrict__ blist,
                                                 unsigned *__restrict__ bcount, int kc)
 {
-    __shared__ T sphi[P3Y][P3X];
-    // Q of the x and y faces: column tx (row ty) holds the one of cell tx (ty)
-    __shared__ T mxs[R3Y][R3X + 1];
-    __shared__ T mys[R3Y + 1][R3X];
+    // rows of P3X slots: the plane with its halo, then Q of the x faces (row ty,
+    // slot tx: of cell tx), then Q of the y faces (row ty: of cell ty).  One row
+    // length for all three, so that a thread's places in them differ by constants.
+    __shared__ T lds[(P3Y + R3Y + R3Y + 1) * P3X];
+    constexpr int MX = P3Y * P3X, MY = (P3Y + R3Y) * P3X;
     static_assert(R3X + R3Y <= 64, "the first faces in one wave");
     // the workgroup's band cells, (plane - k0) * NT + thread, and their count
     __shared__ unsigned short lcell[BTN == 1 ? RKC * NT : 1];
@@ -149,10 +176,10 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     // byte offsets within a plane (a plane holds fewer than 2^28 cells); the
     // plane bases are uniform over the workgroup
     const size_t plane = (size_t)nx * ny;
-    const unsigned col = ((unsigned)gj * nx + gi) * (unsigned)sizeof(T);
-    const unsigned hcol = ((unsigned)clampi(j0 - 4 + hr, 0, ny - 1) * nx + clampi(i0 - 4 + hc, 0, nx - 1)) *
+    unsigned col = ((unsigned)gj * nx + gi) * (unsigned)sizeof(T);
+    unsigned hcol = ((unsigned)clampi(j0 - 4 + hr, 0, ny - 1) * nx + clampi(i0 - 4 + hc, 0, nx - 1)) *
                           (unsigned)sizeof(T);
-    const unsigned hcol2 = ((unsigned)clampi(j0 - 4 + hr2, 0, ny - 1) * nx + clampi(i0 - 4 + hc2, 0, nx - 1)) *
+    unsigned hcol2 = ((unsigned)clampi(j0 - 4 + hr2, 0, ny - 1) * nx + clampi(i0 - 4 + hc2, 0, nx - 1)) *
                            (unsigned)sizeof(T);
     auto base = [&](const T *f, int p) { return f + (size_t)clampi(p, 0, nz - 1) * plane; };
 
@@ -164,8 +191,11 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     // tile, so that the extra work spreads over the SIMDs of a CU
     const int fu = t - 64 * (tile_id % (NT / 64));
     const bool first_x = fu >= 0 && fu < R3Y, first_y = fu >= R3Y && fu < R3Y + R3X;
-    const int f_off = first_x ? (fu + 4) * P3X + 1 : (first_y ? P3X + 4 + (fu - R3Y) : 0);
-    const int f_str = first_x ? 1 : P3X;
+    int f_off = first_x ? (fu + 4) * P3X + 1 : (first_y ? P3X + 4 + (fu - R3Y) : 0);
+    int f_dst = first_x ? MX + fu * P3X : MY + (first_y ? fu - R3Y : 0);
+    int f_str = first_x ? 1 : P3X;
+    const int own = ty * P3X + tx;   // the thread's cell, less 4 rows and 4 slots of halo
+    T *const hdst = &lds[hr * P3X + hc], *const hdst2 = &lds[hr2 * P3X + hc2];
 
     T w0, w1, w2, w3;   // phi(p .. p+3) of this cell's column
     // z: second differences s(p-1), s(p), s(p+1), h(s(p)), e(p) and Q of face
@@ -192,10 +222,14 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     T halo_cur = halo ? load_at(base(phi, k0), hcol) : T(0);
     T halo2_cur = halo2 ? load_at(base(phi, k0), hcol2) : T(0);
     if (BTN == 1 && t == 0) lcount = 0;   // read after the loop's first barrier
-    double lerr = 0.0;
-    for (int pl = k0; pl < k1; ++pl) {
+    T lerr = T(0);
+    // every load of the run-up is in, so that no plane waits for its own loads
+    // where the loop's first entry would have to
+    wait_loads();
+    auto one_plane = [&](int pl) {
         // the plane index is the same in every lane: plane addresses are scalar
         const int p = __builtin_amdgcn_readfirstlane(pl);
+        asm("" : "+v"(col), "+v"(hcol), "+v"(hcol2));
         // next plane's inputs, in flight while this one is computed
         const T w_next = load_at(base(phi, p + 4), col);
         const T halo_next = halo ? load_at(base(phi, p + 1), hcol) : T(0);
@@ -205,9 +239,9 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         const T p0_cur = STAGE > 1 ? load_at(base(phi0, p), col) : T(0);
 
         // the previous plane's readers have passed its second barrier
-        sphi[ty + 4][tx + 4] = w0;
-        if (halo) sphi[hr][hc] = halo_cur;
-        if (halo2) sphi[hr2][hc2] = halo2_cur;
+        lds[own + 4 * P3X + 4] = w0;
+        if (halo) *hdst = halo_cur;
+        if (halo2) *hdst2 = halo2_cur;
 
         // z face p + 1/2: P is this plane's, Q the next one's
         const T zs_new = w1 - T(2) * w2 + w3;   // s(p + 2)
@@ -220,68 +254,76 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         // x face i+1/2: P of this cell, Q of cell i+1
         T xs1, xs2, ys1, ys2;
         {
-            const T *r = &sphi[ty + 4][tx + 4];
+            const T *r = &lds[own + 4 * P3X + 4];
             const T m2 = r[-2], m1 = r[-1], c = w0, p1 = r[1], p2 = r[2], p3 = r[3];
             const T sa = m2 - T(2) * m1 + c, sb = m1 - T(2) * c + p1, sc = c - T(2) * p1 + p2, sd = p1 - T(2) * p2 + p3;
             const T e2 = sc - T(2) * sb + sa;
             T P, Q;
             weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
-            mxs[ty][tx + 1] = Q;
+            lds[MX + own + 1] = Q;
             const T b6 = hj_base(c, p1, sb, sc);
             xs1 = b6 + P;
             xs2 = b6 + e2;
         }
         // y face j+1/2
         {
-            const T *r = &sphi[ty + 4][tx + 4];
+            const T *r = &lds[own + 4 * P3X + 4];
             const T m2 = r[-2 * P3X], m1 = r[-P3X], c = w0, p1 = r[P3X], p2 = r[2 * P3X], p3 = r[3 * P3X];
             const T sa = m2 - T(2) * m1 + c, sb = m1 - T(2) * c + p1, sc = c - T(2) * p1 + p2, sd = p1 - T(2) * p2 + p3;
             const T e2 = sc - T(2) * sb + sa;
             T P, Q;
             weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
-            mys[ty + 1][tx] = Q;
+            lds[MY + own + P3X] = Q;
             const T b6 = hj_base(c, p1, sb, sc);
             ys1 = b6 + P;
             ys2 = b6 + e2;
         }
         if (first_x || first_y) {
-            const T *f = &sphi[0][0] + f_off;
+            asm("" : "+v"(f_off), "+v"(f_str), "+v"(f_dst));   // addresses formed here, not kept
+            const T *f = &lds[f_off];
             const T v0 = f[0], v1 = f[f_str], v2 = f[2 * f_str], v3 = f[3 * f_str], v4 = f[4 * f_str],
                     v5 = f[5 * f_str];
             const T sa = v0 - T(2) * v1 + v2, sb = v1 - T(2) * v2 + v3, sc = v2 - T(2) * v3 + v4,
                     sd = v3 - T(2) * v4 + v5;
             T P, Q;
             weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, sc - T(2) * sb + sa, P, Q);
-            if (first_x) mxs[fu][0] = Q;
-            else mys[0][fu - R3Y] = Q;
+            lds[f_dst] = Q;
         }
         __syncthreads();
-        xs2 = xs2 - mxs[ty][tx];
-        ys2 = ys2 - mys[ty][tx];
+        xs2 = xs2 - lds[MX + own];
+        ys2 = ys2 - lds[MY + own];
         const T grad = godunov_sig(xs1, xs2, ys1, ys2, zs1, zs2, s0_cur, kx, ky, kz);
         // lambda = 0: final off the band, replaced by k_redis3d_band on it
         const T l = s0_cur * grad - s0_cur;
         const T pn = rk_stage<T, STAGE>(w0, p0_cur, l, rdt);
         const bool band = BTN == 1 && inner && in_band_x(w0 * inv_w);
+        // the next plane's inputs are in before this plane's stores go out:
+        // a later wait for them would wait for the stores as well
+        wait_loads();
         if (inner) {
             const size_t off = (size_t)p * plane;
-            *reinterpret_cast<T *>(reinterpret_cast<char *>(phi_out + off) + col) = pn;
+            unsigned at = col;
+            asm("" : "+v"(at));
+            store_at(phi_out + off, at, pn);
             if (band) {
-                bgr[off + col / sizeof(T)] = grad;
+                asm("" : "+v"(at));
+                store_at(bgr + off, at, grad);
             } else if (STAGE == 3) {
-                lerr = fmax(lerr, (double)fabs(pn - p0_cur));
+                lerr = fmax(lerr, fabs(pn - p0_cur));
             }
         }
         if (BTN == 1) {
             // list this plane's band cells in LDS: one LDS atomic per wave
             const unsigned long long vote = __ballot(band);
             if (vote) {
-                const int lane = t & 63, lead = __ffsll((long long)vote) - 1;
+                const unsigned below = __builtin_amdgcn_mbcnt_hi((unsigned)(vote >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)vote, 0u));
+                const int lead = __ffsll((long long)vote) - 1;
                 unsigned at = 0;
-                if (lane == lead) at = atomicAdd(&lcount, (unsigned)__popcll(vote));
-                at = __shfl(at, lead, 64);
+                if (band && below == 0) at = atomicAdd(&lcount, (unsigned)__popcll(vote));
+                at = __builtin_amdgcn_readlane(at, lead);
                 if (band)
-                    lcell[at + (unsigned)__popcll(vote & ((1ull << lane) - 1ull))] =
+                    lcell[at + below] =
                         (unsigned short)((p - k0) * NT + t);
             }
         }
@@ -297,6 +339,17 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         zq = zq_next;
         halo_cur = halo_next;
         halo2_cur = halo2_next;
+    };
+    // four planes a trip: the carried values then need no moves
+    for (int pl = k0;;) {
+        one_plane(pl);
+        if (++pl >= k1) break;
+        one_plane(pl);
+        if (++pl >= k1) break;
+        one_plane(pl);
+        if (++pl >= k1) break;
+        one_plane(pl);
+        if (++pl >= k1) break;
     }
     if (BTN == 1) {
         // the workgroup's list onto the device list: one atomic
@@ -314,7 +367,7 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         }
     }
     if (STAGE == 3) {
-        double m = block_max(lerr);
+        double m = block_max((double)lerr);
         if (t == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, (unsigned)tile_id), m);
     }
 }
