@@ -44,8 +44,8 @@ struct lsmp_ctx {
     int last_lines[3] = {-1, -1, -1};  // listed lines of the last mass correction
     double nb_cells = 0.0;             // narrow band half-width in cells (0: off)
     unsigned char *tiles = nullptr;    // narrow band: 3D reinitialisation workgroups holding a tube cell
-    // 3D reinitialisation, band cells: |grad| side field, the list of band
-    // cells and its two lengths, used by turns (allocated on the first btn = 1
+    // 3D reinitialisation, band cells: side fields (|grad|, s2, s3), the list of
+    // band cells and its two lengths, used by turns (allocated on the first btn = 1
     // reinitialisation); rb_count[rb_par] is zero between stages
     void *rb_gr = nullptr;
     unsigned *rb_list = nullptr, *rb_count = nullptr;

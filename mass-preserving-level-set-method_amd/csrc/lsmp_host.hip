@@ -427,13 +427,14 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
     RedisBand<T> bd;
     if (c->dim == 3 && btn == 1) {
         if (!c->rb_list) {
-            if (alloc(&c->rb_gr, c->ncell * c->esz) || alloc((void **)&c->rb_list, c->ncell * sizeof(unsigned)) ||
+            if (alloc(&c->rb_gr, 3 * c->ncell * c->esz) || alloc((void **)&c->rb_list, c->ncell * sizeof(unsigned)) ||
                 alloc((void **)&c->rb_count, 2 * sizeof(unsigned)))
                 return LSMP_E_HIP;
             launch_zero_bytes(c->st, (unsigned char *)c->rb_count, 2 * sizeof(unsigned));
             c->rb_par = 0;
         }
-        bd.gr = (T *)c->rb_gr;
+        T *const f = (T *)c->rb_gr;
+        bd.f = BandFields<T>{f, f + c->ncell, f + 2 * c->ncell};
         bd.list = c->rb_list;
     }
     launch_redis_ctl(c->st, ctl, 0);

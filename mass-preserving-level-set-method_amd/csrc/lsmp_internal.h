@@ -107,12 +107,16 @@ template <typename T>
 void launch_tube_tiles(hipStream_t st, const T *phi, int nx, int ny, int nz, double wband, unsigned char *tiles);
 // 3D reinitialisation stage (lsmp_redis.hip): band = false launches the pass
 // over every cell with lambda = 0, band = true (btn = 1 only) the pass over the
-// listed band cells with lambda.  gr holds |grad| of the band cells, list
+// listed band cells with lambda.  f holds |grad|, s2 and s3 of the band cells
+// (a cell off the band keeps what an earlier stage left there), list
 // their cell indices (room for every cell); count is the list's length for
 // this stage (zero when the stage starts) and next the one for the next
 // stage, which the band pass clears.
+template <typename T> struct BandFields {
+    T *gr = nullptr, *s2 = nullptr, *s3 = nullptr;
+};
 template <typename T> struct RedisBand {
-    T *gr = nullptr;
+    BandFields<T> f;
     unsigned *list = nullptr, *count = nullptr, *next = nullptr;
 };
 template <typename T>

@@ -4,13 +4,13 @@
 //
 // k_redis3d updates every cell of the domain with lambda = 0.  That is the
 // final value wherever delta = 0 (lambda is multiplied by delta), i.e. outside
-// the band |phi| < ls_wid.  For the cells inside it, it also stores |grad| in
-// a side field and lists the cell: first in the workgroup's list in LDS,
+// the band |phi| < ls_wid.  For the cells inside it, it also stores |grad|,
+// s2 = delta S0 (|grad| - 1) and s3 = |grad| delta^2 in side fields and lists the cell: first in the workgroup's list in LDS,
 // which the workgroup appends to the device list with one atomic at its end.
 // k_redis3d_band then takes the listed cells, four lanes per cell over the
-// whole device, forms s2 = delta S0 (|grad| - 1) and s3 = |grad| delta^2 of each
-// band cell of the 3x3x3 box around it, lambda from their sums (centre weight
-// 51) and the cell's final value with the same expression.  Off the band s2
+// whole device, and forms lambda from the sums of s2 and s3 over the band cells
+// of the 3x3x3 box around each (centre weight 51) and the cell's final value
+// with the same expression.  Off the band s2
 // and s3 are zero, so the box sums take band cells only.
 //
 // k_redis3d: a workgroup of R3X*R3Y threads owns an interior tile in (i, j),
@@ -76,6 +76,29 @@ template <typename T> LSMP_DEV bool in_band_x(T x)
     return !(x > T(1) - T(1.0e-12)) && !(x < T(-1) + T(1.0e-12));
 }
 
+// delta of ls_funs for a cell of the band (its middle branch, |x| < 1 with
+// x = phi / ls_wid): 0.5 (1 + cos(pi x)) / ls_wid = cos(theta)^2 / ls_wid with
+// theta = pi x / 2 in (-pi/2, pi/2), cos from its Taylor series in theta^2 to
+// the term in theta^20 (remainder below 2e-17 there).  Within 2.3e-16 of
+// 0.5 (1 + cos(pi x)) evaluated with a correctly rounded cosine.
+template <typename T> LSMP_DEV T band_delta(T phi, T inv_w)
+{
+    const T th = (phi * inv_w) * T(1.570796326794896619231321691639751442);
+    const T t = th * th;
+    T c = T(1.0 / 2432902008176640000.0);     // 1/20!
+    c = fma(c, t, T(-1.0 / 6402373705728000.0));   // -1/18!
+    c = fma(c, t, T(1.0 / 20922789888000.0));      // 1/16!
+    c = fma(c, t, T(-1.0 / 87178291200.0));        // -1/14!
+    c = fma(c, t, T(1.0 / 479001600.0));           // 1/12!
+    c = fma(c, t, T(-1.0 / 3628800.0));            // -1/10!
+    c = fma(c, t, T(1.0 / 40320.0));               // 1/8!
+    c = fma(c, t, T(-1.0 / 720.0));                // -1/6!
+    c = fma(c, t, T(1.0 / 24.0));                  // 1/4!
+    c = fma(c, t, T(-0.5));                        // -1/2!
+    c = fma(c, t, T(1));
+    return c * c * inv_w;
+}
+
 // Godunov |grad phi| (level_set_rk3_redis.f90:341-360) from the one-sided
 // slopes times 6 dx, 6 dy, 6 dz; k = 1 / (6 dx), ...: with sigma the sign of
 // S0, max(-min(D+, 0), max(D-, 0)) is max(-sigma D+, sigma D-, 0) per direction
@@ -127,7 +150,7 @@ template <typename T, int STAGE, int BTN>
 __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__restrict__ phi_out,
                                                 const T *__restrict__ phi0, const T *__restrict__ S0, RedisArgs ra,
                                                 unsigned long long *ctl, const unsigned char *__restrict__ tiles,
-                                                T *__restrict__ bgr, unsigned *__restrict__ blist,
+                                                BandFields<T> bf, unsigned *__restrict__ blist,
                                                 unsigned *__restrict__ bcount, int kc)
 {
     // rows of P3X slots: the plane with its halo, then Q of the x faces (row ty,
@@ -306,8 +329,11 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
             asm("" : "+v"(at));
             store_at(phi_out + off, at, pn);
             if (band) {
+                const T del = band_delta(w0, inv_w);
                 asm("" : "+v"(at));
-                store_at(bgr + off, at, grad);
+                store_at(bf.gr + off, at, grad);
+                store_at(bf.s2 + off, at, del * s0_cur * (grad - T(1)));
+                store_at(bf.s3 + off, at, grad * del * del);
             } else if (STAGE == 3) {
                 lerr = fmax(lerr, fabs(pn - p0_cur));
             }
@@ -372,29 +398,6 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     }
 }
 
-// delta of ls_funs for a cell of the band (its middle branch, |x| < 1 with
-// x = phi / ls_wid): 0.5 (1 + cos(pi x)) / ls_wid = cos(theta)^2 / ls_wid with
-// theta = pi x / 2 in (-pi/2, pi/2), cos from its Taylor series in theta^2 to
-// the term in theta^20 (remainder below 2e-17 there).  Within 2.3e-16 of
-// 0.5 (1 + cos(pi x)) evaluated with a correctly rounded cosine.
-template <typename T> LSMP_DEV T band_delta(T phi, T inv_w)
-{
-    const T th = (phi * inv_w) * T(1.570796326794896619231321691639751442);
-    const T t = th * th;
-    T c = T(1.0 / 2432902008176640000.0);     // 1/20!
-    c = fma(c, t, T(-1.0 / 6402373705728000.0));   // -1/18!
-    c = fma(c, t, T(1.0 / 20922789888000.0));      // 1/16!
-    c = fma(c, t, T(-1.0 / 87178291200.0));        // -1/14!
-    c = fma(c, t, T(1.0 / 479001600.0));           // 1/12!
-    c = fma(c, t, T(-1.0 / 3628800.0));            // -1/10!
-    c = fma(c, t, T(1.0 / 40320.0));               // 1/8!
-    c = fma(c, t, T(-1.0 / 720.0));                // -1/6!
-    c = fma(c, t, T(1.0 / 24.0));                  // 1/4!
-    c = fma(c, t, T(-0.5));                        // -1/2!
-    c = fma(c, t, T(1));
-    return c * c * inv_w;
-}
-
 // The listed band cells: lambda from the 3x3x3 box sums of s2, s3 (centre
 // weight 51, :409-448) in the reference's order -- in-plane sums row by row,
 // then (plane k-1 + plane k) + plane k+1 -- and the cell's value.  Ghost cells
@@ -411,7 +414,7 @@ template <typename T, int STAGE>
 __global__ __launch_bounds__(NT) void k_redis3d_band(const T *__restrict__ phi, T *__restrict__ phi_out,
                                                      const T *__restrict__ phi0, const T *__restrict__ S0,
                                                      RedisArgs ra, unsigned long long *ctl,
-                                                     const T *__restrict__ bgr, const unsigned *__restrict__ blist,
+                                                     BandFields<T> bf, const unsigned *__restrict__ blist,
                                                      const unsigned *bcount, unsigned *bnext)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) *bnext = 0;
@@ -438,14 +441,13 @@ __global__ __launch_bounds__(NT) void k_redis3d_band(const T *__restrict__ phi, 
         const unsigned rem = c % plane;
         const int k = (int)(c / plane), cj = (int)(rem / (unsigned)nx), ci = (int)(rem % (unsigned)nx);
         T part2 = T(0), part3 = T(0);
-        T phc = T(0), s0 = T(0), grad = T(0), p0 = T(0);
+        T phc = T(0), s0 = T(0), grad = T(0), p0 = T(0), c2 = T(0), c3 = T(0);
         if (q < 3) {
-            // box plane k-1+q: phi (band membership, delta), S0 and |grad| of
-            // its nine cells, all loads in flight together; cells off the band
-            // contribute nothing (their s2, s3 are zero up to sign), whatever
-            // |grad| holds there
+            // box plane k-1+q: phi (band membership), s2 and s3 of its nine
+            // cells, all loads in flight together; cells off the band contribute
+            // nothing, whatever earlier stages left in s2 and s3 there
             const unsigned pb = (unsigned)clampi(k - 1 + q, 0, nz - 1) * plane;
-            T pv[9], sv[9], gv[9];
+            T pv[9], s2[9], s3[9];
 #pragma unroll
             for (int jj = 0; jj < 3; ++jj)
 #pragma unroll
@@ -453,30 +455,29 @@ __global__ __launch_bounds__(NT) void k_redis3d_band(const T *__restrict__ phi, 
                     const unsigned at = pb + (unsigned)clampi(cj - 1 + jj, 0, ny - 1) * (unsigned)nx +
                                         (unsigned)clampi(ci - 1 + ii, 0, nx - 1);
                     pv[jj * 3 + ii] = phi[at];
-                    sv[jj * 3 + ii] = S0[at];
-                    gv[jj * 3 + ii] = bgr[at];
+                    s2[jj * 3 + ii] = bf.s2[at];
+                    s3[jj * 3 + ii] = bf.s3[at];
                 }
-            if (stopped) return;
+            if (stopped || e0 >= ncell) return;
 #pragma unroll
             for (int r = 0; r < 9; ++r) {
                 const bool inb = in_band_x(pv[r] * inv_w);
-                const T dn = band_delta(pv[r], inv_w);
-                const T s2 = dn * sv[r] * (gv[r] - T(1)), s3 = gv[r] * dn * dn;
-                part2 = part2 + (inb ? s2 : T(0));
-                part3 = part3 + (inb ? s3 : T(0));
+                part2 = part2 + (inb ? s2[r] : T(0));
+                part3 = part3 + (inb ? s3[r] : T(0));
             }
         } else {
             phc = phi[c];
             s0 = S0[c];
-            grad = bgr[c];
+            grad = bf.gr[c];
+            c2 = bf.s2[c];
+            c3 = bf.s3[c];
             if (STAGE > 1) p0 = phi0[c];
-            if (stopped) return;
+            if (stopped || e0 >= ncell) return;
         }
         const T a0 = __shfl(part2, g0, 64), a1 = __shfl(part2, g0 + 1, 64), a2 = __shfl(part2, g0 + 2, 64);
         const T b0 = __shfl(part3, g0, 64), b1 = __shfl(part3, g0 + 1, 64), b2 = __shfl(part3, g0 + 2, 64);
         if (q == 3 && e < ncell) {
             const T del = band_delta(phc, inv_w);
-            const T c2 = del * s0 * (grad - T(1)), c3 = grad * del * del;
             const T la = T(51) * c2 + ((a0 + a1) + a2);
             const T lb = T(51) * c3 + ((b0 + b1) + b2);
             T lam = T(0);
@@ -533,10 +534,10 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
     do {                                                                                                       \
         if (!band)                                                                                             \
             hipLaunchKernelGGL((k_redis3d<T, S, B>), g, dim3(NT), 0, st, phi, phi_out, phi0, S0, ra, ctl,      \
-                               tiles, bd.gr, bd.list, bd.count, kc);                                           \
+                               tiles, bd.f, bd.list, bd.count, kc);                                           \
         else if (B == 1)                                                                                       \
             hipLaunchKernelGGL((k_redis3d_band<T, S>), dim3(BAND_GRID), dim3(NT), 0, st, phi, phi_out, phi0,   \
-                               S0, ra, ctl, bd.gr, bd.list, bd.count, bd.next);                                \
+                               S0, ra, ctl, bd.f, bd.list, bd.count, bd.next);                                \
     } while (0)
     if (btn) { if (stage == 1) LSMP_R3(1, 1); else if (stage == 2) LSMP_R3(2, 1); else LSMP_R3(3, 1); }
     else { if (stage == 1) LSMP_R3(1, 0); else if (stage == 2) LSMP_R3(2, 0); else LSMP_R3(3, 0); }
