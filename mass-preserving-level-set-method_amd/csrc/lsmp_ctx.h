@@ -34,7 +34,8 @@ struct lsmp_ctx {
     double *partial = nullptr, *scal = nullptr;
     double *vtab = nullptr;   // per-axis sine tables of the analytic velocity
     unsigned long long *u64 = nullptr;
-    unsigned long long *rctl = nullptr;   // pseudo-time loop control block (k_redis_ctl)
+    unsigned long long *rctl = nullptr;   // pseudo-time loop control block
+    int rset = 0;                         // the last queued pseudo-step's set of its words
     double *hbuf = nullptr;   // pinned readback
     int npartial = 0;
     int band_lines = 1;              // mass correction on band lines: 0 never, 1 where it pays, 2 always

@@ -413,8 +413,8 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
         if (time > timestop) break;
     }
     if (max_iter > 0 && budget > max_iter) budget = max_iter;
-    // the max |dphi| <= 1e-6 stop is taken on the device (k_redis_ctl); steps
-    // are queued CHUNK at a time and the host reads the control block per chunk
+    // the max |dphi| <= 1e-6 stop is taken on the device (redis_begin_step);
+    // steps are queued CHUNK at a time and the host reads the control block per chunk
     constexpr int CHUNK = 16;
     unsigned long long *ctl = c->rctl;
     // narrow band (3D): workgroups with no cell |phi| < W keep their cells
@@ -437,7 +437,6 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
         bd.f = BandFields<T>{f, f + c->ncell, f + 2 * c->ncell};
         bd.list = c->rb_list;
     }
-    launch_redis_ctl(c->st, ctl, 0);
     int launched = 0;
     unsigned long long hc[4] = {0, 0, 0, 0};
     const bool defer = queued && budget <= CHUNK;
@@ -446,6 +445,8 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
         const int k = std::min(CHUNK, budget - launched);
         for (int q = 0; q < k; ++q) {
             T *cur = (T *)c->phi, *b = (T *)c->phiB, *cc = (T *)c->phiC;
+            c->rset = (c->rset + 1) % 3;
+            const RedisStep step = {c->rset, launched + q == 0};
             if (c->dim == 3) {
                 // stages 1..3: every cell (lambda = 0), then the band cells (lambda)
                 const T *in[3] = {cur, b, cc};
@@ -456,24 +457,24 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
                         bd.next = c->rb_count + (1 - c->rb_par);
                     }
                     KT(c, "redis_stage",
-                       (launch_redis3d<T>(c->st, sg + 1, btn, in[sg], outp[sg], cur, S0, ra, ctl, tiles, bd, false)));
+                       (launch_redis3d<T>(c->st, sg + 1, btn, in[sg], outp[sg], cur, S0, ra, ctl, tiles, bd, false, step)));
                     if (btn == 1) {
                         KT(c, "redis_band",
-                           (launch_redis3d<T>(c->st, sg + 1, btn, in[sg], outp[sg], cur, S0, ra, ctl, tiles, bd, true)));
+                           (launch_redis3d<T>(c->st, sg + 1, btn, in[sg], outp[sg], cur, S0, ra, ctl, tiles, bd, true, step)));
                         c->rb_par ^= 1;
                     }
                 }
             } else {
-                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 1, btn, cur, b, cur, S0, ra, ctl)));
-                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 2, btn, b, cc, cur, S0, ra, ctl)));
-                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 3, btn, cc, b, cur, S0, ra, ctl)));
+                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 1, btn, cur, b, cur, S0, ra, ctl, step)));
+                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 2, btn, b, cc, cur, S0, ra, ctl, step)));
+                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 3, btn, cc, b, cur, S0, ra, ctl, step)));
             }
-            launch_redis_ctl(c->st, ctl, 2);
             // the new phi is in b; the old one becomes a spare
             c->phiB = c->phi;
             c->phi = b;
         }
         launched += k;
+        launch_redis_ctl(c->st, ctl, RedisStep{c->rset, false});
         if (defer) {
             *queued = launched;
             return LSMP_OK;
@@ -889,6 +890,7 @@ int lsmp_init(const lsmp_params *params, lsmp_handle *out)
     if (alloc(&c->scr, sc * c->esz)) return fail(LSMP_E_HIP);
     if (alloc((void **)&c->vtab, (size_t)2 * (c->nx + c->ny + c->nz) * sizeof(double))) return fail(LSMP_E_HIP);
     if (alloc((void **)&c->rctl, CTL_WORDS * sizeof(unsigned long long))) return fail(LSMP_E_HIP);
+    launch_zero_u64(c->st, c->rctl, CTL_WORDS);
     for (int d = 0; d < c->dim; ++d) {
         std::vector<double> tab;
         ccd_tables(ns[d] + 2 * GHC, params->dx, tab);   // all three solvers use dx (ccd_solvers.f90:406-408)

@@ -44,15 +44,64 @@ constexpr int RKC = 16;
 // cell is skipped, and an active one's march is the kernel's critical path
 constexpr int RKC_NB = 8;
 
-// The pseudo-time loop's control words (k_redis_ctl): ctl[0..3], then the
-// running max |dphi| striped over CTL_SLOTS words by workgroup, so that the
-// workgroups of a stage, which end close together, do not queue their
-// atomics on one address.
+// The pseudo-time loop's control words: ctl[1] the stop flag, ctl[2] the
+// pseudo-steps run, ctl[3] max |dphi| of the last one (once the loop has stopped
+// or k_redis_ctl has closed a batch), then three sets of CTL_SLOTS words.  A
+// step's running max |dphi| is striped over one set by workgroup, so that the
+// workgroups of a stage, which end close together, do not queue their atomics
+// on one address; the next step reads it, and a step's first kernel clears the
+// next step's set, which the step before last was the last to read.
 constexpr int CTL_SLOTS = 64;
-constexpr int CTL_WORDS = 4 + CTL_SLOTS;
-__device__ inline unsigned long long *ctl_slot(unsigned long long *ctl, unsigned b)
+constexpr int CTL_WORDS = 4 + 3 * CTL_SLOTS;
+// a pseudo-step as the kernels need it: its set, and whether it starts a run
+struct RedisStep {
+    int set;
+    bool first;
+};
+__device__ inline unsigned long long *ctl_slot(unsigned long long *ctl, RedisStep step, unsigned b)
 {
-    return ctl + 4 + b % (unsigned)CTL_SLOTS;
+    return ctl + 4 + step.set * CTL_SLOTS + b % (unsigned)CTL_SLOTS;
+}
+
+// First thing of a pseudo-step, by every wave of its first kernel: whether the
+// loop has stopped (level_set_rk3_redis.f90:17-23, 68) -- before, or with the
+// step just run, whose max |dphi| <= 1e-6 (the bits of non-negative doubles, and
+// of a NaN, which never stops the loop, keep their order as integers).  The
+// lead workgroup counts the step, or sets the flag that the later stages and
+// steps look at, and clears the next step's set.  Two words in flight together
+// instead of a closing launch per step (4.8 us each).
+__device__ inline bool redis_begin_step(unsigned long long *ctl, RedisStep step, bool lead)
+{
+    const int lane = threadIdx.x & 63;
+    bool stopped = false;
+    unsigned long long v = 0, flag = 0;
+    if (!step.first) {
+        v = ctl[4 + (step.set + 2) % 3 * CTL_SLOTS + lane];
+        flag = ctl[1];
+        stopped = flag != 0 || __ballot(v > (unsigned long long)__double_as_longlong(1.0e-6)) == 0;
+    }
+    if (lead && threadIdx.x < 64) {
+        ctl[4 + (step.set + 1) % 3 * CTL_SLOTS + lane] = 0;
+        if (stopped && !flag) {
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) {
+                const unsigned long long o = __shfl_xor(v, d, 64);
+                v = o > v ? o : v;
+            }
+        }
+        if (lane == 0) {
+            if (step.first) {
+                ctl[1] = 0;
+                ctl[2] = 1;
+            } else if (!stopped) {
+                ctl[2] += 1;
+            } else if (!flag) {
+                ctl[1] = 1;
+                ctl[3] = v;
+            }
+        }
+    }
+    return stopped;
 }
 
 struct RedisArgs {
@@ -126,12 +175,12 @@ void launch_adv_tile(hipStream_t st, int mode, int stage, T *phi, const T *vel, 
 template <typename T>
 void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
                     const RedisArgs &ra, unsigned long long *ctl, const unsigned char *tiles, const RedisBand<T> &bd,
-                    bool band);
+                    bool band, RedisStep step);
 template <typename T>
 void launch_combine_markers(hipStream_t st, const T *m1, const T *m2, T *phi, size_t n, unsigned *flag);
 template <typename T>
 void launch_redis_stage2d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
-                          const RedisArgs &ra, unsigned long long *ctl);
+                          const RedisArgs &ra, unsigned long long *ctl, RedisStep step);
 template <typename T> void launch_sign_init(hipStream_t st, const T *phi, T *S0, size_t n, T ls_wid, int raw);
 template <typename T>
 void launch_grad_max(hipStream_t st, int dim, const T *phi, const T *S0, const RedisArgs &ra,
@@ -224,6 +273,6 @@ template <typename T>
 void launch_energy_sums(hipStream_t st, int dim, bool vof_marker, const T *phi, const T *vof, const T *u, const T *v,
                         const T *w, const T *ten, const EnergyArgs &ea, double *partial, int nblocks);
 void launch_energy_finalize(hipStream_t st, const double *partial, int nblk, double dx, double *out);
-void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, int op);
+void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, RedisStep last);
 
 }  // namespace lsmp

@@ -17,8 +17,7 @@ template <typename T> LSMP_DEV double to_d(T v) { return (double)v; }
 
 __global__ void k_zero_u64(unsigned long long *p, int n)
 {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) p[t] = 0ull;
+    for (int t = threadIdx.x; t < n; t += blockDim.x) p[t] = 0ull;
 }
 
 // ---------------------------------------------------------------------------
@@ -745,13 +744,12 @@ static_assert(R2F <= 2 * RNT, "two faces a thread");
 template <typename T, int STAGE, int BTN>
 __global__ __launch_bounds__(RNT) void k_redis_stage2d(const T *__restrict__ phi, T *__restrict__ phi_out,
                                                        const T *__restrict__ phi0, const T *__restrict__ S0,
-                                                       RedisArgs ra, unsigned long long *ctl)
+                                                       RedisArgs ra, unsigned long long *ctl, RedisStep step)
 {
     __shared__ T sphi[RPY][RPX];
     __shared__ T fplus[R2F], fminus[R2F];   // P and Q of the faces
     __shared__ T ss2[REY][REX];
     __shared__ T ss3[REY][REX];
-    if (ctl[1]) return;   // the pseudo-time loop has stopped (k_redis_ctl)
     const int nx = ra.nx, ny = ra.ny;
     const T kx = (T)(2.0 * ra.inv12dx), ky = (T)(2.0 * ra.inv12dy);
     const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt;
@@ -769,6 +767,8 @@ __global__ __launch_bounds__(RNT) void k_redis_stage2d(const T *__restrict__ phi
         sphi[r][c] = phi[(size_t)gy * nx + gx];
     }
     const T s0_p = ext ? S0[(size_t)gj * nx + gi] : T(0);
+    // the pseudo-time loop has stopped
+    if (STAGE == 1 ? redis_begin_step(ctl, step, (blockIdx.x | blockIdx.y) == 0) : ctl[1] != 0) return;
     __syncthreads();
     // the faces: x face f (< R2FX) at ring row f / (RTX + 3), cell i0 - 2 + f % (RTX + 3);
     // y face g = f - R2FX at cell j0 - 2 + g / REX, ring column g % REX.  Past
@@ -859,7 +859,7 @@ __global__ __launch_bounds__(RNT) void k_redis_stage2d(const T *__restrict__ phi
     }
     if (STAGE == 3) {
         double m = block_max(lerr);
-        if (t == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, blockIdx.y * gridDim.x + blockIdx.x), m);
+        if (t == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, step, blockIdx.y * gridDim.x + blockIdx.x), m);
     }
 }
 
@@ -877,40 +877,27 @@ __global__ void k_sign_init(const T *__restrict__ phi, T *__restrict__ S0, size_
     S0[q] = T(2) * H - T(1);
 }
 
-// Device-side control of the pseudo-time loop (level_set_rk3_redis.f90:17-23, 68):
-// ctl[1] stop flag, ctl[2] pseudo-steps run, ctl[3] max |dphi| of the last
-// one; the running pseudo-step's max |dphi| (bits of a non-negative double)
-// is striped over ctl[4 .. 4 + CTL_SLOTS).  One wave: op 0 resets, op 2 closes
-// a pseudo-step -- reduces the stripes to its max |dphi|, clears them for the
-// next step and stops the loop once the step's max |dphi| <= 1e-6 (a NaN
-// never stops it, as in the reference); the time limit is the host's count of
-// launched steps.  Stage kernels return at once when the flag is set, so
-// steps can be queued ahead without host round trips and the step count stays
-// the reference's.
-__global__ void k_redis_ctl(unsigned long long *ctl, int op)
+// Closes a batch of pseudo-steps (redis_begin_step counts them): max |dphi| of
+// the last step run into ctl[3], and the stop flag when it is at most 1e-6 (a
+// NaN never stops the loop, as in the reference); the time limit is the host's
+// count of launched steps.  Stage kernels return at once when the flag is
+// set, so steps can be queued ahead without host round trips and the step
+// count stays the reference's.  One wave.
+__global__ void k_redis_ctl(unsigned long long *ctl, RedisStep last)
 {
     const int t = threadIdx.x;   // stripe t
-    if (op == 0) {
-        ctl[4 + t] = 0;
-        if (t < 4) ctl[t] = 0;
-        return;
-    }
     if (ctl[1]) return;
-    const double v = __longlong_as_double((long long)ctl[4 + t]);
-    ctl[4 + t] = 0;
     // non-negative doubles (and a NaN, whose bits order above them) keep their
     // order as integers: the max of the bit patterns
-    unsigned long long m = (unsigned long long)__double_as_longlong(v);
+    unsigned long long m = *ctl_slot(ctl, last, (unsigned)t);
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
         const unsigned long long o = __shfl_xor(m, d, 64);
         m = o > m ? o : m;
     }
     if (t == 0) {
-        ctl[2] += 1;
         ctl[3] = m;
-        const double e = __longlong_as_double((long long)m);
-        if (e <= 1.0e-6) ctl[1] = 1;
+        if (__longlong_as_double((long long)m) <= 1.0e-6) ctl[1] = 1;
     }
 }
 
@@ -1939,10 +1926,10 @@ void launch_tube_tiles(hipStream_t st, const T *phi, int nx, int ny, int nz, dou
 
 template <typename T>
 void launch_redis_stage2d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
-                          const RedisArgs &ra, unsigned long long *ctl)
+                          const RedisArgs &ra, unsigned long long *ctl, RedisStep step)
 {
     const dim3 g(nblk(ra.nx, RTX), nblk(ra.ny, RTY), 1);
-#define LSMP_R2(S, B) hipLaunchKernelGGL((k_redis_stage2d<T, S, B>), g, dim3(RNT), 0, st, phi, phi_out, phi0, S0, ra, ctl)
+#define LSMP_R2(S, B) hipLaunchKernelGGL((k_redis_stage2d<T, S, B>), g, dim3(RNT), 0, st, phi, phi_out, phi0, S0, ra, ctl, step)
     if (btn) { if (stage == 1) LSMP_R2(1, 1); else if (stage == 2) LSMP_R2(2, 1); else LSMP_R2(3, 1); }
     else { if (stage == 1) LSMP_R2(1, 0); else if (stage == 2) LSMP_R2(2, 0); else LSMP_R2(3, 0); }
 #undef LSMP_R2
@@ -2206,10 +2193,10 @@ void launch_convert(hipStream_t st, TO *out, const TI *in, size_t n)
     hipLaunchKernelGGL((k_convert<TO, TI>), dim3(nblk(n, 256)), dim3(256), 0, st, out, in, n);
 }
 
-void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, int op)
+void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, RedisStep last)
 {
     static_assert(CTL_SLOTS == 64, "one wave, a stripe per lane");
-    hipLaunchKernelGGL(k_redis_ctl, dim3(1), dim3(CTL_SLOTS), 0, st, ctl, op);
+    hipLaunchKernelGGL(k_redis_ctl, dim3(1), dim3(CTL_SLOTS), 0, st, ctl, last);
 }
 
 void launch_zero_u64(hipStream_t st, unsigned long long *p, int n)
@@ -2222,7 +2209,7 @@ void launch_zero_u64(hipStream_t st, unsigned long long *p, int n)
                                      T, T, const int *, int, const TubeMask &);                                \
     template void launch_combine_markers<T>(hipStream_t, const T *, const T *, T *, size_t, unsigned *);         \
     template void launch_redis_stage2d<T>(hipStream_t, int, int, const T *, T *, const T *, const T *,             \
-                                          const RedisArgs &, unsigned long long *);                            \
+                                          const RedisArgs &, unsigned long long *, RedisStep);                 \
     template void launch_tube_tiles<T>(hipStream_t, const T *, int, int, int, double, unsigned char *);          \
     template void launch_sign_init<T>(hipStream_t, const T *, T *, size_t, T, int);                            \
     template void launch_grad_max<T>(hipStream_t, int, const T *, const T *, const RedisArgs &,                \

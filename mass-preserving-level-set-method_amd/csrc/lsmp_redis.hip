@@ -151,7 +151,7 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
                                                 const T *__restrict__ phi0, const T *__restrict__ S0, RedisArgs ra,
                                                 unsigned long long *ctl, const unsigned char *__restrict__ tiles,
                                                 BandFields<T> bf, unsigned *__restrict__ blist,
-                                                unsigned *__restrict__ bcount, int kc)
+                                                unsigned *__restrict__ bcount, int kc, RedisStep step)
 {
     // rows of P3X slots: the plane with its halo, then Q of the x faces (row ty,
     // slot tx: of cell tx), then Q of the y faces (row ty: of cell ty).  One row
@@ -163,7 +163,6 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     __shared__ unsigned short lcell[BTN == 1 ? RKC * NT : 1];
     __shared__ unsigned lcount, lbase;
     static_assert(RKC * NT <= 65536, "local band-cell index in 16 bits");
-    if (ctl[1]) return;   // the pseudo-time loop has stopped (k_redis_ctl)
     const int nx = ra.nx, ny = ra.ny, nz = ra.nz;
     // tiles in x-fastest order, renumbered so that each XCD takes a contiguous
     // run of them: the x and y halos of a tile are then mostly in its XCD's L2
@@ -171,11 +170,15 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     const int tile_id = xcd_renumber((int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x),
                                      gx * gy * (int)gridDim.z);
     const int bx = tile_id % gx, by = (tile_id / gx) % gy, bz = tile_id / (gx * gy);
+    // whether the pseudo-time loop has stopped: looked at once the run-up's loads
+    // are on their way, before anything is written
+    const bool lead = (blockIdx.x | blockIdx.y | blockIdx.z) == 0;
+    auto stopped = [&]() { return STAGE == 1 ? redis_begin_step(ctl, step, lead) : ctl[1] != 0; };
     // narrow band: a workgroup with no cell of the tube keeps its cells.  Stage
     // 1 writes the step's output buffer and stage 2 the one stage 3 reads, so
     // both copy; stage 3 writes the buffer stage 1 filled, which holds them.
     if (tiles && !tiles[tile_id]) {
-        if (STAGE == 3) return;
+        if (stopped() || STAGE == 3) return;
         const int ci = bx * R3X + (int)threadIdx.x % R3X, cj = by * R3Y + (int)threadIdx.x / R3X;
         if (ci >= nx || cj >= ny) return;
         const size_t c0 = (size_t)cj * nx + ci, pl = (size_t)nx * ny;
@@ -220,14 +223,17 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     const int own = ty * P3X + tx;   // the thread's cell, less 4 rows and 4 slots of halo
     T *const hdst = &lds[hr * P3X + hc], *const hdst2 = &lds[hr2 * P3X + hc2];
 
-    T w0, w1, w2, w3;   // phi(p .. p+3) of this cell's column
+    T v[7];   // phi(k0-3 .. k0+3) of this cell's column
+#pragma unroll
+    for (int d = 0; d < 7; ++d) v[d] = load_at(base(phi, k0 - 3 + d), col);
+    T halo_cur = halo ? load_at(base(phi, k0), hcol) : T(0);
+    T halo2_cur = halo2 ? load_at(base(phi, k0), hcol2) : T(0);
+    if (stopped()) return;
+    T w0 = v[3], w1 = v[4], w2 = v[5], w3 = v[6];   // phi(p .. p+3)
     // z: second differences s(p-1), s(p), s(p+1), h(s(p)), e(p) and Q of face
     // p - 1/2, carried from plane to plane
     T za, zb, zc, zhb, ze, zq;
     {
-        T v[7];   // phi(k0-3 .. k0+3)
-#pragma unroll
-        for (int d = 0; d < 7; ++d) v[d] = load_at(base(phi, k0 - 3 + d), col);
         const T s2 = v[0] - T(2) * v[1] + v[2], s1 = v[1] - T(2) * v[2] + v[3];   // s(k0-2), s(k0-1)
         const T s0 = v[2] - T(2) * v[3] + v[4], sp = v[3] - T(2) * v[4] + v[5];   // s(k0), s(k0+1)
         za = s1;
@@ -237,13 +243,7 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         ze = zc - T(2) * zb + za;
         T unused;
         weno_hj_face(s2, s1, s0, sp, hj_h(s1), zhb, ze, s0 - T(2) * s1 + s2, unused, zq);
-        w0 = v[3];
-        w1 = v[4];
-        w2 = v[5];
-        w3 = v[6];
     }
-    T halo_cur = halo ? load_at(base(phi, k0), hcol) : T(0);
-    T halo2_cur = halo2 ? load_at(base(phi, k0), hcol2) : T(0);
     if (BTN == 1 && t == 0) lcount = 0;   // read after the loop's first barrier
     T lerr = T(0);
     // every load of the run-up is in, so that no plane waits for its own loads
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     }
     if (STAGE == 3) {
         double m = block_max((double)lerr);
-        if (t == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, (unsigned)tile_id), m);
+        if (t == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, step, (unsigned)tile_id), m);
     }
 }
 
@@ -415,14 +415,14 @@ __global__ __launch_bounds__(NT) void k_redis3d_band(const T *__restrict__ phi, 
                                                      const T *__restrict__ phi0, const T *__restrict__ S0,
                                                      RedisArgs ra, unsigned long long *ctl,
                                                      BandFields<T> bf, const unsigned *__restrict__ blist,
-                                                     const unsigned *bcount, unsigned *bnext)
+                                                     const unsigned *bcount, unsigned *bnext, RedisStep step)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) *bnext = 0;
     const unsigned ncell = bcount[0];
     // stage 3: the maximum change in this workgroup's stripe, the stage
     // kernel's part of it complete now; a workgroup whose own maximum is not
     // above it skips the atomic (the 1,024 workgroups end together)
-    unsigned long long *slot = ctl_slot(ctl, blockIdx.x);
+    unsigned long long *slot = ctl_slot(ctl, step, blockIdx.x);
     const unsigned long long stage_max = STAGE == 3 ? *slot : 0ull;
     const int nx = ra.nx, ny = ra.ny, nz = ra.nz;
     const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt;
@@ -525,7 +525,7 @@ static int stage_planes(unsigned tiles, int nz)
 template <typename T>
 void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
                     const RedisArgs &ra, unsigned long long *ctl, const unsigned char *tiles, const RedisBand<T> &bd,
-                    bool band)
+                    bool band, RedisStep step)
 {
     // the narrow band (tiles) marches RKC_NB planes per workgroup
     const int kc = tiles ? RKC_NB : stage_planes(nb_of(ra.nx, R3X) * nb_of(ra.ny, R3Y), ra.nz);
@@ -534,10 +534,10 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
     do {                                                                                                       \
         if (!band)                                                                                             \
             hipLaunchKernelGGL((k_redis3d<T, S, B>), g, dim3(NT), 0, st, phi, phi_out, phi0, S0, ra, ctl,      \
-                               tiles, bd.f, bd.list, bd.count, kc);                                           \
+                               tiles, bd.f, bd.list, bd.count, kc, step);                                           \
         else if (B == 1)                                                                                       \
             hipLaunchKernelGGL((k_redis3d_band<T, S>), dim3(BAND_GRID), dim3(NT), 0, st, phi, phi_out, phi0,   \
-                               S0, ra, ctl, bd.f, bd.list, bd.count, bd.next);                                \
+                               S0, ra, ctl, bd.f, bd.list, bd.count, bd.next, step);                                \
     } while (0)
     if (btn) { if (stage == 1) LSMP_R3(1, 1); else if (stage == 2) LSMP_R3(2, 1); else LSMP_R3(3, 1); }
     else { if (stage == 1) LSMP_R3(1, 0); else if (stage == 2) LSMP_R3(2, 0); else LSMP_R3(3, 0); }
@@ -546,9 +546,9 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
 
 template void launch_redis3d<double>(hipStream_t, int, int, const double *, double *, const double *, const double *,
                                      const RedisArgs &, unsigned long long *, const unsigned char *,
-                                     const RedisBand<double> &, bool);
+                                     const RedisBand<double> &, bool, RedisStep);
 template void launch_redis3d<float>(hipStream_t, int, int, const float *, float *, const float *, const float *,
                                     const RedisArgs &, unsigned long long *, const unsigned char *,
-                                    const RedisBand<float> &, bool);
+                                    const RedisBand<float> &, bool, RedisStep);
 
 }  // namespace lsmp
