@@ -334,6 +334,45 @@ template <typename T> LSMP_DEV void ls_funs_fast(T phi, T inv_w, T &H, T &D)
     H = fmax(fmin(H, T(1)), T(0));
 }
 
+// H and delta of ls_funs in FP64 without library calls: with theta = pi x / 2
+// in (-pi/2, pi/2) for a cell of the band (x = phi / w), delta = cos(theta)^2 / w
+// and sin(pi x) = 2 sin(theta) cos(theta), sine and cosine from their Taylor
+// series (remainders below 2e-17).  Within 2.3e-16 of correctly rounded H and
+// delta w.
+LSMP_DEV void ls_funs_taylor(double phi, double w, double &H, double &D)
+{
+    const double eps = 1.0e-12;
+    const double x = phi / w;
+    H = x > 0.0 ? 1.0 : 0.0;
+    D = 0.0;
+    if (x > 1.0 - eps || x < -1.0 + eps) return;
+    const double th = x * 1.570796326794896619231321691639751442, t = th * th;
+    double c = 1.0 / 2432902008176640000.0;        // 1/20!
+    c = fma(c, t, -1.0 / 6402373705728000.0);      // -1/18!
+    c = fma(c, t, 1.0 / 20922789888000.0);         // 1/16!
+    c = fma(c, t, -1.0 / 87178291200.0);           // -1/14!
+    c = fma(c, t, 1.0 / 479001600.0);              // 1/12!
+    c = fma(c, t, -1.0 / 3628800.0);               // -1/10!
+    c = fma(c, t, 1.0 / 40320.0);                  // 1/8!
+    c = fma(c, t, -1.0 / 720.0);                   // -1/6!
+    c = fma(c, t, 1.0 / 24.0);                     // 1/4!
+    c = fma(c, t, -0.5);                           // -1/2!
+    c = fma(c, t, 1.0);
+    double s = 1.0 / 51090942171709440000.0;       // 1/21!
+    s = fma(s, t, -1.0 / 121645100408832000.0);    // -1/19!
+    s = fma(s, t, 1.0 / 355687428096000.0);        // 1/17!
+    s = fma(s, t, -1.0 / 1307674368000.0);         // -1/15!
+    s = fma(s, t, 1.0 / 6227020800.0);             // 1/13!
+    s = fma(s, t, -1.0 / 39916800.0);              // -1/11!
+    s = fma(s, t, 1.0 / 362880.0);                 // 1/9!
+    s = fma(s, t, -1.0 / 5040.0);                  // -1/7!
+    s = fma(s, t, 1.0 / 120.0);                    // 1/5!
+    s = fma(s, t, -1.0 / 6.0);                     // -1/3!
+    s = fma(s, t, 1.0) * th;
+    H = fmax(fmin(0.5 * ((1.0 + x) + 2.0 * (s * c) * 0.318309886183790671537767526745028724), 1.0), 0.0);
+    D = c * c / w;
+}
+
 // Fourth-order central slope times 12 dx (level_set_rk3_redis.f90:290-293).
 template <typename T> LSMP_DEV T central4(T m2, T m1, T c, T p1, T p2)
 {

@@ -1010,7 +1010,7 @@ __global__ __launch_bounds__(256) void k_ccd_seg(const T *__restrict__ phi, cons
             gr[a] = g;
             // the mass integral is formed in FP64 in both forms
             double h, dd;
-            ls_funs<double>((double)pa, ca.ls_wid, h, dd);
+            ls_funs_taylor((double)pa, ca.ls_wid, h, dd);
             const double gg = (double)g;
             const double r12 = ca.rho_12;
             double rho, plam;
@@ -1277,11 +1277,24 @@ __global__ __launch_bounds__(256) void k_ccd_part(const T *__restrict__ phi, con
     }
     const T lo0 = g00 * XS + g01 * XSS + w0, lo1 = g10 * XS + g11 * XSS + w1;   // x at this lane's first row
     const T nx0 = __shfl(lo0, (lane + 1) & 63, 64), nx1 = __shfl(lo1, (lane + 1) & 63, 64);
+    // the final pass's operands, up to CH rows' loads in flight together (phi is in f)
+    constexpr int CH = !FINAL ? 1 : KC <= 9 ? KC : 6;
+    T dxa[CH], dya[CH];
+    auto operands = [&](int top) {   // of rows top, top - 1 .. down to a multiple of CH
+#pragma unroll
+        for (int r = KC - 1; r >= 0; --r)
+            if (r <= top && r / CH == top / CH) {
+                const size_t a = base + (size_t)clampi(lo + r - 3, 0, n - 1) * (size_t)estride;
+                dxa[r % CH] = dxv[a];
+                dya[r % CH] = DIM == 3 ? dyv[a] : T(0);
+            }
+    };
     // this lane's rows, top down, with the reference's arithmetic from x_{hi+1}
     double acc[3] = {0.0, 0.0, 0.0}, cmp[3] = {0.0, 0.0, 0.0};
     T S = s == LPL - 1 ? XS : nx0, SS = s == LPL - 1 ? XSS : nx1;
 #pragma unroll
     for (int r = KC - 1; r >= 0; --r) {
+        if (FINAL && (r == KC - 1 || r % CH == CH - 1)) operands(r);
         if (r < nrow) {
             const int b = lo + r;
             const T s_ = fs[r] - (A[3 * b + 2] * S + B[3 * b + 2] * SS);
@@ -1297,13 +1310,12 @@ __global__ __launch_bounds__(256) void k_ccd_part(const T *__restrict__ phi, con
                 if (!FINAL) {
                     out[a] = S;
                 } else {
-                    const T dxa = dxv[a], dya = DIM == 3 ? dyv[a] : T(0), pa = phi[a];
                     T g;
-                    if (DIM == 3) g = sqrt(sq(dxa) + sq(dya) + sq(S));
-                    else g = sqrt(sq(dxa) + sq(S));
+                    if (DIM == 3) g = sqrt(sq(dxa[r % CH]) + sq(dya[r % CH]) + sq(S));
+                    else g = sqrt(sq(dxa[r % CH]) + sq(S));
                     gr[a] = g;
                     double h, dd;
-                    ls_funs<double>((double)pa, ca.ls_wid, h, dd);
+                    ls_funs_taylor((double)f[r + 1], ca.ls_wid, h, dd);
                     const double gg = (double)g;
                     const double r12 = ca.rho_12;
                     double rho, plam;
@@ -1528,7 +1540,7 @@ __global__ void k_mass_update(T *__restrict__ phi, const T *__restrict__ gr, siz
     const double lam = scal[3];
     const T p = phi[q];
     double H, D;
-    ls_funs<double>((double)p, (double)ls_wid, H, D);
+    ls_funs_taylor((double)p, (double)ls_wid, H, D);
     if (D == 0.0) return;   // phi + lambda 0 |grad phi| is phi: no read of |grad phi|, no store
     phi[q] = (T)((double)p + lam * D * (double)gr[q]);
 }
@@ -1549,7 +1561,7 @@ __global__ void k_mass_update_lines(T *__restrict__ phi, const T *__restrict__ g
     const double lam = scal[3];
     const T p = phi[a];
     double H, D;
-    ls_funs<double>((double)p, (double)ls_wid, H, D);
+    ls_funs_taylor((double)p, (double)ls_wid, H, D);
     if (D == 0.0) return;
     phi[a] = (T)((double)p + lam * D * (double)gr[a]);
 }
