@@ -38,6 +38,7 @@ struct lsmp_ctx {
     int rset = 0;                         // the last queued pseudo-step's set of its words
     double *hbuf = nullptr;   // pinned readback
     int npartial = 0;
+    int mass_hint = 2;               // iterations the last mass correction took
     int band_lines = 1;              // mass correction on band lines: 0 never, 1 where it pays, 2 always
     unsigned char *lflag = nullptr;  // band flags of the x, y, z lines (band_flag_bytes)
     unsigned *lcount = nullptr;      // listed lines per direction

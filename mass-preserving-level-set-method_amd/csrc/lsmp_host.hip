@@ -503,7 +503,7 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
     const CcdArgs ca = ccd_args(c);
     T *phi = (T *)c->phi;
     int iter, nblk = 0, rc = LSMP_OK;
-    double mass = 0.0, prev_rel = 0.0;
+    double mass = 0.0;
     // The correction changes phi only where delta != 0, so no cell enters the
     // band during the iterations: the lines crossing it at the start cover
     // every later iteration.
@@ -545,46 +545,53 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
                                                   &nfixed)));
     }
     double *psolve = c->partial + (size_t)3 * nfixed;
-    for (iter = 1; iter <= 15; ++iter) {
-        KT(c, "ccd_x", (launch_ccd_pass<T>(c->st, 0, c->dim, false, phi, (const T *)c->coef[0], (T *)c->scr,
-                                           (T *)c->dxv, nullptr, nullptr, nullptr, nullptr, c->nx, c->ny, c->nz,
-                                           ca, nullptr, lst[0], nlst[0])));
-        if (c->dim == 3) {
-            KT(c, "ccd_y", (launch_ccd_pass<T>(c->st, 1, 3, false, phi, (const T *)c->coef[1], (T *)c->scr,
-                                               (T *)c->dyv, nullptr, nullptr, nullptr, nullptr, c->nx, c->ny, c->nz,
-                                               ca, nullptr, lst[1], nlst[1])));
-            KT(c, "ccd_z", (launch_ccd_pass<T>(c->st, 2, 3, true, phi, (const T *)c->coef[2], (T *)c->scr, nullptr,
-                                               (const T *)c->dxv, (const T *)c->dyv, (T *)c->gr, psolve, c->nx,
-                                               c->ny, c->nz, ca, &nblk, lst[2], nlst[2])));
-        } else {
-            KT(c, "ccd_y", (launch_ccd_pass<T>(c->st, 1, 2, true, phi, (const T *)c->coef[1], (T *)c->scr, nullptr,
-                                               (const T *)c->dxv, nullptr, (T *)c->gr, psolve, c->nx, c->ny,
-                                               c->nz, ca, &nblk, lst[1], nlst[1])));
-        }
-        nblk += nfixed;
-        if (nblk > c->npartial) return LSMP_E_INVALID;
-        KT(c, "finalize", (launch_finalize3(c->st, c->partial, nblk, imass, c->scal)));
-        if (lst[dfin])
+    // Iterations are queued ahead: as many as the last correction took (two to
+    // start with), then one at a time; the stop test is taken on the device and
+    // the kernels of an iteration past it return at once.  A look by the host
+    // after every iteration cost a round trip each.
+    CcdArgs it = ca;
+    it.scal = c->scal;
+    int last = 0;
+    for (iter = 0; iter < 15 && !last;) {
+        const int batch = std::min(15 - iter, iter ? 1 : std::max(1, std::min(4, c->mass_hint)));
+        for (int q = 0; q < batch; ++q) {
+            it.iter = ++iter;
+            KT(c, "ccd_x", (launch_ccd_pass<T>(c->st, 0, c->dim, false, phi, (const T *)c->coef[0], (T *)c->scr,
+                                               (T *)c->dxv, nullptr, nullptr, nullptr, nullptr, c->nx, c->ny, c->nz,
+                                               it, nullptr, lst[0], nlst[0])));
+            if (c->dim == 3) {
+                KT(c, "ccd_y", (launch_ccd_pass<T>(c->st, 1, 3, false, phi, (const T *)c->coef[1], (T *)c->scr,
+                                                   (T *)c->dyv, nullptr, nullptr, nullptr, nullptr, c->nx, c->ny,
+                                                   c->nz, it, nullptr, lst[1], nlst[1])));
+                KT(c, "ccd_z", (launch_ccd_pass<T>(c->st, 2, 3, true, phi, (const T *)c->coef[2], (T *)c->scr,
+                                                   nullptr, (const T *)c->dxv, (const T *)c->dyv, (T *)c->gr, psolve,
+                                                   c->nx, c->ny, c->nz, it, &nblk, lst[2], nlst[2])));
+            } else {
+                KT(c, "ccd_y", (launch_ccd_pass<T>(c->st, 1, 2, true, phi, (const T *)c->coef[1], (T *)c->scr,
+                                                   nullptr, (const T *)c->dxv, nullptr, (T *)c->gr, psolve, c->nx,
+                                                   c->ny, c->nz, it, &nblk, lst[1], nlst[1])));
+            }
+            nblk += nfixed;
+            if (nblk > c->npartial) return LSMP_E_INVALID;
+            const MassArgs ma = {imass, iter, c->fp32 ? 1 : 0, c->scal, c->hbuf};
+            if (!lst[dfin] && nblk <= MASS_FUSE_MAX && c->ncell <= MASS_FUSE_CELLS) {
+                KT(c, "mass_update", (launch_mass_update<T>(c->st, phi, (const T *)c->gr, c->ncell, (T)c->p.ls_wid,
+                                                            c->partial, nblk, ma)));
+                continue;
+            }
+            KT(c, "finalize", (launch_finalize3(c->st, c->partial, nblk, ma)));
+            const int nup = lst[dfin] ? nlst[dfin] : (int)(c->ncell / (size_t)ns[dfin]);   // no list: every line
             KT(c, "mass_update", (launch_mass_update_lines<T>(c->st, dfin, phi, (const T *)c->gr, (T)c->p.ls_wid,
-                                                              c->scal, lst[dfin], nlst[dfin], c->nx, c->ny, c->nz)));
-        else
-            KT(c, "mass_update",
-               (launch_mass_update<T>(c->st, phi, (const T *)c->gr, c->ncell, (T)c->p.ls_wid, c->scal)));
-        LSMP_HIP(hipMemcpyAsync(c->hbuf, c->scal, 5 * sizeof(double), hipMemcpyDeviceToHost, c->st));
-        LSMP_HIP(hipStreamSynchronize(c->st));
-        mass = c->hbuf[1];
-        if (c->hbuf[4] != 0.0) { rc = LSMP_E_EMPTY_BAND; break; }
-        if (std::isnan(mass) || std::isnan(c->hbuf[3])) { rc = LSMP_E_NAN; break; }
-        const double rel = std::fabs(imass - mass) / imass;
-        if (rel < 1.0e-14) break;   // the reference's exit test (mass_preserving_level_set.f90:70)
-        if (c->fp32) {
-            // FP32 bulk phi resolves the mass only to ~1e-10..1e-8 relative; stop
-            // once the correction no longer halves the defect
-            if (rel < 1.0e-10 || (iter > 1 && rel >= 0.5 * prev_rel)) break;
+                                                              c->scal, iter, lst[dfin], nup, c->nx, c->ny, c->nz)));
         }
-        prev_rel = rel;
+        LSMP_HIP(hipStreamSynchronize(c->st));
+        last = (int)c->hbuf[7];
     }
-    if (iter > 15) iter = 15;
+    if (last) iter = last;
+    mass = c->hbuf[1];
+    if (c->hbuf[4] != 0.0) rc = LSMP_E_EMPTY_BAND;
+    else if (std::isnan(mass) || std::isnan(c->hbuf[3])) rc = LSMP_E_NAN;
+    c->mass_hint = iter;
     c->stats.last_mass_iters = iter;
     if (mass_out) *mass_out = mass;
     if (n_iter) *n_iter = iter;
@@ -593,9 +600,8 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
 
 int reduce_partials(lsmp_ctx *c, int nblk, double *out3)
 {
-    launch_finalize3(c->st, c->partial, nblk, 0.0, c->scal);
+    launch_finalize3(c->st, c->partial, nblk, MassArgs{0.0, 0, 0, c->scal, c->hbuf});
     LSMP_LAUNCHED();
-    LSMP_HIP(hipMemcpyAsync(c->hbuf, c->scal, 3 * sizeof(double), hipMemcpyDeviceToHost, c->st));
     LSMP_HIP(hipStreamSynchronize(c->st));
     out3[0] = c->hbuf[0];
     out3[1] = c->hbuf[1];
@@ -910,7 +916,7 @@ int lsmp_init(const lsmp_params *params, lsmp_handle *out)
     for (int d = 1; d < c->dim; ++d) maxlines = std::max(maxlines, c->ncell / (size_t)ns[d]);
     c->npartial = (int)std::max<size_t>(1024, (maxlines + 7) / 8 + LINE_SEGMENTS * ((maxlines + 255) / 256));
     if (alloc((void **)&c->partial, (size_t)3 * c->npartial * sizeof(double))) return fail(LSMP_E_HIP);
-    if (alloc((void **)&c->scal, 8 * sizeof(double))) return fail(LSMP_E_HIP);
+    if (alloc((void **)&c->scal, SCAL_WORDS * sizeof(double))) return fail(LSMP_E_HIP);
     if (alloc((void **)&c->u64, 4 * sizeof(unsigned long long))) return fail(LSMP_E_HIP);
     if (hipHostMalloc((void **)&c->hbuf, 16 * sizeof(double), hipHostMallocDefault) != hipSuccess)
         return fail(LSMP_E_HIP);

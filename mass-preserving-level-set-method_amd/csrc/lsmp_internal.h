@@ -109,9 +109,27 @@ struct RedisArgs {
     double inv12dx, inv12dy, inv12dz, invdx, invdy, invdz, ls_wid, inv_ls_wid, rdt;
 };
 
+// The mass correction's scalars on the device: scal[0] volume, [1] mass, [2] the
+// denominator, [3] lambda, [4] 1 for an empty band, [6] the relative defect of
+// the last iteration, [7] the iteration after which the loop stops (0: it goes
+// on).  Kernels of later iterations return at once (mass_stopped), so
+// iterations can be queued ahead of the host's look at the scalars.
+constexpr int SCAL_WORDS = 8;
+__device__ inline bool mass_stopped(const double *scal, int iter)
+{
+    return iter > 1 && scal[7] != 0.0 && scal[7] < (double)iter;
+}
 struct CcdArgs {
     double dx, dy, dz, dv, ls_wid, rho_12;
     int inverse;
+    const double *scal = nullptr;   // of a mass correction, whose iteration `iter` this is
+    int iter = 0;
+};
+// what the reduction of a mass iteration's sums needs; host: pinned copy of scal
+struct MassArgs {
+    double imass;
+    int iter, fp32;
+    double *scal, *host;
 };
 
 struct VelArgs {
@@ -197,10 +215,11 @@ constexpr int LINE_SEGMENTS = 8;
 template <typename T>
 void launch_line_hsums(hipStream_t st, int dir, const T *phi, const unsigned char *lflag, int nx, int ny, int nz,
                        const CcdArgs &ca, double *partial, int *nblocks_out);
-// the mass update on the cells of the nlist listed lines of direction dir
+// the mass update on the cells of the nlist listed lines of direction dir (lines
+// null: of every line)
 template <typename T>
 void launch_mass_update_lines(hipStream_t st, int dir, T *phi, const T *gr, T ls_wid, const double *scal,
-                              const int *lines, int nlist, int nx, int ny, int nz);
+                              int iter, const int *lines, int nlist, int nx, int ny, int nz);
 
 // Lines that cross the interface band: one flag byte per line of each
 // direction (x: ny nz, y: nx nz, z: nx ny), each direction's flags starting
@@ -218,14 +237,23 @@ constexpr size_t band_flag_bytes(size_t nfx, size_t nfy, size_t nfz) { return pa
 template <typename T>
 void launch_band_lines(hipStream_t st, int dim, T *phi, int nx, int ny, int nz, double wband,
                        unsigned char *flags, unsigned *count, int *listx, int *listy, int *listz, bool clamp);
-void launch_finalize3(hipStream_t st, const double *partial, int nblk, double imass, double *scal);
+// the block sums' totals into scal and, when given, host (pinned), with lambda
+// and the stop test of a mass iteration (ma.iter > 0)
+void launch_finalize3(hipStream_t st, const double *partial, int nblk, const MassArgs &ma);
 // zero n bytes; the ordered lists and counts of the flagged lines (flags laid
 // out as band_flag_offset; one workgroup per direction)
 void launch_zero_bytes(hipStream_t st, unsigned char *p, size_t n);
 void launch_compact_lines(hipStream_t st, int dim, const unsigned char *flags, int nfx, int nfy, int nfz,
                           int *listx, int *listy, int *listz, unsigned *count);
 template <typename T>
-void launch_mass_update(hipStream_t st, T *phi, const T *gr, size_t n, T ls_wid, const double *scal);
+void launch_mass_update(hipStream_t st, T *phi, const T *gr, size_t n, T ls_wid, const double *partial, int nblk,
+                        const MassArgs &ma);
+// The update of every cell forms the totals itself up to this many block sums
+// and cells: each of its workgroups adds the sums up, which by 1,024^2 cells
+// (4,096 workgroups) costs more than the launch it saves (a correction at
+// 1,024^2: 690 us fused, 663 not; FP32 233, 216).
+constexpr int MASS_FUSE_MAX = 256;
+constexpr size_t MASS_FUSE_CELLS = (size_t)1 << 19;
 template <typename T>
 void launch_mass_vol(hipStream_t st, const T *phi, size_t n, const CcdArgs &ca, double *partial, int nblocks);
 template <typename T>

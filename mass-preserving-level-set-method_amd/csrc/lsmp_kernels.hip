@@ -987,6 +987,7 @@ __global__ __launch_bounds__(256) void k_ccd_seg(const T *__restrict__ phi, cons
     const int line = lines ? lines[Lc] : Lc;   // with a list, lane L solves listed line L of nlines
     const size_t base = (size_t)(line / lw) * (size_t)ostride + (size_t)(line % lw) * (size_t)istride;
     const size_t NL = (size_t)gridDim.x * blockDim.x;
+    if (ca.scal && mass_stopped(ca.scal, ca.iter)) return;
     const T idx = T(1) / (T)ca.dx, idx2 = T(1) / ((T)ca.dx * (T)ca.dx);
     auto ldq = [&](int q) -> T { return phi[base + (size_t)clampi(q, 0, n - 1) * (size_t)estride]; };
     // forward row b from the window f(b-1), f(b), f(b+1) = phi(b-4), phi(b-3), phi(b-2)
@@ -1171,6 +1172,7 @@ __global__ __launch_bounds__(256) void k_ccd_part(const T *__restrict__ phi, con
     T f[KC + 2];   // phi(b-4) for b = lo .. lo + KC + 1
 #pragma unroll
     for (int r = 0; r < KC + 2; ++r) f[r] = ldq(lo - 4 + r);
+    if (ca.scal && mass_stopped(ca.scal, ca.iter)) return;   // the loads are on their way
     auto rhs = [&](int r, T &rs, T &rss) {   // the row's right-hand side from f(b-1), f(b), f(b+1)
         rs = T(15.0 / 16.0) * (-f[r] + f[r + 2]) * idx;
         rss = (T(3) * f[r] - T(6) * f[r + 1] + T(3) * f[r + 2]) * idx2;
@@ -1508,41 +1510,57 @@ __global__ __launch_bounds__(256) void k_uccd_seg(const T *__restrict__ phi, T *
     }
 }
 
-// Deterministic final reduction of per-block partials (fixed order), then the
-// mass-correction multiplier lambda = (imass - mass) / sum (mass_preserving_level_set.f90:46).
-// scal: [0] vol, [1] mass, [2] denominator, [3] lambda, [4] flag (1 = empty band).
-__global__ void k_finalize3(const double *__restrict__ partial, int nblk, double imass, double *scal)
+// Totals of the per-block partials (fixed order), lambda = (imass - mass) / sum
+// (mass_preserving_level_set.f90:46) and the stop test of the iteration
+// (:70; FP32 bulk, whose phi resolves the mass only to 1e-10..1e-8 relative, stops
+// at 1e-10 or once a correction no longer halves the defect), by thread 0.
+LSMP_DEV double mass_close(const double (&acc)[3], const MassArgs &ma)
 {
+    double *const s = ma.scal;
+    const bool empty = acc[2] == 0.0;
+    const double lam = empty ? 0.0 : (ma.imass - acc[1]) / acc[2];
+    const double rel = fabs(ma.imass - acc[1]) / ma.imass;
+    bool stop = empty || isnan(acc[1]) || isnan(lam) || rel < 1.0e-14;
+    if (ma.fp32) stop = stop || rel < 1.0e-10 || (ma.iter > 1 && rel >= 0.5 * s[6]);
+    const double v[SCAL_WORDS] = {acc[0], acc[1], acc[2], lam, empty ? 1.0 : 0.0, 0.0, rel, stop ? (double)ma.iter : 0.0};
+    for (int q = 0; q < SCAL_WORDS; ++q) {
+        s[q] = v[q];
+        if (ma.host) ma.host[q] = v[q];
+    }
+    return lam;
+}
+__global__ void k_finalize3(const double *__restrict__ partial, int nblk, MassArgs ma)
+{
+    if (mass_stopped(ma.scal, ma.iter)) return;
+    double acc[3];
+    sum_partials3(partial, nblk, acc);
+    if (threadIdx.x == 0) mass_close(acc, ma);
+}
+
+// phi += lambda delta |grad phi| (mass_preserving_level_set.f90:52-58).  Every
+// workgroup adds up the iteration's block sums itself (at most MASS_FUSE_MAX,
+// one a thread, in k_finalize3's order) instead of waiting for a launch that
+// does (7 us); the first one stores the scalars.
+template <typename T>
+__global__ __launch_bounds__(256) void k_mass_update(T *__restrict__ phi, const T *__restrict__ gr, size_t n, T ls_wid,
+                                                     const double *__restrict__ partial, int nblk, MassArgs ma)
+{
+    __shared__ double slam;
+    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const T p = q < n ? phi[q] : T(0), g = q < n ? gr[q] : T(0);
+    if (mass_stopped(ma.scal, ma.iter)) return;
     double acc[3];
     sum_partials3(partial, nblk, acc);
     if (threadIdx.x == 0) {
-        scal[0] = acc[0];
-        scal[1] = acc[1];
-        scal[2] = acc[2];
-        if (acc[2] != 0.0) {
-            scal[3] = (imass - acc[1]) / acc[2];
-            scal[4] = 0.0;
-        } else {
-            scal[3] = 0.0;
-            scal[4] = 1.0;
-        }
+        if (blockIdx.x == 0) slam = mass_close(acc, ma);
+        else slam = acc[2] == 0.0 ? 0.0 : (ma.imass - acc[1]) / acc[2];
     }
-}
-
-// phi += lambda delta |grad phi| (mass_preserving_level_set.f90:52-58); lambda
-// is read from device memory so the host need not round-trip it.
-template <typename T>
-__global__ void k_mass_update(T *__restrict__ phi, const T *__restrict__ gr, size_t n, T ls_wid,
-                              const double *__restrict__ scal)
-{
-    size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __syncthreads();
     if (q >= n) return;
-    const double lam = scal[3];
-    const T p = phi[q];
     double H, D;
     ls_funs_taylor((double)p, (double)ls_wid, H, D);
-    if (D == 0.0) return;   // phi + lambda 0 |grad phi| is phi: no read of |grad phi|, no store
-    phi[q] = (T)((double)p + lam * D * (double)gr[q]);
+    if (D == 0.0) return;   // phi + lambda 0 |grad phi| is phi: no store
+    phi[q] = (T)((double)p + slam * D * (double)g);
 }
 
 // The same update on the cells of the listed lines (every cell where delta can
@@ -1550,12 +1568,12 @@ __global__ void k_mass_update(T *__restrict__ phi, const T *__restrict__ gr, siz
 // t % nlist, so neighbouring lanes take neighbouring lines.
 template <typename T>
 __global__ void k_mass_update_lines(T *__restrict__ phi, const T *__restrict__ gr, T ls_wid,
-                                    const double *__restrict__ scal, const int *__restrict__ lines, int nlist, int n,
-                                    int lw, long ostride, long istride, long estride)
+                                    const double *__restrict__ scal, int iter, const int *__restrict__ lines,
+                                    int nlist, int n, int lw, long ostride, long istride, long estride)
 {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)nlist * n) return;
-    const int l = lines[t % (size_t)nlist], q = (int)(t / (size_t)nlist);
+    if (t >= (size_t)nlist * n || mass_stopped(scal, iter)) return;
+    const int at = (int)(t % (size_t)nlist), l = lines ? lines[at] : at, q = (int)(t / (size_t)nlist);
     const size_t a = (size_t)(l / lw) * (size_t)ostride + (size_t)(l % lw) * (size_t)istride +
                      (size_t)q * (size_t)estride;
     const double lam = scal[3];
@@ -2059,7 +2077,7 @@ void launch_line_hsums(hipStream_t st, int dir, const T *phi, const unsigned cha
 
 template <typename T>
 void launch_mass_update_lines(hipStream_t st, int dir, T *phi, const T *gr, T ls_wid, const double *scal,
-                              const int *lines, int nlist, int nx, int ny, int nz)
+                              int iter, const int *lines, int nlist, int nx, int ny, int nz)
 {
     if (nlist <= 0) return;
     const int n = dir == 0 ? nx : dir == 1 ? ny : nz;
@@ -2069,7 +2087,7 @@ void launch_mass_update_lines(hipStream_t st, int dir, T *phi, const T *gr, T ls
     const long estride = dir == 0 ? 1 : dir == 1 ? (long)nx : (long)nx * ny;
     const size_t total = (size_t)nlist * n;
     hipLaunchKernelGGL((k_mass_update_lines<T>), dim3(nblk(total, 256)), dim3(256), 0, st, phi, gr, ls_wid, scal,
-                       lines, nlist, n, lw, ostride, istride, estride);
+                       iter, lines, nlist, n, lw, ostride, istride, estride);
 }
 
 template <typename T>
@@ -2102,9 +2120,9 @@ void launch_uccd_pass(hipStream_t st, int dir, int mode, int stage, const T *phi
 #undef LSMP_UCCD
 }
 
-void launch_finalize3(hipStream_t st, const double *partial, int nblk_, double imass, double *scal)
+void launch_finalize3(hipStream_t st, const double *partial, int nblk_, const MassArgs &ma)
 {
-    hipLaunchKernelGGL(k_finalize3, dim3(1), dim3(1024), 0, st, partial, nblk_, imass, scal);
+    hipLaunchKernelGGL(k_finalize3, dim3(1), dim3(1024), 0, st, partial, nblk_, ma);
 }
 
 template <typename T>
@@ -2139,9 +2157,12 @@ void launch_compact_lines(hipStream_t st, int dim, const unsigned char *flags, i
 }
 
 template <typename T>
-void launch_mass_update(hipStream_t st, T *phi, const T *gr, size_t n, T ls_wid, const double *scal)
+void launch_mass_update(hipStream_t st, T *phi, const T *gr, size_t n, T ls_wid, const double *partial, int nblk_,
+                        const MassArgs &ma)
 {
-    hipLaunchKernelGGL((k_mass_update<T>), dim3(nblk(n, 256)), dim3(256), 0, st, phi, gr, n, ls_wid, scal);
+    static_assert(MASS_FUSE_MAX <= 256, "a block sum per thread");
+    hipLaunchKernelGGL((k_mass_update<T>), dim3(nblk(n, 256)), dim3(256), 0, st, phi, gr, n, ls_wid, partial, nblk_,
+                       ma);
 }
 
 template <typename T>
@@ -2232,11 +2253,12 @@ void launch_zero_u64(hipStream_t st, unsigned long long *p, int n)
                                      const int *, int);                                                        \
     template void launch_line_hsums<T>(hipStream_t, int, const T *, const unsigned char *, int, int, int,          \
                                        const CcdArgs &, double *, int *);                                      \
-    template void launch_mass_update_lines<T>(hipStream_t, int, T *, const T *, T, const double *, const int *,   \
-                                              int, int, int, int);                                             \
+    template void launch_mass_update_lines<T>(hipStream_t, int, T *, const T *, T, const double *, int,            \
+                                              const int *, int, int, int, int);                                \
     template void launch_band_lines<T>(hipStream_t, int, T *, int, int, int, double, unsigned char *,            \
                                        unsigned *, int *, int *, int *, bool);                                 \
-    template void launch_mass_update<T>(hipStream_t, T *, const T *, size_t, T, const double *);               \
+    template void launch_mass_update<T>(hipStream_t, T *, const T *, size_t, T, const double *, int,             \
+                                        const MassArgs &);                                                     \
     template void launch_mass_vol<T>(hipStream_t, const T *, size_t, const CcdArgs &, double *, int);           \
     template void launch_l1<T>(hipStream_t, const T *, const T *, size_t, double, double *, int);              \
     template void launch_velocity<T>(hipStream_t, T *, T *, T *, const VelArgs &, double *);                  \

@@ -895,7 +895,7 @@ int residual(lsmp_ctx *c, double band_cells, double *res, int pending = 0, doubl
                            (const T *)c->S0, ra, band_cells * c->p.dx, c->partial, (const T *)c->phiB, ctl,
                            pending);
     NET_HIP(hipGetLastError());
-    launch_finalize3(c->st, c->partial, (int)b, 0.0, c->scal);
+    launch_finalize3(c->st, c->partial, (int)b, MassArgs{0.0, 0, 0, c->scal, nullptr});
     NET_HIP(hipGetLastError());
     NET_HIP(hipMemcpyAsync(c->hbuf, c->scal, 2 * sizeof(double), hipMemcpyDeviceToHost, c->st));
     if (ctl)
