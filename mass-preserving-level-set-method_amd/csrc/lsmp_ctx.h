@@ -35,6 +35,7 @@ struct lsmp_ctx {
     double *vtab = nullptr;   // per-axis sine tables of the analytic velocity
     unsigned long long *u64 = nullptr;
     unsigned long long *rctl = nullptr;   // pseudo-time loop control block
+    int redis_hint[2] = {0, 0};           // pseudo-steps the last run took, by btn
     int rset = 0;                         // the last queued pseudo-step's set of its words
     double *hbuf = nullptr;   // pinned readback
     int npartial = 0;

@@ -301,6 +301,6 @@ template <typename T>
 void launch_energy_sums(hipStream_t st, int dim, bool vof_marker, const T *phi, const T *vof, const T *u, const T *v,
                         const T *w, const T *ten, const EnergyArgs &ea, double *partial, int nblocks);
 void launch_energy_finalize(hipStream_t st, const double *partial, int nblk, double dx, double *out);
-void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, RedisStep last);
+void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, RedisStep last, unsigned long long *host);
 
 }  // namespace lsmp

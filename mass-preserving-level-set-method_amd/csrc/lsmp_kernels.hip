@@ -882,11 +882,12 @@ __global__ void k_sign_init(const T *__restrict__ phi, T *__restrict__ S0, size_
 // NaN never stops the loop, as in the reference); the time limit is the host's
 // count of launched steps.  Stage kernels return at once when the flag is
 // set, so steps can be queued ahead without host round trips and the step
-// count stays the reference's.  One wave.
-__global__ void k_redis_ctl(unsigned long long *ctl, RedisStep last)
+// count stays the reference's.  One wave;
+// host: the control words' pinned copy.
+__global__ void k_redis_ctl(unsigned long long *ctl, RedisStep last, unsigned long long *host)
 {
     const int t = threadIdx.x;   // stripe t
-    if (ctl[1]) return;
+    const unsigned long long stopped = ctl[1], run = ctl[2], kept = ctl[3];
     // non-negative doubles (and a NaN, whose bits order above them) keep their
     // order as integers: the max of the bit patterns
     unsigned long long m = *ctl_slot(ctl, last, (unsigned)t);
@@ -895,10 +896,15 @@ __global__ void k_redis_ctl(unsigned long long *ctl, RedisStep last)
         const unsigned long long o = __shfl_xor(m, d, 64);
         m = o > m ? o : m;
     }
-    if (t == 0) {
+    if (t != 0) return;
+    const bool now = __longlong_as_double((long long)m) <= 1.0e-6;
+    if (!stopped) {
         ctl[3] = m;
-        if (__longlong_as_double((long long)m) <= 1.0e-6) ctl[1] = 1;
+        if (now) ctl[1] = 1;
     }
+    host[1] = stopped || now;
+    host[2] = run;
+    host[3] = stopped ? kept : m;
 }
 
 // Godunov |grad phi| of every interior cell from global loads, reduced to a
@@ -2226,10 +2232,10 @@ void launch_convert(hipStream_t st, TO *out, const TI *in, size_t n)
     hipLaunchKernelGGL((k_convert<TO, TI>), dim3(nblk(n, 256)), dim3(256), 0, st, out, in, n);
 }
 
-void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, RedisStep last)
+void launch_redis_ctl(hipStream_t st, unsigned long long *ctl, RedisStep last, unsigned long long *host)
 {
     static_assert(CTL_SLOTS == 64, "one wave, a stripe per lane");
-    hipLaunchKernelGGL(k_redis_ctl, dim3(1), dim3(CTL_SLOTS), 0, st, ctl, last);
+    hipLaunchKernelGGL(k_redis_ctl, dim3(1), dim3(CTL_SLOTS), 0, st, ctl, last, host);
 }
 
 void launch_zero_u64(hipStream_t st, unsigned long long *p, int n)
