@@ -151,6 +151,14 @@ LSMP_DEV double sqrt_w(double x)
     return x > 0.0 ? r : 0.0;
 }
 LSMP_DEV float sqrt_w(float x) { return __builtin_amdgcn_sqrtf(x); }
+// the same to an ulp: a second step in FP64, the rounded square root in FP32
+LSMP_DEV double sqrt_n(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x), h = 0.5 * y, s = x * y;
+    const double r = fma(fma(-s, s, x), h, s);
+    return x > 0.0 ? fma(fma(-r, r, x), h, r) : 0.0;
+}
+LSMP_DEV float sqrt_n(float x) { return sqrt(x); }
 
 // The same two rows with the weight divisions folded into one reciprocal:
 // with e_k = EPS + b_k and tau = |b3 - b1| the reference's
@@ -315,25 +323,6 @@ LSMP_DEV void weno_hj_pm_fast(T m3, T m2, T m1, T c, T p1, T p2, T p3, T inv12d,
     dm = a - invd * phyn_fast(sm2, sm1, s0, sp1, qm, qp);
 }
 
-// ls_funs with the divisions by ls_wid and pi replaced by products with
-// precomputed reciprocals.
-template <typename T> LSMP_DEV void ls_funs_fast(T phi, T inv_w, T &H, T &D)
-{
-    const T eps = T(1.0e-12);
-    const T pi = T(3.141592653589793238462643383279502884);
-    const T inv_pi = T(0.318309886183790671537767526745028724);
-    T x = phi * inv_w;
-    if (x > T(1) - eps) {
-        H = T(1); D = T(0);
-    } else if (x < T(-1) + eps) {
-        H = T(0); D = T(0);
-    } else {
-        H = T(0.5) * ((T(1) + x) + sin(pi * x) * inv_pi);
-        D = T(0.5) * (T(1) + cos(pi * x)) * inv_w;
-    }
-    H = fmax(fmin(H, T(1)), T(0));
-}
-
 // H and delta of ls_funs in FP64 without library calls: with theta = pi x / 2
 // in (-pi/2, pi/2) for a cell of the band (x = phi / w), delta = cos(theta)^2 / w
 // and sin(pi x) = 2 sin(theta) cos(theta), sine and cosine from their Taylor
@@ -405,6 +394,66 @@ LSMP_DEV T godunov(T xs1, T xs2, T ys1, T ys2, T zs1, T zs2, T s0)
         if (s0 >= T(0)) return sqrt(sq(fmax(upm, ump)) + sq(fmax(vpm, vmp)));
         return sqrt(sq(fmax(upp, umm)) + sq(fmax(vpp, vmm)));
     }
+}
+
+// delta != 0 only where ls_funs takes its middle branch
+template <typename T> LSMP_DEV bool in_band_x(T x)
+{
+    return !(x > T(1) - T(1.0e-12)) && !(x < T(-1) + T(1.0e-12));
+}
+
+// delta of ls_funs for a cell of the band (its middle branch, |x| < 1 with
+// x = phi / ls_wid): 0.5 (1 + cos(pi x)) / ls_wid = cos(theta)^2 / ls_wid with
+// theta = pi x / 2 in (-pi/2, pi/2), cos from its Taylor series in theta^2 to
+// the term in theta^20 (remainder below 2e-17 there).  Within 2.3e-16 of
+// 0.5 (1 + cos(pi x)) evaluated with a correctly rounded cosine.
+template <typename T> LSMP_DEV T band_delta(T phi, T inv_w)
+{
+    const T th = (phi * inv_w) * T(1.570796326794896619231321691639751442);
+    const T t = th * th;
+    T c = T(1.0 / 2432902008176640000.0);     // 1/20!
+    c = fma(c, t, T(-1.0 / 6402373705728000.0));   // -1/18!
+    c = fma(c, t, T(1.0 / 20922789888000.0));      // 1/16!
+    c = fma(c, t, T(-1.0 / 87178291200.0));        // -1/14!
+    c = fma(c, t, T(1.0 / 479001600.0));           // 1/12!
+    c = fma(c, t, T(-1.0 / 3628800.0));            // -1/10!
+    c = fma(c, t, T(1.0 / 40320.0));               // 1/8!
+    c = fma(c, t, T(-1.0 / 720.0));                // -1/6!
+    c = fma(c, t, T(1.0 / 24.0));                  // 1/4!
+    c = fma(c, t, T(-0.5));                        // -1/2!
+    c = fma(c, t, T(1));
+    return c * c * inv_w;
+}
+
+// Godunov |grad phi| (level_set_rk3_redis.f90:341-360) from the one-sided
+// slopes times 6 dx, 6 dy, 6 dz (2D: without the last pair); k = 1 / (6 dx), ...: with sigma the sign of
+// S0, max(-min(D+, 0), max(D-, 0)) is max(-sigma D+, sigma D-, 0) per direction
+// (and max(max(D+, 0), -min(D-, 0)) the same with sigma = -1).  Where S0 is a
+// zero of either sign the pseudo-time right-hand side S0 (|grad| - 1) is zero.
+template <typename T>
+LSMP_DEV T godunov_sig(T xp, T xm, T yp, T ym, T zp, T zm, T s0, T kx, T ky, T kz)
+{
+    const T sx = copysign(kx, s0), sy = copysign(ky, s0), sz = copysign(kz, s0);
+    const T gx = fmax(fmax(-(sx * xp), sx * xm), T(0));
+    const T gy = fmax(fmax(-(sy * yp), sy * ym), T(0));
+    const T gz = fmax(fmax(-(sz * zp), sz * zm), T(0));
+    return sqrt_w(sq(gx) + sq(gy) + sq(gz));
+}
+
+template <typename T> LSMP_DEV T godunov_sig(T xp, T xm, T yp, T ym, T s0, T kx, T ky)
+{
+    const T sx = copysign(kx, s0), sy = copysign(ky, s0);
+    const T gx = fmax(fmax(-(sx * xp), sx * xm), T(0));
+    const T gy = fmax(fmax(-(sy * yp), sy * ym), T(0));
+    return sqrt_n(sq(gx) + sq(gy));
+}
+
+// The stage's new value from the pseudo-time RHS l (Shu-Osher form).
+template <typename T, int STAGE> LSMP_DEV T rk_stage(T phi_c, T p0, T l, T rdt)
+{
+    if (STAGE == 1) return phi_c - rdt * l;
+    if (STAGE == 2) return T(0.75) * p0 + T(0.25) * (phi_c - rdt * l);
+    return p0 * T(1.0 / 3.0) + T(2.0 / 3.0) * (phi_c - rdt * l);
 }
 
 // Smoothed Heaviside and delta (ns_solver/others.f90:18-31).

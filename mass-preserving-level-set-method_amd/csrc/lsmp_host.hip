@@ -470,9 +470,9 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
                     }
                 }
             } else {
-                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 1, btn, cur, b, cur, S0, ra, ctl, step)));
-                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 2, btn, b, cc, cur, S0, ra, ctl, step)));
-                KT(c, "redis_stage", (launch_redis_stage2d<T>(c->st, 3, btn, cc, b, cur, S0, ra, ctl, step)));
+                KT(c, "redis_stage", (launch_redis2d<T>(c->st, 1, btn, cur, b, cur, S0, ra, ctl, step)));
+                KT(c, "redis_stage", (launch_redis2d<T>(c->st, 2, btn, b, cc, cur, S0, ra, ctl, step)));
+                KT(c, "redis_stage", (launch_redis2d<T>(c->st, 3, btn, cc, b, cur, S0, ra, ctl, step)));
             }
             // the new phi is in b; the old one becomes a spare
             c->phiB = c->phi;

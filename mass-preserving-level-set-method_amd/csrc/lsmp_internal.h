@@ -24,14 +24,6 @@ constexpr int KCC = 17;   // CCD rows per lane at most (9 up to 284 cells, 17 up
 #endif
 constexpr int PART_MAX_LISTED_X = LSMP_PART_LISTED_X, PART_MAX_LISTED_STRIDED = LSMP_PART_LISTED_STRIDED;
 
-// reinitialisation tile: RTX x RTY interior cells, one ring for the lambda
-// box, four for the WENO-HJ stencil; RKC planes per workgroup in z
-constexpr int RTX = 32, RTY = 16;
-constexpr int REX = RTX + 2, REY = RTY + 2;
-constexpr int RPX = RTX + 8, RPY = RTY + 8;
-constexpr int RNT = 640;
-static_assert(REX * REY <= RNT, "reinit tile needs one thread per ring cell");
-
 // 3D reinitialisation tile: R3X x R3Y interior cells, one thread each (a
 // 4-wave workgroup); at most RKC planes per workgroup in z.
 #ifndef LSMP_R3Y
@@ -197,8 +189,8 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
 template <typename T>
 void launch_combine_markers(hipStream_t st, const T *m1, const T *m2, T *phi, size_t n, unsigned *flag);
 template <typename T>
-void launch_redis_stage2d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
-                          const RedisArgs &ra, unsigned long long *ctl, RedisStep step);
+void launch_redis2d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
+                    const RedisArgs &ra, unsigned long long *ctl, RedisStep step);
 template <typename T> void launch_sign_init(hipStream_t st, const T *phi, T *S0, size_t n, T ls_wid, int raw);
 template <typename T>
 void launch_grad_max(hipStream_t st, int dim, const T *phi, const T *S0, const RedisArgs &ra,

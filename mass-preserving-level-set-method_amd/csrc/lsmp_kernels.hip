@@ -696,173 +696,6 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
 }
 
 
-// ---------------------------------------------------------------------------
-// Reinitialisation stage, 2D (level_set_rk3_redis.f90:176-264 with the
-// gradient :266-369, lambda :371-454 and ls_funs ns_solver/others.f90:1-45);
-// the 3D stage is in lsmp_redis.hip.
-// ---------------------------------------------------------------------------
-
-// Extended-tile position (row ey, column ex) of ring cell number u of a
-// TX x TY tile + 1 ring: the top and bottom rows, then the left and right
-// columns.
-template <int TX, int TY> LSMP_DEV void ext_ring_pos(int u, int &ey, int &ex)
-{
-    constexpr int EX = TX + 2, EY = TY + 2;
-    if (u < EX) { ey = 0; ex = u; }
-    else if (u < 2 * EX) { ey = EY - 1; ex = u - EX; }
-    else if (u < 2 * EX + TY) { ey = 1 + u - 2 * EX; ex = 0; }
-    else { ey = 1 + u - 2 * EX - TY; ex = EX - 1; }
-}
-
-// Thread t's cell of the extended 2D tile: tile cells first, ring after them.
-LSMP_DEV void ext_pos(int t, int &ey, int &ex)
-{
-    if (t < RTX * RTY) { ex = 1 + t % RTX; ey = 1 + t / RTX; }
-    else if (t < REX * REY) ext_ring_pos<RTX, RTY>(t - RTX * RTY, ey, ex);
-    else { ex = 0; ey = 0; }
-}
-
-// delta(phi) != 0 exactly where ls_funs_fast takes its middle branch
-template <typename T> LSMP_DEV bool in_band(T x)
-{
-    return !(x > T(1) - T(1.0e-12)) && !(x < T(-1) + T(1.0e-12));
-}
-
-// 2D stage: one tile, no marching (Disk/ and Vortex2D/ forms: |grad| without
-// z, lambda box 3x3 with centre weight 17, Disk/...redis.f90:357-361, 434-438).
-// The tile's RTX x RTY cells and the ring around them (the lambda box) need
-// D+ and D- in x and y.  Each WENO-HJ face m+1/2 gives the P term of cell m
-// and the Q term of cell m+1 (weno_hj_face), so the workgroup forms every
-// face once -- x faces i+1/2 for i = i0-2 .. i0+RTX on the REY ring rows, y
-// faces j+1/2 for j = j0-2 .. j0+RTY on the REX ring columns, two faces a
-// thread -- into LDS, and each cell of the tile and ring reads its four terms
-// there.
-constexpr int R2FX = (RTX + 3) * REY;   // x faces
-constexpr int R2F = R2FX + REX * (RTY + 3);   // and y faces
-static_assert(R2F <= 2 * RNT, "two faces a thread");
-
-template <typename T, int STAGE, int BTN>
-__global__ __launch_bounds__(RNT) void k_redis_stage2d(const T *__restrict__ phi, T *__restrict__ phi_out,
-                                                       const T *__restrict__ phi0, const T *__restrict__ S0,
-                                                       RedisArgs ra, unsigned long long *ctl, RedisStep step)
-{
-    __shared__ T sphi[RPY][RPX];
-    __shared__ T fplus[R2F], fminus[R2F];   // P and Q of the faces
-    __shared__ T ss2[REY][REX];
-    __shared__ T ss3[REY][REX];
-    const int nx = ra.nx, ny = ra.ny;
-    const T kx = (T)(2.0 * ra.inv12dx), ky = (T)(2.0 * ra.inv12dy);
-    const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt;
-    const int t = threadIdx.x;
-    const int i0 = blockIdx.x * RTX, j0 = blockIdx.y * RTY;
-    const bool ext = t < REX * REY;
-    int ex, ey;
-    ext_pos(t, ey, ex);   // tile cells on whole waves, the ring after them
-    const int gi = clampi(i0 - 1 + ex, 0, nx - 1), gj = clampi(j0 - 1 + ey, 0, ny - 1);
-    const bool inner = t < RTX * RTY && (i0 - 1 + ex) < nx && (j0 - 1 + ey) < ny;
-    const int pc = gi - (i0 - 4), pr = gj - (j0 - 4);
-    for (int idx = t; idx < RPX * RPY; idx += RNT) {
-        int c = idx % RPX, r = idx / RPX;
-        int gx = clampi(i0 - 4 + c, 0, nx - 1), gy = clampi(j0 - 4 + r, 0, ny - 1);
-        sphi[r][c] = phi[(size_t)gy * nx + gx];
-    }
-    const T s0_p = ext ? S0[(size_t)gj * nx + gi] : T(0);
-    // the pseudo-time loop has stopped
-    if (STAGE == 1 ? redis_begin_step(ctl, step, (blockIdx.x | blockIdx.y) == 0) : ctl[1] != 0) return;
-    __syncthreads();
-    // the faces: x face f (< R2FX) at ring row f / (RTX + 3), cell i0 - 2 + f % (RTX + 3);
-    // y face g = f - R2FX at cell j0 - 2 + g / REX, ring column g % REX.  Past
-    // the domain edge the LDS plane holds the boundary cell, as the ghosts do.
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int f = t + h * RNT;
-        if (f < R2F) {
-            const bool fx = f < R2FX;
-            const int g = fx ? f : f - R2FX;
-            const int r = fx ? g / (RTX + 3) + 3 : g / REX + 2;   // LDS row of the face's cell m
-            const int c = fx ? g % (RTX + 3) + 2 : g % REX + 3;   // and column
-            const int st = fx ? 1 : RPX;
-            const T *v = &sphi[r][c];
-            const T vm2 = v[-2 * st], vm1 = v[-st], v0 = v[0], vp1 = v[st], vp2 = v[2 * st], vp3 = v[3 * st];
-            const T sa = vm2 - T(2) * vm1 + v0, sb = vm1 - T(2) * v0 + vp1, sc = v0 - T(2) * vp1 + vp2,
-                    sd = vp1 - T(2) * vp2 + vp3;
-            T P, Q;
-            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, sc - T(2) * sb + sa, P, Q);
-            fplus[f] = P;
-            fminus[f] = Q;
-        }
-    }
-    __syncthreads();
-    T grad_p = T(0), del_p = T(0), phi_p = T(0);
-    // a ring cell's gradient only enters lambda through s2, s3 = 0 where delta = 0
-    if (ext && !inner && !(BTN == 1 && in_band(sphi[pr][pc] * inv_w))) {
-        if (BTN == 1) {
-            ss2[ey][ex] = T(0);
-            ss3[ey][ex] = T(0);
-        }
-    } else if (ext) {
-        const T c0 = sphi[pr][pc];
-        // a cell past the domain edge takes the boundary cell's values (gi, gj):
-        // at ring position (cx, cy) its x faces i -/+ 1/2 are x faces
-        // cy (RTX + 3) + cx (+ 1), its y faces j -/+ 1/2 y faces cy REX + cx (+ REX)
-        const int cx = gi - i0 + 1, cy = gj - j0 + 1;
-        const int fxm = cy * (RTX + 3) + cx, fym = R2FX + cy * REX + cx;
-        auto slopes = [&](int st, T k, T P, T Q, T &dp, T &dm) {
-            const T *v = &sphi[pr][pc];
-            const T sa = v[-2 * st] - T(2) * v[-st] + c0, sb = v[-st] - T(2) * c0 + v[st],
-                    sc = c0 - T(2) * v[st] + v[2 * st];
-            const T b6 = hj_base(c0, v[st], sb, sc);
-            dp = k * (b6 + P);
-            dm = k * ((b6 + (sc - T(2) * sb + sa)) - Q);
-        };
-        T xs1, xs2, ys1, ys2;
-        slopes(1, kx, fplus[fxm + 1], fminus[fxm], xs1, xs2);
-        slopes(RPX, ky, fplus[fym + REX], fminus[fym], ys1, ys2);
-        grad_p = godunov<T, 2>(xs1, xs2, ys1, ys2, T(0), T(0), s0_p);
-        phi_p = c0;
-        if (BTN == 1) {
-            T H;
-            ls_funs_fast(c0, inv_w, H, del_p);
-            ss2[ey][ex] = del_p * s0_p * (grad_p - T(1));
-            ss3[ey][ex] = grad_p * del_p * del_p;
-        }
-    }
-    if (BTN == 1) __syncthreads();
-    double lerr = 0.0;
-    if (inner) {
-        T lam = T(0);
-        if (BTN == 1) {
-            T a = T(17) * ss2[ey][ex];
-            T b = T(17) * ss3[ey][ex];
-#pragma unroll
-            for (int jj = -1; jj <= 1; ++jj)
-#pragma unroll
-                for (int ii = -1; ii <= 1; ++ii) {
-                    a = a + ss2[ey + jj][ex + ii];
-                    b = b + ss3[ey + jj][ex + ii];
-                }
-            if (fabs(b) > T(1.0e-12)) lam = a / b * del_p;
-        }
-        const T l = (s0_p - lam) * grad_p - s0_p;
-        const size_t gidx = (size_t)gj * nx + gi;
-        T pn;
-        if (STAGE == 1) {
-            pn = phi_p - rdt * l;
-        } else if (STAGE == 2) {
-            pn = T(0.75) * phi0[gidx] + T(0.25) * (phi_p - rdt * l);
-        } else {
-            const T p0 = phi0[gidx];
-            pn = p0 * T(1.0 / 3.0) + T(2.0 / 3.0) * (phi_p - rdt * l);
-            lerr = fmax(lerr, (double)fabs(pn - p0));
-        }
-        phi_out[gidx] = pn;
-    }
-    if (STAGE == 3) {
-        double m = block_max(lerr);
-        if (t == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, step, blockIdx.y * gridDim.x + blockIdx.x), m);
-    }
-}
-
 // S0 = 2 H(phi) - 1 (level_set_redis_init, redis.f90:95-109) or S0 = phi for
 // btn = 0 (level_set_redis_stable, :123-135).
 template <typename T>
@@ -1961,17 +1794,6 @@ void launch_tube_tiles(hipStream_t st, const T *phi, int nx, int ny, int nz, dou
 }
 
 template <typename T>
-void launch_redis_stage2d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
-                          const RedisArgs &ra, unsigned long long *ctl, RedisStep step)
-{
-    const dim3 g(nblk(ra.nx, RTX), nblk(ra.ny, RTY), 1);
-#define LSMP_R2(S, B) hipLaunchKernelGGL((k_redis_stage2d<T, S, B>), g, dim3(RNT), 0, st, phi, phi_out, phi0, S0, ra, ctl, step)
-    if (btn) { if (stage == 1) LSMP_R2(1, 1); else if (stage == 2) LSMP_R2(2, 1); else LSMP_R2(3, 1); }
-    else { if (stage == 1) LSMP_R2(1, 0); else if (stage == 2) LSMP_R2(2, 0); else LSMP_R2(3, 0); }
-#undef LSMP_R2
-}
-
-template <typename T>
 void launch_sign_init(hipStream_t st, const T *phi, T *S0, size_t n, T ls_wid, int raw)
 {
     hipLaunchKernelGGL((k_sign_init<T>), dim3(nblk(n, 256)), dim3(256), 0, st, phi, S0, n, ls_wid, raw);
@@ -2247,8 +2069,6 @@ void launch_zero_u64(hipStream_t st, unsigned long long *p, int n)
     template void launch_adv_pass<T>(hipStream_t, int, int, int, T *, const T *, T *, T *, T *, T *, int, int, int, \
                                      T, T, const int *, int, const TubeMask &);                                \
     template void launch_combine_markers<T>(hipStream_t, const T *, const T *, T *, size_t, unsigned *);         \
-    template void launch_redis_stage2d<T>(hipStream_t, int, int, const T *, T *, const T *, const T *,             \
-                                          const RedisArgs &, unsigned long long *, RedisStep);                 \
     template void launch_tube_tiles<T>(hipStream_t, const T *, int, int, int, double, unsigned char *);          \
     template void launch_sign_init<T>(hipStream_t, const T *, T *, size_t, T, int);                            \
     template void launch_grad_max<T>(hipStream_t, int, const T *, const T *, const RedisArgs &,                \

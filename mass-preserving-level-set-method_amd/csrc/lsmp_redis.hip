@@ -70,58 +70,6 @@ LSMP_DEV void halo_cell(int t, int &r, int &c)
     else { const int u = t - 8 * P3X; r = 4 + u / 8; c = u % 8 < 4 ? u % 8 : P3X - 8 + u % 8; }
 }
 
-// delta != 0 only where ls_funs_fast takes its middle branch
-template <typename T> LSMP_DEV bool in_band_x(T x)
-{
-    return !(x > T(1) - T(1.0e-12)) && !(x < T(-1) + T(1.0e-12));
-}
-
-// delta of ls_funs for a cell of the band (its middle branch, |x| < 1 with
-// x = phi / ls_wid): 0.5 (1 + cos(pi x)) / ls_wid = cos(theta)^2 / ls_wid with
-// theta = pi x / 2 in (-pi/2, pi/2), cos from its Taylor series in theta^2 to
-// the term in theta^20 (remainder below 2e-17 there).  Within 2.3e-16 of
-// 0.5 (1 + cos(pi x)) evaluated with a correctly rounded cosine.
-template <typename T> LSMP_DEV T band_delta(T phi, T inv_w)
-{
-    const T th = (phi * inv_w) * T(1.570796326794896619231321691639751442);
-    const T t = th * th;
-    T c = T(1.0 / 2432902008176640000.0);     // 1/20!
-    c = fma(c, t, T(-1.0 / 6402373705728000.0));   // -1/18!
-    c = fma(c, t, T(1.0 / 20922789888000.0));      // 1/16!
-    c = fma(c, t, T(-1.0 / 87178291200.0));        // -1/14!
-    c = fma(c, t, T(1.0 / 479001600.0));           // 1/12!
-    c = fma(c, t, T(-1.0 / 3628800.0));            // -1/10!
-    c = fma(c, t, T(1.0 / 40320.0));               // 1/8!
-    c = fma(c, t, T(-1.0 / 720.0));                // -1/6!
-    c = fma(c, t, T(1.0 / 24.0));                  // 1/4!
-    c = fma(c, t, T(-0.5));                        // -1/2!
-    c = fma(c, t, T(1));
-    return c * c * inv_w;
-}
-
-// Godunov |grad phi| (level_set_rk3_redis.f90:341-360) from the one-sided
-// slopes times 6 dx, 6 dy, 6 dz; k = 1 / (6 dx), ...: with sigma the sign of
-// S0, max(-min(D+, 0), max(D-, 0)) is max(-sigma D+, sigma D-, 0) per direction
-// (and max(max(D+, 0), -min(D-, 0)) the same with sigma = -1).  Where S0 is a
-// zero of either sign the pseudo-time right-hand side S0 (|grad| - 1) is zero.
-template <typename T>
-LSMP_DEV T godunov_sig(T xp, T xm, T yp, T ym, T zp, T zm, T s0, T kx, T ky, T kz)
-{
-    const T sx = copysign(kx, s0), sy = copysign(ky, s0), sz = copysign(kz, s0);
-    const T gx = fmax(fmax(-(sx * xp), sx * xm), T(0));
-    const T gy = fmax(fmax(-(sy * yp), sy * ym), T(0));
-    const T gz = fmax(fmax(-(sz * zp), sz * zm), T(0));
-    return sqrt_w(sq(gx) + sq(gy) + sq(gz));
-}
-
-// The stage's new value from the pseudo-time RHS l (Shu-Osher form).
-template <typename T, int STAGE> LSMP_DEV T rk_stage(T phi_c, T p0, T l, T rdt)
-{
-    if (STAGE == 1) return phi_c - rdt * l;
-    if (STAGE == 2) return T(0.75) * p0 + T(0.25) * (phi_c - rdt * l);
-    return p0 * T(1.0 / 3.0) + T(2.0 / 3.0) * (phi_c - rdt * l);
-}
-
 // Element of a plane at a byte offset: the plane's address, the same in every
 // lane, stays in scalar registers and the offset in one vector register (the
 // empty statements, here and on the offsets in the plane loop, keep the
