@@ -38,6 +38,8 @@ struct lsmp_ctx {
     int redis_hint[2] = {0, 0};           // pseudo-steps the last run took, by btn
     int rset = 0;                         // the last queued pseudo-step's set of its words
     double *hbuf = nullptr;   // pinned readback
+    char *hstage = nullptr;   // pinned, two halves of hstage_rows rows: fields read out
+    size_t hstage_rows = 0;
     int npartial = 0;
     int mass_hint = 2;               // iterations the last mass correction took
     int band_lines = 1;              // mass correction on band lines: 0 never, 1 where it pays, 2 always
