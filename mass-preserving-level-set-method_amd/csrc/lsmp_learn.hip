@@ -24,6 +24,7 @@
 namespace lsmp {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int NF = 128;      // 125 stencil values, the centre value, 2 zeros
@@ -35,6 +36,7 @@ constexpr int OFF_B2 = OFF_W2 + NH * NH;
 constexpr int OFF_W3 = OFF_B2 + NH;          // W3[k], k < NH
 constexpr int OFF_B3 = OFF_W3 + NH;
 constexpr int NPARAM = OFF_B3 + 1;           // 12481
+constexpr int PART_PITCH = (NPARAM + 31) / 32 * 32;   // of the workgroups' gradients: whole 128-byte lines
 constexpr int TILE = 64;                     // samples per workgroup (4 waves x 16)
 // LDS row pitches (in bf16) of the MFMA operand tiles: 16 bytes past a
 // multiple of the bank width, so that the 16 rows a lane group reads at once
@@ -315,24 +317,51 @@ struct NetLds {
     float b3;
 };
 
-// w2: optional [n1][n2] copy of the hi part of W2 for the backward pass.
+// The weights into LDS, by a workgroup of 256.  w2: optional [n1][n2] copy of the
+// hi part of W2 for the backward pass.  A thread takes eight inputs k of one
+// neuron: its 48 loads (256 coalesced bytes a wave each) are in flight together,
+// and eight values are one 16-byte LDS store.
 LSMP_DEV void stage_weights(NetLds &L, const float *__restrict__ P, __bf16 (*w2)[KP2])
 {
-    for (int idx = threadIdx.x; idx < NF * NH; idx += blockDim.x) {
-        const int k = idx / NH, n = idx % NH;
-        split_bf16(P[OFF_W1 + idx], L.w1h[n][k], L.w1l[n][k]);
+    const int n = threadIdx.x & 63, kg = threadIdx.x >> 6;
+    float a[4][8], b[2][8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[q][j] = P[OFF_W1 + (8 * (kg + 4 * q) + j) * NH + n];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) b[q][j] = P[OFF_W2 + (8 * (kg + 4 * q) + j) * NH + n];
+    const float vec = kg < 3 ? P[(kg == 0 ? OFF_B1 : kg == 1 ? OFF_B2 : OFF_W3) + n] : P[OFF_B3];
+    auto pack = [](const float (&v)[8], bf16x8 &hi, bf16x8 &lo) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            __bf16 h, l;
+            split_bf16(v[j], h, l);
+            hi[j] = h;
+            lo[j] = l;
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        bf16x8 hi, lo;
+        pack(a[q], hi, lo);
+        *(bf16x8 *)&L.w1h[n][8 * (kg + 4 * q)] = hi;
+        *(bf16x8 *)&L.w1l[n][8 * (kg + 4 * q)] = lo;
     }
-    for (int idx = threadIdx.x; idx < NH * NH; idx += blockDim.x) {
-        const int k = idx / NH, n = idx % NH;
-        split_bf16(P[OFF_W2 + idx], L.w2h[n][k], L.w2l[n][k]);
-        if (w2) w2[k][n] = L.w2h[n][k];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        bf16x8 hi, lo;
+        pack(b[q], hi, lo);
+        *(bf16x8 *)&L.w2h[n][8 * (kg + 4 * q)] = hi;
+        *(bf16x8 *)&L.w2l[n][8 * (kg + 4 * q)] = lo;
+        if (w2)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w2[8 * (kg + 4 * q) + j][n] = hi[j];
     }
-    for (int idx = threadIdx.x; idx < NH; idx += blockDim.x) {
-        L.b1[idx] = P[OFF_B1 + idx];
-        L.b2[idx] = P[OFF_B2 + idx];
-        L.w3[idx] = P[OFF_W3 + idx];
-    }
-    if (threadIdx.x == 0) L.b3 = P[OFF_B3];
+    if (kg < 3) (kg == 0 ? L.b1 : kg == 1 ? L.b2 : L.w3)[n] = vec;
+    else if (n == 0) L.b3 = vec;
 }
 
 // Forward pass of one wave's 16 samples.  xh/xl: the input rows in A layout
@@ -393,8 +422,8 @@ LSMP_DEV void net_forward(const NetLds &L, const bf16x8 (&xh)[4], const bf16x8 (
     for (int i = 0; i < 4; ++i) o[i] = group16_sum(p[i]) + L.b3;
 }
 
-// Rows of X for this wave in A layout, split into hi and lo parts.
-LSMP_DEV void load_rows(const float *__restrict__ X, long srow, bool valid, bf16x8 (&xh)[4], bf16x8 (&xl)[4])
+// A wave's rows of X in A layout: the loads, and the split into hi and lo parts.
+LSMP_DEV void load_rows(const float *__restrict__ X, long srow, bool valid, float (&v)[4][8])
 {
     const int l = threadIdx.x & 63, lg = l >> 4;
 #pragma unroll
@@ -404,15 +433,21 @@ LSMP_DEV void load_rows(const float *__restrict__ X, long srow, bool valid, bf16
             a = *(const float4 *)&X[srow * NF + 32 * ks + 8 * lg];
             b = *(const float4 *)&X[srow * NF + 32 * ks + 8 * lg + 4];
         }
-        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        v[ks][0] = a.x; v[ks][1] = a.y; v[ks][2] = a.z; v[ks][3] = a.w;
+        v[ks][4] = b.x; v[ks][5] = b.y; v[ks][6] = b.z; v[ks][7] = b.w;
+    }
+}
+LSMP_DEV void split_rows(const float (&v)[4][8], bf16x8 (&xh)[4], bf16x8 (&xl)[4])
+{
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             __bf16 hi, lo;
-            split_bf16(v[j], hi, lo);
+            split_bf16(v[ks][j], hi, lo);
             xh[ks][j] = hi;
             xl[ks][j] = lo;
         }
-    }
 }
 
 LSMP_DEV unsigned hash32(unsigned x)
@@ -424,9 +459,14 @@ LSMP_DEV unsigned hash32(unsigned x)
 // One training step's forward and backward pass over a minibatch: each
 // workgroup handles 64 samples and writes its gradient of
 // L = (1/B) sum w (o - y)^2, w = c^2 / (y^2 + c^2) (w = 1 for c = 0), to
-// part[blockIdx.x][NPARAM] and its loss sum to lpart[blockIdx.x].  Samples
+// part[blockIdx.x][PART_PITCH] and its loss sum to lpart[blockIdx.x].  Samples
 // are drawn with replacement by a hash of (seed, position), or taken in
-// order when `ordered` is set.
+// order when `ordered` is set.  Bound by its chain of loads, LDS relayouts and
+// barriers in one workgroup a CU (the arithmetic is under 2 us): the sample rows,
+// the labels and the weights are all in flight together, and values that lie
+// next to each other in LDS are stored in 8 or 16 bytes.  28.8 -> 15.1 us at a
+// batch of 16,384 against weights stored 2 bytes at a time in 48 rounds before the
+// first sample was loaded (a training step 35.5 -> 20.8 us; 512: 25.3 -> 12.2).
 __global__ __launch_bounds__(256) void k_net_grad(const float *__restrict__ P, const float *__restrict__ X,
                                                   const float *__restrict__ Y, unsigned nsamp, int batch,
                                                   unsigned seed, int ordered, float wc, float *__restrict__ part,
@@ -442,38 +482,44 @@ __global__ __launch_bounds__(256) void k_net_grad(const float *__restrict__ P, c
     __shared__ __attribute__((aligned(16))) __bf16 dz1t[NH][KPT];       // [n1][sample]
     __shared__ __attribute__((aligned(16))) __bf16 xt[NF][KPT];         // [feature][sample]
     __shared__ float red[4][3 * NH + 2];
-    stage_weights(L, P, w2);
-    __syncthreads();
-
     const int t = threadIdx.x, wv = t >> 6, l = t & 63, lr = l & 15, lg = l >> 4;
+    auto sample = [&](int p) {
+        return ordered ? (unsigned)p : hash32(seed * 0x9e3779b9u + (unsigned)p) % nsamp;
+    };
     const int pos = blockIdx.x * TILE + wv * 16 + lr;    // position in the minibatch of this lane's row
+    const int rpos = blockIdx.x * TILE + wv * 16 + 4 * lg;   // and of its first output row
     const bool valid = pos < batch;
-    unsigned s = 0;
-    if (valid) s = ordered ? (unsigned)pos : hash32(seed * 0x9e3779b9u + (unsigned)pos) % nsamp;
+    float xv[4][8], yv[4];
+    load_rows(X, valid ? (long)sample(pos) : 0L, valid, xv);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) yv[i] = rpos + i < batch ? Y[sample(rpos + i)] : 0.f;
+    stage_weights(L, P, w2);
     bf16x8 xh[4], xl[4];
-    load_rows(X, (long)s, valid, xh, xl);
+    split_rows(xv, xh, xl);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
         for (int j = 0; j < 8; ++j) xt[32 * ks + 8 * lg + j][wv * 16 + lr] = xh[ks][j];
+    __syncthreads();
     f32x4 z1[4], z2[4];
     float o[4];
     net_forward(L, xh, xl, sh1[wv], sl1[wv], z1, z2, o);
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < 4; ++nt) {
+        bf16x4 h;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) h1t[16 * nt + lr][wv * 16 + 4 * lg + i] = sh1[wv][4 * lg + i][16 * nt + lr];
+        for (int i = 0; i < 4; ++i) h[i] = (__bf16)silu(z1[nt][i]);
+        *(bf16x4 *)&h1t[16 * nt + lr][wv * 16 + 4 * lg] = h;
+    }
 
     // output layer: dO = 2 (o - y) / B for the rows 4*lg + i
     const float invB = 1.0f / (float)batch;
     float dO[4], lsum = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int rpos = blockIdx.x * TILE + wv * 16 + 4 * lg + i;
         float e = 0.f, w = 1.f;
-        if (rpos < batch) {
-            const unsigned rs = ordered ? (unsigned)rpos : hash32(seed * 0x9e3779b9u + (unsigned)rpos) % nsamp;
-            const float y = Y[rs];
+        if (rpos + i < batch) {
+            const float y = yv[i];
             e = o[i] - y;
             if (wc > 0.f) w = wc * wc / (y * y + wc * wc);
         }
@@ -485,15 +531,17 @@ __global__ __launch_bounds__(256) void k_net_grad(const float *__restrict__ P, c
     for (int nt = 0; nt < 4; ++nt) {
         const float w = L.w3[16 * nt + lr];
         float pw = 0.f, pb = 0.f;
+        bf16x4 dz;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float h2 = silu(z2[nt][i]);
             pw += h2 * dO[i];
             const float d = dO[i] * w * dsilu(z2[nt][i]);
             pb += d;
-            sdz2[wv][4 * lg + i][16 * nt + lr] = (__bf16)d;
-            dz2t[16 * nt + lr][wv * 16 + 4 * lg + i] = (__bf16)d;
+            dz[i] = (__bf16)d;
+            sdz2[wv][4 * lg + i][16 * nt + lr] = dz[i];
         }
+        *(bf16x4 *)&dz2t[16 * nt + lr][wv * 16 + 4 * lg] = dz;
         gw3[nt] = across_groups_sum(pw);
         gb2[nt] = across_groups_sum(pb);
     }
@@ -511,12 +559,14 @@ __global__ __launch_bounds__(256) void k_net_grad(const float *__restrict__ P, c
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) acc = mma(ad[ks], *(const bf16x8 *)&w2[16 * nt + lr][32 * ks + 8 * lg], acc);
         float pb = 0.f;
+        bf16x4 dz;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float d = acc[i] * dsilu(z1[nt][i]);
             pb += d;
-            dz1t[16 * nt + lr][wv * 16 + 4 * lg + i] = (__bf16)d;
+            dz[i] = (__bf16)d;
         }
+        *(bf16x4 *)&dz1t[16 * nt + lr][wv * 16 + 4 * lg] = dz;
         gb1[nt] = across_groups_sum(pb);
     }
     // per-wave vector gradients into LDS, summed over waves below
@@ -535,7 +585,7 @@ __global__ __launch_bounds__(256) void k_net_grad(const float *__restrict__ P, c
     }
     __syncthreads();
 
-    float *out = part + (size_t)blockIdx.x * NPARAM;
+    float *out = part + (size_t)blockIdx.x * PART_PITCH;
     // dW2 = H1^T dZ2 (64 x 64, K = 64 samples): wave wv computes rows 16 wv ..
     {
         const int mt = wv;
@@ -597,7 +647,7 @@ __global__ __launch_bounds__(UPD_P * UPD_W) void k_net_update(float *__restrict_
     const int p = blockIdx.x * UPD_P + l, pc = min(p, NPARAM - 1);
     float a = 0.f;
 #pragma unroll 16
-    for (int b = wv; b < nblk; b += UPD_W) a += part[(size_t)b * NPARAM + pc];
+    for (int b = wv; b < nblk; b += UPD_W) a += part[(size_t)b * PART_PITCH + pc];
     sum[wv][l] = a;
     if (blockIdx.x == 0 && wv == UPD_W - 1) {   // a wave sums the losses
         double s = 0.0;
@@ -787,7 +837,7 @@ int ensure_parts(lsmp_net *net, int nblk)
     if (net->lpart) (void)hipFree(net->lpart);
     net->part = nullptr;
     net->lpart = nullptr;
-    NET_HIP(hipMalloc(&net->part, (size_t)nblk * NPARAM * sizeof(float)));
+    NET_HIP(hipMalloc(&net->part, (size_t)nblk * PART_PITCH * sizeof(float)));
     NET_HIP(hipMalloc(&net->lpart, (size_t)nblk * sizeof(double)));
     net->part_blocks = nblk;
     return LSMP_OK;
