@@ -68,6 +68,7 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
     T *tg = reinterpret_cast<T *>(adv_lds);   // TL rows of rs slots: g fluxes, then g flux differences
     T *tf = tg + TL * rs;                     // the same for f, cells in reversed order
     __shared__ size_t sbase[TL];
+    __shared__ int2 stube[TL];   // i, j of a z line (the tube's lines are along z in the stage pass)
     // boundary faces: [line][0] g face 0, [1] g face n, [2] f face n, [3] f face 0
     // (the f system's start and end in its reversed order)
     __shared__ T sbc[TL][4];
@@ -78,28 +79,45 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
         const int Lc = min(L0 + tid, nlines - 1);
         const int bl = lines ? lines[Lc] : Lc;
         sbase[tid] = (size_t)(bl / lw) * (size_t)ostride + (size_t)(bl % lw) * (size_t)istride;
+        if (MODE == 2 && TUBE) stube[tid] = make_int2(bl % lw, bl / lw);
     }
     __syncthreads();
     const int ne = TL * n;
     const bool along = estride == 1;   // x lines: cells of a line are contiguous
+    // cell e of the tile: line l, cell q (the product with 1 / n is exact enough
+    // for the at most 8 x 1,025 cells)
+    const float inv_n = 1.0f / (float)n;
     auto cell_of = [&](int e, int &l, int &q) {
         if (along) {
-            l = e / n;
+            l = (int)(((float)e + 0.5f) * inv_n);
             q = e - l * n;
         } else {
             q = e / TL;
             l = e - q * TL;
         }
     };
-    // (1) split fluxes of the TL lines into the tiles
-    for (int e = tid; e < ne; e += TW * 64) {
-        int l, q;
-        cell_of(e, l, q);
-        const size_t a = sbase[l] + (size_t)q * (size_t)estride;
-        T g, f;
-        flux_split(phi[a], vel[a], g, f);
-        tg[l * rs + tpos(q)] = g;
-        tf[l * rs + tpos(n - 1 - q)] = f;
+    // (1) split fluxes of the TL lines into the tiles, the loads of U cells in flight
+    constexpr int U = 4, NT = TW * 64;
+    for (int e0 = tid; e0 < ne; e0 += U * NT) {
+        T pv[U], uv[U];
+        int at[U], rt[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            int l, q;
+            cell_of(min(e0 + i * NT, ne - 1), l, q);
+            const size_t a = sbase[l] + (size_t)q * (size_t)estride;
+            pv[i] = phi[a];
+            uv[i] = vel[a];
+            at[i] = l * rs + tpos(q);
+            rt[i] = l * rs + tpos(n - 1 - q);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {   // past the end: the last cell once more
+            T g, f;
+            flux_split(pv[i], uv[i], g, f);
+            tg[at[i]] = g;
+            tf[rt[i]] = f;
+        }
     }
     __syncthreads();
     if (tid < 4 * TL) {
@@ -214,6 +232,7 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
         // then reads its own, finite row)
 #pragma unroll
         for (int st = 1; st < 64; st <<= 1) {
+            if (st * KR >= 16 && all_uncoupled(ra, rb, rc)) break;
             const bool hasm = s - st >= 0, hasp = s + st < 64;
             const int lm = hasm ? lane - st : lane, lp = hasp ? lane + st : lane;
             const T ib = rcp_w(rb);
@@ -249,26 +268,47 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
     __syncthreads();
 
     // (3) the RHS or the RK stage of every cell of the TL lines
-    for (int e = tid; e < ne; e += TW * 64) {
-        int l, q;
-        cell_of(e, l, q);
-        if (L0 + l >= nlines) continue;
-        const size_t a = sbase[l] + (size_t)q * (size_t)estride;
-        const T t1 = tg[l * rs + tpos(q)], t2 = tf[l * rs + tpos(n - 1 - q)];
-        if (MODE == 0) {
-            R[a] = t1 + t2;
-        } else if (MODE == 1) {
-            R[a] = (R[a] + t1) + t2;
-        } else if (!TUBE || tm.in(a)) {
-            const T r = (R[a] + t1) + t2, Pv = phi[a];
-            if (STAGE == 1) {
+    constexpr int U3 = 4;
+    for (int e0 = tid; e0 < ne; e0 += U3 * NT) {
+        T t1[U3], t2[U3], Rv[U3], Pv[U3], l1[U3], l2[U3];
+        size_t at[U3];
+        bool on[U3];
+#pragma unroll
+        for (int i = 0; i < U3; ++i) {
+            int l, q;
+            cell_of(min(e0 + i * NT, ne - 1), l, q);
+            const size_t a = sbase[l] + (size_t)q * (size_t)estride;
+            at[i] = a;
+            on[i] = e0 + i * NT < ne && L0 + l < nlines;
+            if (MODE == 2 && TUBE) on[i] = on[i] && tm.in(stube[l].x, stube[l].y, q);
+            if (MODE != 0) Rv[i] = R[a];
+            if (MODE == 2) {
+                Pv[i] = phi[a];
+                if (STAGE > 1) l1[i] = L1[a];
+                if (STAGE > 2) l2[i] = L2[a];
+            }
+            t1[i] = tg[l * rs + tpos(q)];
+            t2[i] = tf[l * rs + tpos(n - 1 - q)];
+        }
+#pragma unroll
+        for (int i = 0; i < U3; ++i) {
+            if (!on[i]) continue;
+            const size_t a = at[i];
+            if (MODE == 0) {
+                R[a] = t1[i] + t2[i];
+                continue;
+            }
+            const T r = (Rv[i] + t1[i]) + t2[i];
+            if (MODE == 1) {
+                R[a] = r;
+            } else if (STAGE == 1) {
                 L1[a] = r;
-                phi[a] = Pv + r * dt;
+                phi[a] = Pv[i] + r * dt;
             } else if (STAGE == 2) {
                 L2[a] = r;
-                phi[a] = Pv + (T(-3) * L1[a] + r) / T(4) * dt;
+                phi[a] = Pv[i] + (T(-3) * l1[i] + r) / T(4) * dt;
             } else {
-                phi[a] = Pv + (-L1[a] - L2[a] + T(8) * r) / T(12) * dt;
+                phi[a] = Pv[i] + (-l1[i] - l2[i] + T(8) * r) / T(12) * dt;
             }
         }
     }

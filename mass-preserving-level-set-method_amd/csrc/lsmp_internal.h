@@ -148,6 +148,10 @@ struct TubeMask {
         const size_t i = a % (size_t)nx, r = a / (size_t)nx, j = r % (size_t)ny, k = r / (size_t)ny;
         return fx[j + (size_t)ny * k] && (!fy || fy[i + (size_t)nx * k]);
     }
+    __device__ bool in(int i, int j, int k) const
+    {
+        return !fx || (fx[j + (size_t)ny * k] && (!fy || fy[i + (size_t)nx * k]));
+    }
 };
 
 // listed strided lines solved one wave per line up to this count
