@@ -15,20 +15,25 @@
 // mirrors the stencil and exchanges A and C, which is what an f row does to a
 // g row, so the f system of a line is the g system of its reversed f fluxes,
 // with the reversed orientation's sign on the flux differences.  (2) Each
-// wave solves 2 TL / TW of the TL lines' 2 TL systems in turn (g, and f
-// reversed, both with the g rows): lane s eliminates its K = ceil((n-1)/64)
-// rows with the two neighbouring interface values as parameters,
-// X_i = p_i + q_i L + r_i R; the interface rows form a tridiagonal system
-// across the 64 lanes, solved by parallel cyclic reduction; then each lane
-// back-substitutes its rows, reading its stencils from the tiles.  (64 lanes
-// per system measured faster than 32 with both systems in one wave: fewer
-// rows per lane, 106 VGPRs instead of 144.)  The flux differences of the g and f systems go
-// back into the tiles, over the line's own fluxes, which only its wave reads.
+// wave solves 2 TL / TW of the TL lines' 2 TL systems (g, and f reversed, both
+// with the g rows), with SL lanes per system: lane s eliminates its
+// K = ceil((n-1)/SL) rows with the two neighbouring interface values as
+// parameters, X_i = p_i + q_i L + r_i R; the interface rows form a tridiagonal
+// system across the SL lanes, solved by parallel cyclic reduction; then each lane
+// back-substitutes its rows, reading its stencils from the tiles.  The flux
+// differences of the g and f systems go back into the tiles, over the line's own
+// fluxes, which only its wave reads.
 // (3) Every thread forms the RHS or the RK stage of cells of the TL lines and
 // stores them, coalesced as in (1).  Nothing goes to scratch memory: the HBM
 // traffic is the pass's own fields.  In MODE 2 the in-place update of phi is
 // safe: the stencils run along the lines, and a workgroup reads and writes
 // only its own lines.
+//
+// Bound by issue and LDS together (256^3 FP64: 57% and 39% of the time), so a
+// system is as narrow as four rows a lane allow: both of a line in one wave up
+// to 129 cells (128^3 advection 443 -> 352 us, FP32 265 -> 233), a wave per system up
+// to 257, where half the lanes with eight rows take 144 VGPRs instead of 104
+// (256^3 2256 against 2305, FP32 1290 against 1366).
 //
 // Same rows as the reference's (an f row is the g row of the mirrored stencil
 // with A and C exchanged); the solve differs from one Thomas sweep only in
@@ -57,7 +62,7 @@ static int adv_tile_row_slots(int n)
 }
 
 // TW waves per workgroup, TL lines per workgroup: 2 TL / TW systems per wave
-template <typename T, int MODE, int STAGE, int KR, bool TUBE, int TL, int TW>
+template <typename T, int MODE, int STAGE, int KR, int SL, bool TUBE, int TL, int TW>
 __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restrict__ vel, T *R, T *L1, T *L2,
                                                        int nlines, int n, int lw, long ostride, long istride,
                                                        long estride, T dd, T dt, const int *__restrict__ lines,
@@ -136,10 +141,10 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
     }
     __syncthreads();
 
-    // (2) one (line, system) at a time per wave, 64 lanes per system
+    // (2) one system at a time per wave, or both of a line (SL = 32)
     const int wave = tid >> 6, lane = tid & 63;
-    const int s = lane;
-    const int N = n - 1, K = (N + 63) / 64;
+    const int s = lane & (SL - 1);
+    const int N = n - 1, K = (N + SL - 1) / SL;
     const int lo = s * K + 1;
     const bool active = lo <= N;
     const bool last = (s + 1) * K >= N;
@@ -147,9 +152,9 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
     const int nrow = active ? hi - lo + 1 : 0;
     const bool irow = active && !last;
     const bool next_last = (s + 2) * K >= N;
-    for (int job = wave; job < 2 * TL; job += TW) {
-        const int l = job >> 1;
-        const bool isf = job & 1;
+    for (int job = wave; job < TL * (SL / 32); job += TW) {
+        const int l = SL == 32 ? job : job >> 1;
+        const bool isf = SL == 32 ? lane >= 32 : job & 1;
         const T sdd = isf ? -(T(1) / dd) : T(1) / dd;
         T *tile = (isf ? tf : tg) + l * rs;
         auto flux = [&](int c) { return tile[tpos(clampi(c - 1, 0, n - 1))]; };   // cell c = 1..n, clamped
@@ -226,27 +231,7 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
                 rc = T(0);
             }
         }
-        // parallel cyclic reduction over the 64 lanes; each lane
-        // hands its neighbours 1 / b with its row.  Past the ends of the line
-        // the neighbour is an identity row: its multiplier is zero (the lane
-        // then reads its own, finite row)
-#pragma unroll
-        for (int st = 1; st < 64; st <<= 1) {
-            if (st * KR >= 16 && all_uncoupled(ra, rb, rc)) break;
-            const bool hasm = s - st >= 0, hasp = s + st < 64;
-            const int lm = hasm ? lane - st : lane, lp = hasp ? lane + st : lane;
-            const T ib = rcp_w(rb);
-            const T am = __shfl(ra, lm, 64), im = __shfl(ib, lm, 64), cm = __shfl(rc, lm, 64), dm = __shfl(rd, lm, 64);
-            const T ap = __shfl(ra, lp, 64), ip = __shfl(ib, lp, 64), cq = __shfl(rc, lp, 64), dq = __shfl(rd, lp, 64);
-            const T k1 = hasm ? ra * im : T(0), k2 = hasp ? rc * ip : T(0);
-            const T na = -am * k1, nc = -cq * k2;
-            const T nb = rb - cm * k1 - ap * k2, nd = rd - dm * k1 - dq * k2;
-            ra = na;
-            rb = nb;
-            rc = nc;
-            rd = nd;
-        }
-        const T Xb = rd * rcp_w(rb);
+        const T Xb = pcr_solve<SL>(ra, rb, rc, rd);
         const T Xprev = __shfl(Xb, (lane - 1) & 63, 64);
         const T Lv = s == 0 ? bc0 : Xprev;
         const T Rv = last ? bcN : Xb;
@@ -321,32 +306,36 @@ void launch_adv_tile(hipStream_t st, int mode, int stage, T *phi, const T *vel, 
 {
     const int rs = adv_tile_row_slots(n);
     const bool tube = tm.fx != nullptr;
-    const bool k4 = n <= 64 * 4 + 1;   // four rows per lane suffice, else eight (up to 513 cells)
+    const bool h4 = n <= 32 * 4 + 1;   // half a wave per system and four rows a lane suffice
+    const bool k4 = n <= 64 * 4 + 1;   // else a wave per system and four, or eight (up to 513 cells)
     // lines of 514..1025 cells: sixteen rows per lane, four lines per workgroup
     const bool k16 = n > 64 * 8 + 1;
     const int tl = k16 ? 4 : 8;
     const size_t lds = 2 * (size_t)tl * rs * sizeof(T);
     const dim3 g((unsigned)((nlines + tl - 1) / tl)), b(k16 ? 8 * 64 : 4 * 64);
     // tiles of lines longer than 257 cells take more than 64 KiB of LDS (FP64)
-#define LSMP_TILEK(M, S, KR, TB, TLV, TWV)                                                                     \
+#define LSMP_TILEK(M, S, KR, SL, TB, TLV, TWV)                                                                 \
     do {                                                                                                       \
         if (lds > 65536)                                                                                       \
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_adv_tile<T, M, S, KR, TB, TLV, TWV>),  \
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_adv_tile<T, M, S, KR, SL, TB, TLV, TWV>), \
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                   \
-        hipLaunchKernelGGL((k_adv_tile<T, M, S, KR, TB, TLV, TWV>), g, b, lds, st, phi, vel, R, L1, L2, nlines, \
-                           n, lw, ostride, istride, estride, dd, dt, lines, tm, rs);                           \
+        hipLaunchKernelGGL((k_adv_tile<T, M, S, KR, SL, TB, TLV, TWV>), g, b, lds, st, phi, vel, R, L1, L2,    \
+                           nlines, n, lw, ostride, istride, estride, dd, dt, lines, tm, rs);                   \
+    } while (0)
+#define LSMP_TILET(M, S, TB)                                                                                   \
+    do {                                                                                                       \
+        if (h4) LSMP_TILEK(M, S, 4, 32, TB, 8, 4);                                                             \
+        else if (k4) LSMP_TILEK(M, S, 4, 64, TB, 8, 4);                                                        \
+        else LSMP_TILEK(M, S, 8, 64, TB, 8, 4);                                                                \
     } while (0)
 #define LSMP_TILE(M, S)                                                                                        \
     do {                                                                                                       \
-        if (k16) LSMP_TILEK(M, S, 16, false, 4, 8);                                                            \
+        if (k16) LSMP_TILEK(M, S, 16, 64, false, 4, 8);                                                        \
         else if constexpr (M == 2) {                                                                           \
-            if (k4 && tube) LSMP_TILEK(M, S, 4, true, 8, 4);                                                   \
-            else if (k4) LSMP_TILEK(M, S, 4, false, 8, 4);                                                     \
-            else if (tube) LSMP_TILEK(M, S, 8, true, 8, 4);                                                    \
-            else LSMP_TILEK(M, S, 8, false, 8, 4);                                                             \
+            if (tube) LSMP_TILET(M, S, true);                                                                  \
+            else LSMP_TILET(M, S, false);                                                                      \
         } else {                                                                                               \
-            if (k4) LSMP_TILEK(M, S, 4, false, 8, 4);                                                          \
-            else LSMP_TILEK(M, S, 8, false, 8, 4);                                                             \
+            LSMP_TILET(M, S, false);                                                                           \
         }                                                                                                      \
     } while (0)
     if (mode == 0) LSMP_TILE(0, 0);
@@ -355,6 +344,7 @@ void launch_adv_tile(hipStream_t st, int mode, int stage, T *phi, const T *vel, 
     else if (stage == 2) LSMP_TILE(2, 2);
     else LSMP_TILE(2, 3);
 #undef LSMP_TILE
+#undef LSMP_TILET
 #undef LSMP_TILEK
 }
 

@@ -141,20 +141,56 @@ LSMP_DEV double rcp_w(double x)
 }
 LSMP_DEV float rcp_w(float x) { return rcp_pos(x); }
 
-// Whether every lane's row a X(-st) + b X + c X(+st) of a cyclic reduction has lost
-// its neighbours: with |a|, |c| <= tol |b| leaving them out changes X by at most
-// 2 tol max |X|, half an ulp of the largest (FP32 a quarter).  The couplings square with
-// each step (0.55^K per interface of K rows on smooth data), so the later steps
-// are seldom needed.
-LSMP_DEV bool all_uncoupled(double a, double b, double c)
+// Lane l - 1's and lane l + 1's value (wave_shr:1, wave_shl:1); the first and
+// the last lane keep their own.
+template <int CTRL> LSMP_DEV float lane_shift(float v)
 {
-    const double t = fabs(b) * 0x1p-54;
-    return __all(fabs(a) <= t && fabs(c) <= t);
+    const int i = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false));
 }
-LSMP_DEV bool all_uncoupled(float a, float b, float c)
+template <int CTRL> LSMP_DEV double lane_shift(double v)
 {
-    const float t = fabsf(b) * 0x1p-26f;
-    return __all(fabsf(a) <= t && fabsf(c) <= t);
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
+}
+template <typename T> LSMP_DEV T from_left(T v) { return lane_shift<0x138>(v); }
+template <typename T> LSMP_DEV T from_right(T v) { return lane_shift<0x130>(v); }
+
+// X of a tridiagonal system a X(-1) + b X + c X(+1) = d, one row a lane of groups of
+// LANES (a = 0 in a group's first lane, c = 0 in its last), by parallel cyclic
+// reduction.  A row divided by its b is handed to the neighbours as three
+// values; a lane whose neighbour lies outside has a (c) = 0 by then and may read
+// any finite row.  The couplings square with every step (0.55^K to begin with for
+// interfaces K CRWENO rows apart on smooth data): once |a|, |c| <= TOL in every
+// lane, leaving them out changes X by at most 2 TOL max |X| (half an ulp; FP32 a
+// quarter), and the remaining steps are left out.
+template <int LANES, typename T> LSMP_DEV T pcr_solve(T a, T b, T c, T d)
+{
+    constexpr T TOL = sizeof(T) == 8 ? T(0x1p-54) : T(0x1p-26);
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int st = 1; st < LANES; st <<= 1) {
+        const T r = rcp_pos(b);
+        a *= r;
+        c *= r;
+        d *= r;
+        if (__all(fabs(a) <= TOL && fabs(c) <= TOL)) return d;
+        T am, cm, dm, ap, cq, dq;
+        if (st == 1) {
+            am = from_left(a); cm = from_left(c); dm = from_left(d);
+            ap = from_right(a); cq = from_right(c); dq = from_right(d);
+        } else {
+            const int lm = lane - st, lp = lane + st;   // (modulo 64)
+            am = __shfl(a, lm, 64); cm = __shfl(c, lm, 64); dm = __shfl(d, lm, 64);
+            ap = __shfl(a, lp, 64); cq = __shfl(c, lp, 64); dq = __shfl(d, lp, 64);
+        }
+        b = (T(1) - cm * a) - ap * c;
+        d = (d - dm * a) - dq * c;
+        a = -am * a;
+        c = -cq * c;
+    }
+    return d * rcp_pos(b);
 }
 
 // sqrt of x >= 0 from the hardware reciprocal square root (good to about 6e-8)

@@ -512,8 +512,11 @@ __global__ __launch_bounds__(256) void k_adv_pair_x(const T *__restrict__ phi, c
 // goes to scratch memory.  Same rows as the reference's (an f row is the g
 // row of the mirrored stencil with A and C exchanged); the solve differs from
 // one Thomas sweep only in rounding.  In MODE 2 the in-place update is safe:
-// a line's cells are read by its own wave only, all before the reduction.
-
+// a line's cells are read by its own wave only, all before the reduction.  Bound
+// by the latency of its chain at such sizes: the boundary faces come from cells
+// already loaded, what the pass updates is loaded during the reduction (200^2
+// advection 104 -> 90 us; before, with divisions in the reduction, two more rounds of loads
+// for the faces and a load per cell updated).
 template <typename T, int MODE, int STAGE, int KR, bool TUBE>
 __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ vel, T *R, T *L1, T *L2,
                                                    int nlines, int n, int lw, long ostride, long istride,
@@ -535,22 +538,24 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
     const size_t base = (size_t)(line / lw) * (size_t)ostride + (size_t)(line % lw) * (size_t)istride;
     const T inv_dd = T(1) / dd;
     auto at = [&](int c) -> size_t { return base + (size_t)clampi(c - 1, 0, n - 1) * (size_t)estride; };
-    auto emit = [&](int c, T t1, T t2) {   // cell c of the line
-        const size_t a = at(c);
+    // what the pass updates: R, phi, L1 and L2 of cells lo .. lo + KR
+    T Ro[KR + 1], Pv[KR + 1], l1[KR + 1], l2[KR + 1];
+    auto emit = [&](int j, T t1, T t2) {   // cell lo + j of the line
+        const size_t a = at(lo + j);
         if (MODE == 0) {
             R[a] = t1 + t2;
         } else if (MODE == 1) {
-            R[a] = (R[a] + t1) + t2;
+            R[a] = (Ro[j] + t1) + t2;
         } else if (!TUBE || tm.in(a)) {
-            const T r = (R[a] + t1) + t2, Pv = phi[a];
+            const T r = (Ro[j] + t1) + t2;
             if (STAGE == 1) {
                 L1[a] = r;
-                phi[a] = Pv + r * dt;
+                phi[a] = Pv[j] + r * dt;
             } else if (STAGE == 2) {
                 L2[a] = r;
-                phi[a] = Pv + (T(-3) * L1[a] + r) / T(4) * dt;
+                phi[a] = Pv[j] + (T(-3) * l1[j] + r) / T(4) * dt;
             } else {
-                phi[a] = Pv + (-L1[a] - L2[a] + T(8) * r) / T(12) * dt;
+                phi[a] = Pv[j] + (-l1[j] - l2[j] + T(8) * r) / T(12) * dt;
             }
         }
     };
@@ -565,6 +570,7 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
     T fl[KR + 6];
 #pragma unroll
     for (int t = 0; t < KR + 6; ++t) fl[t] = flux(lo - 2 + t);
+    const T fe[3] = {flux(n - 2), flux(n - 1), flux(n)};
     auto coeffs = [&](int j, T &A, T &B, T &C, T &S) {   // row lo + j
         const T x0 = isf ? fl[j + 5] : fl[j], x1 = isf ? fl[j + 4] : fl[j + 1], x2 = isf ? fl[j + 3] : fl[j + 2];
         const T x3 = isf ? fl[j + 2] : fl[j + 3], x4 = isf ? fl[j + 1] : fl[j + 4];
@@ -573,20 +579,11 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
         A = isf ? Cg : Ag;
         C = isf ? Ag : Cg;
     };
-    // boundary faces of this system, where a lane needs them
+    // boundary faces of this system, where a lane needs them: cells -2 .. 3, the
+    // clamped ones being cell 1, and cells n-2 .. n+3
     T bc0 = T(0), bcN = T(0);
-    if (s == 0) {
-        T v[6];
-#pragma unroll
-        for (int t = 0; t < 6; ++t) v[t] = flux(-2 + t);
-        bc0 = isf ? wenojs_f(v[1], v[2], v[3], v[4], v[5]) : wenojs_g(v[0], v[1], v[2], v[3], v[4]);
-    }
-    if (active && last) {
-        T v[6];
-#pragma unroll
-        for (int t = 0; t < 6; ++t) v[t] = flux(n - 2 + t);
-        bcN = isf ? wenojs_f(v[1], v[2], v[3], v[4], v[5]) : wenojs_g(v[0], v[1], v[2], v[3], v[4]);
-    }
+    if (s == 0) bc0 = isf ? wenojs_f(fl[0], fl[1], fl[2], fl[3], fl[4]) : wenojs_g(fl[0], fl[0], fl[1], fl[2], fl[3]);
+    if (active && last) bcN = isf ? wenojs_f(fe[1], fe[2], fe[2], fe[2], fe[2]) : wenojs_g(fe[0], fe[1], fe[2], fe[2], fe[2]);
 
     // local sweep: X_i = d'_i + e'_i L - c'_i X_{i+1}; the row after the last
     // (j == nrow) is the interface row of a lane that has one
@@ -654,24 +651,17 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
             rc = T(0);
         }
     }
-    // parallel cyclic reduction over the 32 lanes of the half
+    if (MODE != 0 && !isf) {   // on their way during the reduction
 #pragma unroll
-    for (int st = 1; st < 32; st <<= 1) {
-        const bool hasm = s - st >= 0, hasp = s + st < 32;
-        const int lm = hasm ? lane - st : lane, lp = hasp ? lane + st : lane;
-        T am = __shfl(ra, lm, 64), bm = __shfl(rb, lm, 64), cm = __shfl(rc, lm, 64), dm = __shfl(rd, lm, 64);
-        T ap = __shfl(ra, lp, 64), bp = __shfl(rb, lp, 64), cq = __shfl(rc, lp, 64), dq = __shfl(rd, lp, 64);
-        if (!hasm) { am = T(0); bm = T(1); cm = T(0); dm = T(0); }
-        if (!hasp) { ap = T(0); bp = T(1); cq = T(0); dq = T(0); }
-        const T k1 = ra / bm, k2 = rc / bp;
-        const T na = -am * k1, nc = -cq * k2;
-        const T nb = rb - cm * k1 - ap * k2, nd = rd - dm * k1 - dq * k2;
-        ra = na;
-        rb = nb;
-        rc = nc;
-        rd = nd;
+        for (int j = 0; j <= KR; ++j) {
+            const size_t a = at(lo + j);
+            Ro[j] = R[a];
+            if (MODE == 2) Pv[j] = phi[a];
+            if (MODE == 2 && STAGE > 1) l1[j] = L1[a];
+            if (MODE == 2 && STAGE > 2) l2[j] = L2[a];
+        }
     }
-    const T Xb = rd / rb;
+    const T Xb = pcr_solve<32>(ra, rb, rc, rd);
     const T Xprev = __shfl(Xb, (lane - 1) & 63, 64);
     const T Lv = s == 0 ? bc0 : Xprev;
     const T Rv = last ? bcN : Xb;
@@ -684,14 +674,14 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
             const T xn = dp[j] + ep[j] * Lv - cp[j] * x;
             const T t = (xn - x) * inv_dd;
             const T t2 = __shfl_xor(t, 32, 64);
-            if (!isf) emit(lo + j + 1, t, t2);
+            if (!isf) emit(j + 1, t, t2);
             x = xn;
         }
     }
     {
         const T t = (Lv - x) * inv_dd;
         const T t2 = __shfl_xor(t, 32, 64);
-        if (!isf && active) emit(lo, t, t2);
+        if (!isf && active) emit(0, t, t2);
     }
 }
 

@@ -13,22 +13,6 @@ namespace lsmp {
 
 namespace {
 
-// Lane l - 1's and lane l + 1's value (wave_shr:1, wave_shl:1); the first and
-// the last lane keep their own.
-template <int CTRL> LSMP_DEV float lane_shift(float v)
-{
-    const int i = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false));
-}
-template <int CTRL> LSMP_DEV double lane_shift(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false),
-                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
-}
-template <typename T> LSMP_DEV T from_left(T v) { return lane_shift<0x138>(v); }
-template <typename T> LSMP_DEV T from_right(T v) { return lane_shift<0x130>(v); }
-
 // cells a wave finishes of its 64 columns: a WENO-HJ face takes its lanes l - 2
 // to l + 3, the slopes of a cell two faces, lambda the cells beside it
 constexpr int r2_margin(int btn) { return btn ? 4 : 3; }
