@@ -316,22 +316,28 @@ template <typename T> LSMP_DEV T hj_h(T s) { return fma(T(0.609375) * s, s, T(1.
 // 6 qA qB, and Q the same with A and B, e1 and e2 exchanged.  FP64 takes both
 // reciprocals from one (the product of the two denominators stays within
 // [1e-58, 1e28]); FP32 denominators stay within [1e-28, 1e13].
-template <typename T> LSMP_DEV void weno_hj_face(T sa, T sb, T sc, T sd, T hb, T hc, T e1, T e2, T &P, T &Q)
+template <typename T> struct HjFace {
+    T dp, dm, yp, ym;   // P = yp / dp, Q = ym / dm
+};
+template <typename T> LSMP_DEV HjFace<T> weno_hj_parts(T sa, T sb, T sc, T sd, T hb, T hc, T e1, T e2)
 {
     const T tA = fma(T(-1.375), sc, sd), tJ = fma(T(-0.625), sc, sb), tB = fma(T(-1.375), sb, sa);
     const T qA = sq(fma(tA, tA, hc)), qJ = sq(fma(tJ, tJ, hc)), qB = sq(fma(tB, tB, hb));
     const T pJB = qJ * qB, pAJ = qA * qJ, pAB = qA * qB;
     const T w = fma(T(6), pAB, pAJ + pJB);
-    const T dp = fma(T(2), pAJ, w), dm = fma(T(2), pJB, w);
     const T u1 = pJB * e1, u2 = pAJ * e2, t = u1 + u2;
-    const T yp = fma(T(2), t, u2), ym = fma(T(2), t, u1);
+    return {fma(T(2), pAJ, w), fma(T(2), pJB, w), fma(T(2), t, u2), fma(T(2), t, u1)};
+}
+template <typename T> LSMP_DEV void weno_hj_face(T sa, T sb, T sc, T sd, T hb, T hc, T e1, T e2, T &P, T &Q)
+{
+    const HjFace<T> f = weno_hj_parts(sa, sb, sc, sd, hb, hc, e1, e2);
     if constexpr (sizeof(T) == 8) {
-        const T r = rcp_w(dp * dm);
-        P = (dm * r) * yp;
-        Q = (dp * r) * ym;
+        const T r = rcp_w(f.dp * f.dm);
+        P = (f.dm * r) * f.yp;
+        Q = (f.dp * r) * f.ym;
     } else {
-        P = rcp_w(dp) * yp;
-        Q = rcp_w(dm) * ym;
+        P = rcp_w(f.dp) * f.yp;
+        Q = rcp_w(f.dm) * f.ym;
     }
 }
 
@@ -339,6 +345,30 @@ template <typename T> LSMP_DEV void weno_hj_face(T sa, T sb, T sc, T sd, T hb, T
 template <typename T> LSMP_DEV T hj_base(T c, T p1, T s0, T s1)
 {
     return fma(T(-2), s0, fma(T(6), p1 - c, -s1));
+}
+
+// D+ and D- times 6 d of one cell from phi(m-3 .. m+3), its two faces formed for it alone
+template <typename T>
+LSMP_DEV void weno_hj_cell(T m3, T m2, T m1, T c, T p1, T p2, T p3, T &dp6, T &dm6)
+{
+    const T sa = m3 - T(2) * m2 + m1, sb = m2 - T(2) * m1 + c, sc = m1 - T(2) * c + p1, sd = c - T(2) * p1 + p2,
+            se = p1 - T(2) * p2 + p3;   // s(m-2) .. s(m+2)
+    const T e0 = sc - T(2) * sb + sa, e1 = sd - T(2) * sc + sb, e2 = se - T(2) * sd + sc;   // e(m-1), e(m), e(m+1)
+    const T hc = hj_h(sc);
+    const HjFace<T> l = weno_hj_parts(sa, sb, sc, sd, hj_h(sb), hc, e1, e0);   // face m-1/2, for its Q
+    const HjFace<T> r = weno_hj_parts(sb, sc, sd, se, hc, hj_h(sd), e2, e1);   // face m+1/2, for its P
+    T P, Q;
+    if constexpr (sizeof(T) == 8) {
+        const T i = rcp_w(r.dp * l.dm);
+        P = (l.dm * i) * r.yp;
+        Q = (r.dp * i) * l.ym;
+    } else {
+        P = rcp_w(r.dp) * r.yp;
+        Q = rcp_w(l.dm) * l.ym;
+    }
+    const T b6 = hj_base(c, p1, sc, sd);
+    dp6 = b6 + P;
+    dm6 = (b6 + e1) - Q;
 }
 
 // D+ and D- from the five second differences s_m = phi(m+1) - 2 phi(m) + phi(m-1),

@@ -516,7 +516,8 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
         tiles = c->tiles;
     }
     RedisBand<T> bd;
-    if (c->dim == 3 && btn == 1) {
+    const bool boxed = c->dim == 3 && btn == 1 && !tiles && redis3d_box_suits(c->nx, c->ny, c->nz);
+    if (c->dim == 3 && btn == 1 && !boxed) {
         if (!c->rb_list) {
             if (alloc(&c->rb_gr, 3 * c->ncell * c->esz) || alloc((void **)&c->rb_list, c->ncell * sizeof(unsigned)) ||
                 alloc((void **)&c->rb_count, 2 * sizeof(unsigned)))
@@ -540,10 +541,14 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
             c->rset = (c->rset + 1) % 3;
             const RedisStep step = {c->rset, launched + q == 0};
             if (c->dim == 3) {
-                // stages 1..3: every cell (lambda = 0), then the band cells (lambda)
+                // stages 1..3: every cell (lambda = 0), then the band cells (lambda), or both in one
                 const T *in[3] = {cur, b, cc};
                 T *outp[3] = {b, cc, b};
                 for (int sg = 0; sg < 3; ++sg) {
+                    if (boxed) {
+                        KT(c, "redis_stage", (launch_redis3d_box<T>(c->st, sg + 1, in[sg], outp[sg], cur, S0, ra, ctl, step)));
+                        continue;
+                    }
                     if (btn == 1) {
                         bd.count = c->rb_count + c->rb_par;
                         bd.next = c->rb_count + (1 - c->rb_par);

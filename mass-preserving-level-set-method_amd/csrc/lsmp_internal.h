@@ -192,6 +192,12 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
                     bool band, RedisStep step);
 template <typename T>
 void launch_combine_markers(hipStream_t st, const T *m1, const T *m2, T *phi, size_t n, unsigned *flag);
+// the whole stage of a small 3D grid, lambda included (lsmp_redis_box.hip), and
+// the grids that it suits
+bool redis3d_box_suits(int nx, int ny, int nz);
+template <typename T>
+void launch_redis3d_box(hipStream_t st, int stage, const T *phi, T *phi_out, const T *phi0, const T *S0,
+                        const RedisArgs &ra, unsigned long long *ctl, RedisStep step);
 template <typename T>
 void launch_redis2d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out, const T *phi0, const T *S0,
                     const RedisArgs &ra, unsigned long long *ctl, RedisStep step);
