@@ -11,6 +11,12 @@ constexpr int CSEG = 16;   // rows per CCD checkpoint segment
 // every line of a direction goes through the partitioned (one wave or 32
 // lanes per line) solves up to these counts
 constexpr int PART_MAX_LINES_X = 32768, PART_MAX_LINES_STRIDED = 4096;
+// the CCD solve's count for y and z lines (x lines have none).  The nine solves of
+// the energy integrals, one lane per line, then with 32 lanes along x only, then
+// along y and z as well: 96^3 497, 393, 273 us; 160x96x128 663, 456, 372 (FP32 611,
+// -, 271); 192^3 (36,864 lines) 1003, 835, 799 (FP32 889, 680, 565); 256^3 1546,
+// 1380, 1583 (FP32 1272, 1038, 1061); 400x400x30 (160,000 z lines) 1358, 860, 937.
+constexpr int PART_MAX_CCD_STRIDED = 40960;
 constexpr int KCC = 17;   // CCD rows per lane at most (9 up to 284 cells, 17 up to 540 with 32 lanes per line, 1084 with 64)
 
 // listed band lines solved with 32 lanes per line up to these counts (x lines

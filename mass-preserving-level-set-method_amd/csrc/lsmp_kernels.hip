@@ -1833,9 +1833,8 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
             hipLaunchKernelGGL((k_ccd_seg<T, D, F, false>), g, b, 0, st, phi, coef, scr, out, dxv, dyv, gr,      \
                                partial, nlines, n, lw, ostride, istride, estride, ca, lines);                  \
     } while (0)
-    // few lines (the 2D grids, or the lines crossing the band): 32 lanes per
-    // line instead of one
-    const int part_max = !lines ? PART_MAX_LINES_STRIDED : dir == 0 ? PART_MAX_LISTED_X : PART_MAX_LISTED_STRIDED;
+    // x lines, and y and z lines that are few or listed: 32 lanes per line instead of one
+    const int part_max = dir == 0 ? PART_MAX_LISTED_X : lines ? PART_MAX_LISTED_STRIDED : PART_MAX_CCD_STRIDED;
     // lines of up to 540 cells: 32 lanes per line; up to 1084 cells: 64
     const bool part32 = n + 4 <= 32 * KCC;
     const bool part = nlines <= part_max && n + 4 <= 64 * KCC;
