@@ -461,11 +461,19 @@ constexpr unsigned BAND_GRID = 1024;
 // tail of the last round counts (192^3: 238 us, 246 with 16, 274 with 32) and
 // 16 from three rounds of 16 (256^3: 534 us, 550 with 8, 536 with 32), beyond
 // which the three planes of run-up per march cost less than they save.
-static int stage_planes(unsigned tiles, int nz)
+//
+// FP32 holds twice the workgroups, so its marches are cut to two thousand, but
+// not below three planes: 131x77x101 55.0 -> 51.2 us per pseudo-step, 128^3
+// 68.5 -> 65.7, 96^3 47.0 with four or three planes and 49.5 with two.
+static int stage_planes(unsigned tiles, int nz, bool fp32)
 {
     constexpr int ROUND = 1024;
-    const int blocks = std::max(1, ROUND / (int)tiles);   // blocks in z that fit one round
-    const int one = std::max(1, (nz + blocks - 1) / blocks);
+    auto fit = [&](int groups) {   // planes of the shortest marches that make so many workgroups
+        const int blocks = std::max(1, groups / (int)tiles);
+        return std::max(1, (nz + blocks - 1) / blocks);
+    };
+    int one = fit(ROUND);
+    if (fp32) one = std::min(one, std::max(3, fit(2 * ROUND)));
     if (one <= 8) return one;
     return (size_t)tiles * nb_of(nz, RKC) >= (size_t)3 * ROUND ? RKC : 8;
 }
@@ -476,7 +484,7 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
                     bool band, RedisStep step)
 {
     // the narrow band (tiles) marches RKC_NB planes per workgroup
-    const int kc = tiles ? RKC_NB : stage_planes(nb_of(ra.nx, R3X) * nb_of(ra.ny, R3Y), ra.nz);
+    const int kc = tiles ? RKC_NB : stage_planes(nb_of(ra.nx, R3X) * nb_of(ra.ny, R3Y), ra.nz, sizeof(T) == 4);
     const dim3 g(nb_of(ra.nx, R3X), nb_of(ra.ny, R3Y), nb_of(ra.nz, kc));
 #define LSMP_R3(S, B)                                                                                          \
     do {                                                                                                       \
