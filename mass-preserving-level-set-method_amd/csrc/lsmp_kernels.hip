@@ -1854,13 +1854,22 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
     const bool part9 = n + 4 <= 32 * 9;
     // two lines per wave (one with 64 lanes per line), four waves per block
     const dim3 gp(nblk(nlines, part32 ? 8 : 4));
+    // The table in LDS where it takes at most 64 KiB, and up to nearly all of it
+    // where the launch gives a CU no more than two workgroups anyway: lines of 1,024
+    // cells read it from memory row by row in 650 us per correction at 1,024^2
+    // (FP64), from LDS in 301.
+    const bool plds = lds || (tab <= 150 * 1024 && gp.x <= 512);
+    const size_t pshm = plds ? tab : 0;
 #define LSMP_CCDQ(D, F, KC, LPL)                                                                               \
     do {                                                                                                       \
-        if (lds)                                                                                               \
-            hipLaunchKernelGGL((k_ccd_part<T, D, F, true, KC, LPL>), gp, b, shm, st, phi, coef, out, dxv, dyv,   \
-                               gr, partial, nlines, n, lw, ostride, istride, estride, ca, lines);              \
-        else                                                                                                   \
-            hipLaunchKernelGGL((k_ccd_part<T, D, F, false, KC, LPL>), gp, b, 0, st, phi, coef, out, dxv, dyv,    \
+        if (plds) {                                                                                            \
+            if (pshm > 65536)                                                                                  \
+                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ccd_part<T, D, F, true, KC, LPL>), \
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)pshm);              \
+            hipLaunchKernelGGL((k_ccd_part<T, D, F, true, KC, LPL>), gp, b, pshm, st, phi, coef, out, dxv,     \
+                               dyv, gr, partial, nlines, n, lw, ostride, istride, estride, ca, lines);         \
+        } else                                                                                                 \
+            hipLaunchKernelGGL((k_ccd_part<T, D, F, false, KC, LPL>), gp, b, 0, st, phi, coef, out, dxv, dyv,  \
                                gr, partial, nlines, n, lw, ostride, istride, estride, ca, lines);              \
     } while (0)
 #define LSMP_CCDP(D, F)                                                                                        \

@@ -1,5 +1,6 @@
 """The CCD solve on both sides of the rule that gives a line 32 lanes or one
-(40,960 lines along y or z; x lines always 32): the energy integrals, which
+(40,960 lines along y or z; x lines always 32), and of the one that keeps a large
+coefficient table in LDS (512 workgroups): the energy integrals, which
 solve every line of three fields, to 1e-12 of the oracle's, and the mass
 correction on every line against the one on band lines."""
 import numpy as np
@@ -15,6 +16,8 @@ CASES = [
     dict(nx=200, ny=8, nz=204, dim=3),   # 40,800 y lines
     dict(nx=200, ny=8, nz=205, dim=3),   # 41,000
     dict(nx=11, ny=210, nz=200, dim=3),  # 42,000 x lines
+    dict(nx=700, ny=40, nz=40, dim=3),   # a table of 73 KB in LDS: 400 workgroups
+    dict(nx=700, ny=52, nz=40, dim=3),   # and in memory: 520
 ]
 
 
