@@ -163,7 +163,7 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
 #pragma unroll
         for (int t = 0; t < KR + 6; ++t) fl[t] = flux(lo - 2 + t);
         auto coeffs = [&](int j, T &A, T &B, T &C, T &S) {   // row lo + j
-            crweno_g_row_fast(fl[j], fl[j + 1], fl[j + 2], fl[j + 3], fl[j + 4], A, B, C, S);
+            crweno_row<T, TUBE>(fl[j], fl[j + 1], fl[j + 2], fl[j + 3], fl[j + 4], A, B, C, S);
         };
         // boundary faces at the system's start and end
         const T bc0 = sbc[l][isf ? 2 : 0], bcN = sbc[l][isf ? 3 : 1];
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
                 rc = T(0);
             }
         }
-        const T Xb = pcr_solve<SL>(ra, rb, rc, rd);
+        const T Xb = adv_exact<T, TUBE>() ? pcr_solve_full<SL, false>(ra, rb, rc, rd) : pcr_solve<SL>(ra, rb, rc, rd);
         const T Xprev = __shfl(Xb, (lane - 1) & 63, 64);
         const T Lv = s == 0 ? bc0 : Xprev;
         const T Rv = last ? bcN : Xb;
@@ -305,8 +305,8 @@ void launch_adv_tile(hipStream_t st, int mode, int stage, T *phi, const T *vel, 
                      const TubeMask &tm)
 {
     const int rs = adv_tile_row_slots(n);
-    const bool tube = tm.fx != nullptr;
-    const bool h4 = n <= 32 * 4 + 1;   // half a wave per system and four rows a lane suffice
+    const bool tube = lines != nullptr;   // the narrow band's lines, whose stage pass has the mask tm
+    const bool h4 = n <= 32 * 4 + 1 && !(tube && sizeof(T) == 4);   // half a wave per system and four rows a lane suffice
     const bool k4 = n <= 64 * 4 + 1;   // else a wave per system and four, or eight (up to 513 cells)
     // lines of 514..1025 cells: sixteen rows per lane, four lines per workgroup
     const bool k16 = n > 64 * 8 + 1;
@@ -331,12 +331,8 @@ void launch_adv_tile(hipStream_t st, int mode, int stage, T *phi, const T *vel, 
 #define LSMP_TILE(M, S)                                                                                        \
     do {                                                                                                       \
         if (k16) LSMP_TILEK(M, S, 16, 64, false, 4, 8);                                                        \
-        else if constexpr (M == 2) {                                                                           \
-            if (tube) LSMP_TILET(M, S, true);                                                                  \
-            else LSMP_TILET(M, S, false);                                                                      \
-        } else {                                                                                               \
-            LSMP_TILET(M, S, false);                                                                           \
-        }                                                                                                      \
+        else if (tube) LSMP_TILET(M, S, true);                                                                 \
+        else LSMP_TILET(M, S, false);                                                                          \
     } while (0)
     if (mode == 0) LSMP_TILE(0, 0);
     else if (mode == 1) LSMP_TILE(1, 1);

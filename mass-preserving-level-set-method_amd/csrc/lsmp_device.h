@@ -193,6 +193,29 @@ template <int LANES, typename T> LSMP_DEV T pcr_solve(T a, T b, T c, T d)
     return d * rcp_pos(b);
 }
 
+// The same by every step of the reduction, four values a row (adv_exact): with the
+// neighbours' reciprocals (DIV false) or divisions by them.
+template <int LANES, bool DIV, typename T> LSMP_DEV T pcr_solve_full(T ra, T rb, T rc, T rd)
+{
+    const int lane = threadIdx.x & 63, s = lane & (LANES - 1);
+#pragma unroll
+    for (int st = 1; st < LANES; st <<= 1) {
+        const bool hasm = s - st >= 0, hasp = s + st < LANES;
+        const int lm = hasm ? lane - st : lane, lp = hasp ? lane + st : lane;
+        const T ib = DIV ? rb : rcp_w(rb);
+        const T am = __shfl(ra, lm, 64), im = __shfl(ib, lm, 64), cm = __shfl(rc, lm, 64), dm = __shfl(rd, lm, 64);
+        const T ap = __shfl(ra, lp, 64), ip = __shfl(ib, lp, 64), cq = __shfl(rc, lp, 64), dq = __shfl(rd, lp, 64);
+        const T k1 = !hasm ? T(0) : DIV ? ra / im : ra * im, k2 = !hasp ? T(0) : DIV ? rc / ip : rc * ip;
+        const T na = -am * k1, nc = -cq * k2;
+        const T nb = rb - cm * k1 - ap * k2, nd = rd - dm * k1 - dq * k2;
+        ra = na;
+        rb = nb;
+        rc = nc;
+        rd = nd;
+    }
+    return DIV ? rd / rb : rd * rcp_w(rb);
+}
+
 // sqrt of x >= 0 from the hardware reciprocal square root (good to about 6e-8)
 // and one Newton step: good to about 5e-15 of sqrt(x); exactly 0 at x = 0.
 LSMP_DEV double sqrt_w(double x)
@@ -256,6 +279,34 @@ LSMP_DEV void crweno_g_row_fast(T g0, T g1, T g2, T g3, T g4, T &A, T &B, T &C, 
     B = w1 + T(2) * (w2 + w3);
     C = w3;
     S = (w1 * g1 + (T(5) * (w1 + w2) + w3) * g2 + (w2 + T(5) * w3) * g3) * T(0.5);
+}
+
+// The normalised row itself, for the narrow band in FP32 (adv_exact).
+LSMP_DEV void crweno_g_row_unit(float g0, float g1, float g2, float g3, float g4, float &A, float &B, float &C,
+                                float &S)
+{
+    float b1 = 13.0f * sq(g0 - 2.0f * g1 + g2) + 3.0f * sq(g0 - 4.0f * g1 + 3.0f * g2);
+    float b2 = 13.0f * sq(g1 - 2.0f * g2 + g3) + 3.0f * sq(g1 - g3);
+    float b3 = 13.0f * sq(g2 - 2.0f * g3 + g4) + 3.0f * sq(3.0f * g2 - 4.0f * g3 + g4);
+    float w1, w2, w3;
+    crweno_weights_fast(b1, b2, b3, w1, w2, w3);
+    const float third = float(1.0 / 3.0), sixth = float(1.0 / 6.0);
+    A = (2.0f * w1 + w2) * third;
+    B = (w1 + 2.0f * (w2 + w3)) * third;
+    C = w3 * third;
+    S = (w1 * g1 + (5.0f * (w1 + w2) + w3) * g2 + (w2 + 5.0f * w3) * g3) * sixth;
+}
+
+// FP32 in the narrow band keeps the rounding of the full reduction over normalised
+// rows: the tube's tiles are the ones with a cell |phi| < W, and beyond its edge phi
+// is +-W up to the rounding of the advection, so that other roundings would move
+// the tube's edge by a tile here and there (0.2 dx in the tile's flat cells).
+template <typename T, bool NB> constexpr bool adv_exact() { return NB && sizeof(T) == 4; }
+template <typename T, bool NB>
+LSMP_DEV void crweno_row(T g0, T g1, T g2, T g3, T g4, T &A, T &B, T &C, T &S)
+{
+    if constexpr (adv_exact<T, NB>()) crweno_g_row_unit(g0, g1, g2, g3, g4, A, B, C, S);
+    else crweno_g_row_fast(g0, g1, g2, g3, g4, A, B, C, S);
 }
 
 // WENO-HJ correction term (level_set_rk3_redis.f90:456-471).

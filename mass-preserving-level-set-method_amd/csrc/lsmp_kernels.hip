@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
         const T x0 = isf ? fl[j + 5] : fl[j], x1 = isf ? fl[j + 4] : fl[j + 1], x2 = isf ? fl[j + 3] : fl[j + 2];
         const T x3 = isf ? fl[j + 2] : fl[j + 3], x4 = isf ? fl[j + 1] : fl[j + 4];
         T Ag, Cg;
-        crweno_g_row_fast(x0, x1, x2, x3, x4, Ag, B, Cg, S);
+        crweno_row<T, TUBE>(x0, x1, x2, x3, x4, Ag, B, Cg, S);
         A = isf ? Cg : Ag;
         C = isf ? Ag : Cg;
     };
@@ -661,7 +661,7 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
             if (MODE == 2 && STAGE > 2) l2[j] = L2[a];
         }
     }
-    const T Xb = pcr_solve<32>(ra, rb, rc, rd);
+    const T Xb = adv_exact<T, TUBE>() ? pcr_solve_full<32, true>(ra, rb, rc, rd) : pcr_solve<32>(ra, rb, rc, rd);
     const T Xprev = __shfl(Xb, (lane - 1) & 63, 64);
     const T Lv = s == 0 ? bc0 : Xprev;
     const T Rv = last ? bcN : Xb;
@@ -1716,7 +1716,7 @@ void launch_adv_pass(hipStream_t st, int dir, int mode, int stage, T *phi, const
     const size_t threads = (size_t)((nlines + 31) / 32) * 64;       // two lanes per line (x)
     const size_t threads4 = (size_t)((nlines + 15) / 16) * 64;      // four lanes per line (y, z)
     const dim3 g((unsigned)((threads + 255) / 256)), g4((unsigned)((threads4 + 255) / 256)), b(256);
-    // the tube mask exists in separate instantiations of the stage kernels
+    // listed lines (the narrow band's) exist in separate instantiations, with the mask in the stage pass
     const bool tube = tm.fx != nullptr;
 #define LSMP_ADVK(M, S, TB)                                                                                     \
     hipLaunchKernelGGL((k_adv_twist<T, M, S, TB>), g4, b, 0, st, phi, vel, R, L1, L2, scr, nlines, n, lw, ostride, \
@@ -1737,15 +1737,10 @@ void launch_adv_pass(hipStream_t st, int dir, int mode, int stage, T *phi, const
                        istride, estride, dd, dt, lines, tm)
 #define LSMP_PART(M, S)                                                                                       \
     do {                                                                                                      \
-        if constexpr (M == 2) {                                                                               \
-            if (part8 && tube) LSMP_PARTK(M, S, 8, true);                                                     \
-            else if (part8) LSMP_PARTK(M, S, 8, false);                                                       \
-            else if (tube) LSMP_PARTK(M, S, PKX, true);                                                       \
-            else LSMP_PARTK(M, S, PKX, false);                                                                \
-        } else {                                                                                              \
-            if (part8) LSMP_PARTK(M, S, 8, false);                                                            \
-            else LSMP_PARTK(M, S, PKX, false);                                                                \
-        }                                                                                                     \
+        if (part8 && lines) LSMP_PARTK(M, S, 8, true);                                                        \
+        else if (part8) LSMP_PARTK(M, S, 8, false);                                                           \
+        else if (lines) LSMP_PARTK(M, S, PKX, true);                                                          \
+        else LSMP_PARTK(M, S, PKX, false);                                                                    \
     } while (0)
     if (mode == 0) {
         if (part) LSMP_PART(0, 0);

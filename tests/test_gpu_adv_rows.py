@@ -56,3 +56,23 @@ def test_advection_rows_fp32(case):
     diff = np.max(np.abs(boxes[0] - boxes[1]))
     print(f"{ids(case)} fp32: max diff {diff:.2e}", flush=True)
     assert diff <= 1e-5
+
+
+@pytest.mark.parametrize("case", [dict(nx=129, ny=97, nz=64, dim=3), dict(nx=40, ny=36, nz=45, dim=3),
+                                  dict(nx=258, ny=36, nz=130, dim=3)], ids=ids)
+@pytest.mark.parametrize("precision", [0, 1])
+def test_advection_rows_listed(case, precision):
+    """Every line listed (a narrow band wider than the domain) against the plain
+    pass: FP64 to the drop-in tolerance, FP32, whose listed lines take every
+    step of the reduction over normalised rows, to some roundings of the field."""
+    boxes = []
+    for band in (0.0, 1000.0):
+        o, s = pair(precision=precision, **case)
+        load_state(o, s, shape=2, perturb=True, field=2)
+        s.set_narrow_band(band)
+        s.rk3_advect()
+        boxes.append(s.download_phi())
+        s.close()
+    diff = np.max(np.abs(boxes[0] - boxes[1])) / np.max(np.abs(boxes[0]))
+    print(f"{ids(case)} precision {precision}: diff {diff:.2e}", flush=True)
+    assert diff <= (1e-5 if precision else TOL)
