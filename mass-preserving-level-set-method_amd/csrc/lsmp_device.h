@@ -398,6 +398,27 @@ template <typename T> LSMP_DEV T hj_base(T c, T p1, T s0, T s1)
     return fma(T(-2), s0, fma(T(6), p1 - c, -s1));
 }
 
+// The same face times 12 d with its indicators over shared squares, and the central
+// part times 12 d: FP32 in the narrow band (redis_exact) keeps these roundings, for
+// the reason given at adv_exact.
+LSMP_DEV void weno_hj_face12(float sa, float sb, float sc, float sd, float &plus, float &minus)
+{
+    const float eps = 1.0e-6f;
+    const float bb = sb * sb, cc = sc * sc;
+    const float fA = fma(40.0f, cc, fma(sd, fma(16.0f, sd, -44.0f * sc), eps));
+    const float fJ = fma(16.0f, bb, fma(sc, fma(16.0f, sc, -20.0f * sb), eps));
+    const float fB = fma(40.0f, bb, fma(sa, fma(16.0f, sa, -44.0f * sb), eps));
+    const float qA = sq(fA), qJ = sq(fJ), qB = sq(fB);
+    const float pJB = qJ * qB, pAJ = qA * qJ, pAB = qA * qB;
+    const float dp = fma(3.0f, fma(2.0f, pAB, pAJ), pJB), dm = fma(3.0f, fma(2.0f, pAB, pJB), pAJ);
+    const float e1 = sd - 2.0f * sc + sb, e2 = sc - 2.0f * sb + sa;
+    const float u1 = pJB * e1, u2 = pAJ * e2;
+    plus = fma(rcp_w(dp), fma(4.0f, u1, 6.0f * u2), -e2);
+    minus = fma(rcp_w(dm), fma(4.0f, u2, 6.0f * u1), -e1);
+}
+LSMP_DEV float central12(float m2, float m1, float p1, float p2) { return fma(8.0f, p1 - m1, m2 - p2); }
+template <typename T, bool NB> constexpr bool redis_exact() { return NB && sizeof(T) == 4; }
+
 // D+ and D- times 6 d of one cell from phi(m-3 .. m+3), its two faces formed for it alone
 template <typename T>
 LSMP_DEV void weno_hj_cell(T m3, T m2, T m1, T c, T p1, T p2, T p3, T &dp6, T &dm6)

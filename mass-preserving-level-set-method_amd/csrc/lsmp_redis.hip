@@ -94,7 +94,8 @@ LSMP_DEV void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 }  // namespace
 
-template <typename T, int STAGE, int BTN>
+// NB: the narrow band (tiles), which keeps the roundings of redis_exact in FP32
+template <typename T, int STAGE, int BTN, bool NB>
 __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__restrict__ phi_out,
                                                 const T *__restrict__ phi0, const T *__restrict__ S0, RedisArgs ra,
                                                 unsigned long long *ctl, const unsigned char *__restrict__ tiles,
@@ -134,7 +135,14 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
             phi_out[(size_t)k * pl + c0] = phi[(size_t)k * pl + c0];
         return;
     }
-    const T kx = (T)(2.0 * ra.inv12dx), ky = (T)(2.0 * ra.inv12dy), kz = (T)(2.0 * ra.inv12dz);
+    constexpr bool EXACT = redis_exact<T, NB>();
+    // slopes are times 6 dx, ... until the Godunov sum (EXACT: scaled as they are formed)
+    const T kx = EXACT ? (T)ra.inv12dx : (T)(2.0 * ra.inv12dx), ky = EXACT ? (T)ra.inv12dy : (T)(2.0 * ra.inv12dy),
+            kz = EXACT ? (T)ra.inv12dz : (T)(2.0 * ra.inv12dz);
+    auto face = [&](T sa, T sb, T sc, T sd, T hb, T hc, T e1, T e2, T &P, T &Q) {
+        if constexpr (EXACT) weno_hj_face12(sa, sb, sc, sd, P, Q);
+        else weno_hj_face(sa, sb, sc, sd, hb, hc, e1, e2, P, Q);
+    };
     const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt;
     const int t = threadIdx.x;
     const int i0 = bx * R3X, j0 = by * R3Y, k0 = bz * kc;
@@ -178,6 +186,7 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     T halo2_cur = halo2 ? load_at(base(phi, k0), hcol2) : T(0);
     if (stopped()) return;
     T w0 = v[3], w1 = v[4], w2 = v[5], w3 = v[6];   // phi(p .. p+3)
+    T wm1 = v[2], wm2 = v[1];                       // phi(p-1), phi(p-2) (EXACT)
     // z: second differences s(p-1), s(p), s(p+1), h(s(p)), e(p) and Q of face
     // p - 1/2, carried from plane to plane
     T za, zb, zc, zhb, ze, zq;
@@ -190,7 +199,7 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         zhb = hj_h(zb);
         ze = zc - T(2) * zb + za;
         T unused;
-        weno_hj_face(s2, s1, s0, sp, hj_h(s1), zhb, ze, s0 - T(2) * s1 + s2, unused, zq);
+        face(s2, s1, s0, sp, hj_h(s1), zhb, ze, s0 - T(2) * s1 + s2, unused, zq);
     }
     if (BTN == 1 && t == 0) lcount = 0;   // read after the loop's first barrier
     T lerr = T(0);
@@ -218,9 +227,14 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
         const T zs_new = w1 - T(2) * w2 + w3;   // s(p + 2)
         const T zhc = hj_h(zc), ze_next = zs_new - T(2) * zc + zb;
         T zp, zq_next;
-        weno_hj_face(za, zb, zc, zs_new, zhb, zhc, ze_next, ze, zp, zq_next);
+        face(za, zb, zc, zs_new, zhb, zhc, ze_next, ze, zp, zq_next);
         const T bz6 = hj_base(w0, w1, zb, zc);
-        const T zs1 = bz6 + zp, zs2 = (bz6 + ze) - zq;
+        T zs1 = bz6 + zp, zs2 = (bz6 + ze) - zq;
+        if constexpr (EXACT) {
+            const T az = kz * central12(wm2, wm1, w1, w2);
+            zs1 = az + kz * zp;
+            zs2 = az - kz * zq;
+        }
         __syncthreads();
         // x face i+1/2: P of this cell, Q of cell i+1
         T xs1, xs2, ys1, ys2;
@@ -230,11 +244,15 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
             const T sa = m2 - T(2) * m1 + c, sb = m1 - T(2) * c + p1, sc = c - T(2) * p1 + p2, sd = p1 - T(2) * p2 + p3;
             const T e2 = sc - T(2) * sb + sa;
             T P, Q;
-            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
+            face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
             lds[MX + own + 1] = Q;
             const T b6 = hj_base(c, p1, sb, sc);
             xs1 = b6 + P;
             xs2 = b6 + e2;
+            if constexpr (EXACT) {
+                xs2 = kx * central12(m2, m1, p1, p2);
+                xs1 = xs2 + kx * P;
+            }
         }
         // y face j+1/2
         {
@@ -243,11 +261,15 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
             const T sa = m2 - T(2) * m1 + c, sb = m1 - T(2) * c + p1, sc = c - T(2) * p1 + p2, sd = p1 - T(2) * p2 + p3;
             const T e2 = sc - T(2) * sb + sa;
             T P, Q;
-            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
+            face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, e2, P, Q);
             lds[MY + own + P3X] = Q;
             const T b6 = hj_base(c, p1, sb, sc);
             ys1 = b6 + P;
             ys2 = b6 + e2;
+            if constexpr (EXACT) {
+                ys2 = ky * central12(m2, m1, p1, p2);
+                ys1 = ys2 + ky * P;
+            }
         }
         if (first_x || first_y) {
             asm("" : "+v"(f_off), "+v"(f_str), "+v"(f_dst));   // addresses formed here, not kept
@@ -257,13 +279,14 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
             const T sa = v0 - T(2) * v1 + v2, sb = v1 - T(2) * v2 + v3, sc = v2 - T(2) * v3 + v4,
                     sd = v3 - T(2) * v4 + v5;
             T P, Q;
-            weno_hj_face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, sc - T(2) * sb + sa, P, Q);
+            face(sa, sb, sc, sd, hj_h(sb), hj_h(sc), sd - T(2) * sc + sb, sc - T(2) * sb + sa, P, Q);
             lds[f_dst] = Q;
         }
         __syncthreads();
-        xs2 = xs2 - lds[MX + own];
-        ys2 = ys2 - lds[MY + own];
-        const T grad = godunov_sig(xs1, xs2, ys1, ys2, zs1, zs2, s0_cur, kx, ky, kz);
+        xs2 = EXACT ? xs2 - kx * lds[MX + own] : xs2 - lds[MX + own];
+        ys2 = EXACT ? ys2 - ky * lds[MY + own] : ys2 - lds[MY + own];
+        const T grad = EXACT ? godunov_sig(xs1, xs2, ys1, ys2, zs1, zs2, s0_cur, T(1), T(1), T(1))
+                             : godunov_sig(xs1, xs2, ys1, ys2, zs1, zs2, s0_cur, kx, ky, kz);
         // lambda = 0: final off the band, replaced by k_redis3d_band on it
         const T l = s0_cur * grad - s0_cur;
         const T pn = rk_stage<T, STAGE>(w0, p0_cur, l, rdt);
@@ -301,6 +324,8 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
                         (unsigned short)((p - k0) * NT + t);
             }
         }
+        wm2 = wm1;
+        wm1 = w0;
         w0 = w1;
         w1 = w2;
         w2 = w3;
@@ -489,8 +514,8 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
 #define LSMP_R3(S, B)                                                                                          \
     do {                                                                                                       \
         if (!band)                                                                                             \
-            hipLaunchKernelGGL((k_redis3d<T, S, B>), g, dim3(NT), 0, st, phi, phi_out, phi0, S0, ra, ctl,      \
-                               tiles, bd.f, bd.list, bd.count, kc, step);                                           \
+            hipLaunchKernelGGL((tiles ? &k_redis3d<T, S, B, true> : &k_redis3d<T, S, B, false>), g, dim3(NT), 0, st, \
+                               phi, phi_out, phi0, S0, ra, ctl, tiles, bd.f, bd.list, bd.count, kc, step);         \
         else if (B == 1)                                                                                       \
             hipLaunchKernelGGL((k_redis3d_band<T, S>), dim3(BAND_GRID), dim3(NT), 0, st, phi, phi_out, phi0,   \
                                S0, ra, ctl, bd.f, bd.list, bd.count, bd.next, step);                                \
