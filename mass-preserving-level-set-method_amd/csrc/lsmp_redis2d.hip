@@ -50,8 +50,10 @@ __global__ __launch_bounds__(64 * R2_WAVES) void k_redis2d(const T *__restrict__
     const T inv_w = (T)ra.inv_ls_wid, rdt = (T)ra.rdt;
     const int lane = threadIdx.x & 63, waves = (int)(blockDim.x >> 6);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int i = (int)blockIdx.x * r2_cols(BTN) - MARGIN + lane;
-    const int top = (int)blockIdx.y * (waves * R - 2 * BTN) - BTN;   // the workgroup's rows
+    // column strips fastest, in one grid dimension (no bound on nx or ny)
+    const unsigned strips = (unsigned)(nx + r2_cols(BTN) - 1) / (unsigned)r2_cols(BTN);
+    const int i = (int)(blockIdx.x % strips) * r2_cols(BTN) - MARGIN + lane;
+    const int top = (int)(blockIdx.x / strips) * (waves * R - 2 * BTN) - BTN;   // the workgroup's rows
     const int ja = top + wave * R;                                   // the wave's
     const int jo0 = BTN ? std::max(top + 1, 0) : top, jo1 = std::min(top + waves * R - BTN, ny);   // rows to finish
     const bool own = lane >= MARGIN && lane < 64 - MARGIN && i < nx;
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(64 * R2_WAVES) void k_redis2d(const T *__restrict__
 #pragma unroll
         for (int k = 0; k < R; ++k) qv[k] = (phi0 + (size_t)clampi(ja + k, 0, ny - 1) * nx)[ic];
     // the pseudo-time loop has stopped
-    if (STAGE == 1 ? redis_begin_step(ctl, step, (blockIdx.x | blockIdx.y) == 0) : ctl[1] != 0) return;
+    if (STAGE == 1 ? redis_begin_step(ctl, step, blockIdx.x == 0) : ctl[1] != 0) return;
     double lerr = 0.0;
     T a[R], b[R], g[R], c2[R], c3[R], d[R];   // sums of s2 and s3, |grad|, s2, s3, delta
     bool any[R];                              // the row has a band cell
@@ -151,7 +153,7 @@ __global__ __launch_bounds__(64 * R2_WAVES) void k_redis2d(const T *__restrict__
     }
     if (STAGE == 3) {
         const double m = block_max(lerr);
-        if (threadIdx.x == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, step, blockIdx.y * gridDim.x + blockIdx.x), m);
+        if (threadIdx.x == 0 && m > 0.0) atomic_max_nonneg(ctl_slot(ctl, step, blockIdx.x), m);
     }
 }
 
@@ -167,15 +169,15 @@ void launch_redis2d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
     const size_t n = (size_t)ra.nx * ra.ny;
     const int rows = n <= ((size_t)1 << 17) ? 1 : 2, waves = btn && n > ((size_t)1 << 14) ? 8 : 4;
     const int per = waves * rows - 2 * btn;   // rows a workgroup finishes
-    const dim3 g((unsigned)((ra.nx + r2_cols(btn) - 1) / r2_cols(btn)), (unsigned)((ra.ny + per - 1) / per));
+    const unsigned g = (unsigned)((ra.nx + r2_cols(btn) - 1) / r2_cols(btn)) * (unsigned)((ra.ny + per - 1) / per);
     const size_t lds = btn ? (size_t)waves * 256 * sizeof(T) : 0;
 #define LSMP_R2(S, B)                                                                                              \
     {                                                                                                              \
         if (rows == 1)                                                                                             \
-            hipLaunchKernelGGL((k_redis2d<T, S, B, 1>), g, dim3(64 * waves), lds, st, phi, phi_out, phi0, S0, ra,  \
+            hipLaunchKernelGGL((k_redis2d<T, S, B, 1>), dim3(g), dim3(64 * waves), lds, st, phi, phi_out, phi0, S0, ra,  \
                                ctl, step);                                                                         \
         else                                                                                                       \
-            hipLaunchKernelGGL((k_redis2d<T, S, B, 2>), g, dim3(64 * waves), lds, st, phi, phi_out, phi0, S0, ra,  \
+            hipLaunchKernelGGL((k_redis2d<T, S, B, 2>), dim3(g), dim3(64 * waves), lds, st, phi, phi_out, phi0, S0, ra,  \
                                ctl, step);                                                                         \
     }
     if (btn) { if (stage == 1) LSMP_R2(1, 1) else if (stage == 2) LSMP_R2(2, 1) else LSMP_R2(3, 1) }
