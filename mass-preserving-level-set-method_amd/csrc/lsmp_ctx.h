@@ -40,7 +40,8 @@ struct lsmp_ctx {
     double *hbuf = nullptr;   // pinned readback
     char *hstage = nullptr;   // pinned, two halves of hstage_rows rows: fields read out
     size_t hstage_rows = 0;
-    int npartial = 0;
+    int npartial = 0;         // blocks of a reduction over the cells at most
+    long nsums = 0;           // block sums that partial has room for
     int mass_hint = 2;               // iterations the last mass correction took
     int band_lines = 1;              // mass correction on band lines: 0 never, 1 where it pays, 2 always
     unsigned char *lflag = nullptr;  // band flags of the x, y, z lines (band_flag_bytes)

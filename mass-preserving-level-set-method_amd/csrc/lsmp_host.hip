@@ -615,6 +615,7 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
     // most 540 cells.  Elsewhere every line already goes through the 32-lane
     // solve, or the one-lane solve of long lines gains nothing from fewer lanes.
     const int ns[3] = {c->nx, c->ny, c->nz};
+    const long nfin = (long)(c->ncell / (size_t)ns[dfin]);   // lines of the final pass
     bool pays = c->dim == 3;
     size_t maxl = 0;
     for (int d = 0; d < c->dim; ++d) {
@@ -636,11 +637,15 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
         for (int d = 0; d < 3; ++d) c->last_lines[d] = nlst[d];
         const unsigned char *ffin =
             c->lflag + band_flag_offset(dfin, (size_t)c->ny * c->nz, (size_t)c->nx * c->nz);
+        if (hsum_blocks(ns[dfin], nfin) > c->nsums) return LSMP_E_INVALID;
         // the unlisted lines have delta = 0 on every cell, so the correction
         // leaves them as they are: their mass and volume are summed once
         KT(c, "line_hsums", (launch_line_hsums<T>(c->st, dfin, phi, ffin, c->nx, c->ny, c->nz, ca, c->partial,
                                                   &nfixed)));
     }
+    // the final pass's block sums, before anything writes them
+    if (nfixed + ccd_plan(dfin, ns[dfin], lst[dfin] ? nlst[dfin] : nfin, lst[dfin] != nullptr).blocks > c->nsums)
+        return LSMP_E_INVALID;
     double *psolve = c->partial + (size_t)3 * nfixed;
     // Iterations are queued ahead: as many as the last correction took (two to
     // start with), then one at a time; the stop test is taken on the device and
@@ -669,7 +674,6 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
                                                    c->ny, c->nz, it, &nblk, lst[1], nlst[1])));
             }
             nblk += nfixed;
-            if (nblk > c->npartial) return LSMP_E_INVALID;
             const MassArgs ma = {imass, iter, c->fp32 ? 1 : 0, c->scal, c->hbuf};
             if (!lst[dfin] && nblk <= MASS_FUSE_MAX && c->ncell <= MASS_FUSE_CELLS) {
                 KT(c, "mass_update", (launch_mass_update<T>(c->st, phi, (const T *)c->gr, c->ncell, (T)c->p.ls_wid,
@@ -677,7 +681,7 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
                 continue;
             }
             KT(c, "finalize", (launch_finalize3(c->st, c->partial, nblk, ma)));
-            const int nup = lst[dfin] ? nlst[dfin] : (int)(c->ncell / (size_t)ns[dfin]);   // no list: every line
+            const int nup = lst[dfin] ? nlst[dfin] : (int)nfin;   // no list: every line
             KT(c, "mass_update", (launch_mass_update_lines<T>(c->st, dfin, phi, (const T *)c->gr, (T)c->p.ls_wid,
                                                               c->scal, iter, lst[dfin], nup, c->nx, c->ny, c->nz)));
         }
@@ -1008,12 +1012,13 @@ int lsmp_init(const lsmp_params *params, lsmp_handle *out)
             return fail(LSMP_E_HIP);
         }
     }
-    // partial sums: one slot per block of the last CCD pass (a solve with up to
-    // 8 lines per block, then the unlisted lines' sums) or reduction kernel
+    // partial sums: a slot per block of a reduction kernel or of the mass
+    // correction's final pass and unlisted lines
     size_t maxlines = 0;
     for (int d = 1; d < c->dim; ++d) maxlines = std::max(maxlines, c->ncell / (size_t)ns[d]);
     c->npartial = (int)std::max<size_t>(1024, (maxlines + 7) / 8 + LINE_SEGMENTS * ((maxlines + 255) / 256));
-    if (alloc((void **)&c->partial, (size_t)3 * c->npartial * sizeof(double))) return fail(LSMP_E_HIP);
+    c->nsums = std::max((long)c->npartial, mass_sums(c->dim, c->nx, c->ny, c->nz));
+    if (alloc((void **)&c->partial, (size_t)3 * c->nsums * sizeof(double))) return fail(LSMP_E_HIP);
     if (alloc((void **)&c->scal, SCAL_WORDS * sizeof(double))) return fail(LSMP_E_HIP);
     if (alloc((void **)&c->u64, 4 * sizeof(unsigned long long))) return fail(LSMP_E_HIP);
     if (hipHostMalloc((void **)&c->hbuf, 16 * sizeof(double), hipHostMallocDefault) != hipSuccess)

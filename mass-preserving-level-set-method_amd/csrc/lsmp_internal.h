@@ -4,31 +4,15 @@
 #include <hip/hip_runtime.h>
 #include <cstddef>
 
+#include "lsmp_ccd_plan.h"
+
 namespace lsmp {
 
 constexpr int CSEG = 16;   // rows per CCD checkpoint segment
 
-// every line of a direction goes through the partitioned (one wave or 32
-// lanes per line) solves up to these counts
+// the advection's partitioned solve (a wave per line) takes every line of a
+// direction up to these counts; the CCD solve's counts are in lsmp_ccd_plan.h
 constexpr int PART_MAX_LINES_X = 32768, PART_MAX_LINES_STRIDED = 4096;
-// the CCD solve's count for y and z lines (x lines have none).  The nine solves of
-// the energy integrals, one lane per line, then with 32 lanes along x only, then
-// along y and z as well: 96^3 497, 393, 273 us; 160x96x128 663, 456, 372 (FP32 611,
-// -, 271); 192^3 (36,864 lines) 1003, 835, 799 (FP32 889, 680, 565); 256^3 1546,
-// 1380, 1583 (FP32 1272, 1038, 1061); 400x400x30 (160,000 z lines) 1358, 860, 937.
-constexpr int PART_MAX_CCD_STRIDED = 40960;
-constexpr int KCC = 17;   // CCD rows per lane at most (9 up to 284 cells, 17 up to 540 with 32 lanes per line, 1084 with 64)
-
-// listed band lines solved with 32 lanes per line up to these counts (x lines
-// are contiguous; y and z lines are strided, and 32 lanes on one of them read
-// 32 separate cache lines per row)
-#ifndef LSMP_PART_LISTED_X
-#define LSMP_PART_LISTED_X (1 << 30)
-#endif
-#ifndef LSMP_PART_LISTED_STRIDED
-#define LSMP_PART_LISTED_STRIDED (1 << 30)
-#endif
-constexpr int PART_MAX_LISTED_X = LSMP_PART_LISTED_X, PART_MAX_LISTED_STRIDED = LSMP_PART_LISTED_STRIDED;
 
 // 3D reinitialisation tile: R3X x R3Y interior cells, one thread each (a
 // 4-wave workgroup); at most RKC planes per workgroup in z.
@@ -217,9 +201,7 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
                      const T *dxv, const T *dyv, T *gr, double *partial, int nx, int ny, int nz, const CcdArgs &ca,
                      int *nblocks_out, const int *lines = nullptr, int nlist = 0);
 // mass and volume partial sums of the lines of direction dir with lflag 0,
-// each line in up to LINE_SEGMENTS segments (one block of partial sums per 256
-// lines and segment)
-constexpr int LINE_SEGMENTS = 8;
+// each line in hsum_segments segments (hsum_blocks block sums)
 template <typename T>
 void launch_line_hsums(hipStream_t st, int dir, const T *phi, const unsigned char *lflag, int nx, int ny, int nz,
                        const CcdArgs &ca, double *partial, int *nblocks_out);

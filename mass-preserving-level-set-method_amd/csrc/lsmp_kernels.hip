@@ -1828,7 +1828,8 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
     const long ostride = dir == 0 ? 0 : dir == 1 ? (long)nx * ny : (long)nx;
     const long istride = dir == 0 ? (long)nx : 1;
     const long estride = dir == 0 ? 1 : dir == 1 ? (long)nx : (long)nx * ny;
-    const dim3 g(nblk(nlines, 256)), b(256);
+    const CcdPlan plan = ccd_plan(dir, n, nlines, lines != nullptr);
+    const dim3 g((unsigned)plan.blocks), b(256);
     const size_t tab = (size_t)13 * (n + 6) * sizeof(T);
     const bool lds = tab <= 64 * 1024;
     const size_t shm = lds ? tab : 0;
@@ -1841,19 +1842,15 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
             hipLaunchKernelGGL((k_ccd_seg<T, D, F, false>), g, b, 0, st, phi, coef, scr, out, dxv, dyv, gr,      \
                                partial, nlines, n, lw, ostride, istride, estride, ca, lines);                  \
     } while (0)
-    // x lines, and y and z lines that are few or listed: 32 lanes per line instead of one
-    const int part_max = dir == 0 ? PART_MAX_LISTED_X : lines ? PART_MAX_LISTED_STRIDED : PART_MAX_CCD_STRIDED;
-    // lines of up to 540 cells: 32 lanes per line; up to 1084 cells: 64
-    const bool part32 = n + 4 <= 32 * KCC;
-    const bool part = nlines <= part_max && n + 4 <= 64 * KCC;
+    // 32 lanes a line (two lines a wave) or 64 for lines of more than 540 cells,
+    // four waves a block; one lane a line for many or longer ones
+    const bool part32 = plan.lanes == 32, part = plan.lanes > 1;
     const bool part9 = n + 4 <= 32 * 9;
-    // two lines per wave (one with 64 lanes per line), four waves per block
-    const dim3 gp(nblk(nlines, part32 ? 8 : 4));
     // The table in LDS where it takes at most 64 KiB, and up to nearly all of it
     // where the launch gives a CU no more than two workgroups anyway: lines of 1,024
     // cells read it from memory row by row in 650 us per correction at 1,024^2
     // (FP64), from LDS in 301.
-    const bool plds = lds || (tab <= 150 * 1024 && gp.x <= 512);
+    const bool plds = lds || (tab <= 150 * 1024 && g.x <= 512);
     const size_t pshm = plds ? tab : 0;
 #define LSMP_CCDQ(D, F, KC, LPL)                                                                               \
     do {                                                                                                       \
@@ -1861,10 +1858,10 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
             if (pshm > 65536)                                                                                  \
                 (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ccd_part<T, D, F, true, KC, LPL>), \
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)pshm);              \
-            hipLaunchKernelGGL((k_ccd_part<T, D, F, true, KC, LPL>), gp, b, pshm, st, phi, coef, out, dxv,     \
+            hipLaunchKernelGGL((k_ccd_part<T, D, F, true, KC, LPL>), g, b, pshm, st, phi, coef, out, dxv,     \
                                dyv, gr, partial, nlines, n, lw, ostride, istride, estride, ca, lines);         \
         } else                                                                                                 \
-            hipLaunchKernelGGL((k_ccd_part<T, D, F, false, KC, LPL>), gp, b, 0, st, phi, coef, out, dxv, dyv,  \
+            hipLaunchKernelGGL((k_ccd_part<T, D, F, false, KC, LPL>), g, b, 0, st, phi, coef, out, dxv, dyv,  \
                                gr, partial, nlines, n, lw, ostride, istride, estride, ca, lines);              \
     } while (0)
 #define LSMP_CCDP(D, F)                                                                                        \
@@ -1882,7 +1879,7 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
         } else if (!final_pass) LSMP_CCD(3, false);
         else if (dim == 3) LSMP_CCD(3, true);
         else LSMP_CCD(2, true);
-        nbl = (int)(part ? gp.x : g.x);
+        nbl = (int)plan.blocks;
     }
 #undef LSMP_CCD
 #undef LSMP_CCDP
@@ -1900,8 +1897,7 @@ void launch_line_hsums(hipStream_t st, int dir, const T *phi, const unsigned cha
     const long ostride = dir == 0 ? 0 : dir == 1 ? (long)nx * ny : (long)nx;
     const long istride = dir == 0 ? (long)nx : 1;
     const long estride = dir == 0 ? 1 : dir == 1 ? (long)nx : (long)nx * ny;
-    // up to LINE_SEGMENTS segments of at least 32 cells per line
-    const int nseg = std::max(1, std::min(LINE_SEGMENTS, n / 32));
+    const int nseg = hsum_segments(n);
     const int seg = (n + nseg - 1) / nseg;
     const dim3 g(nblk(nall, 256), (unsigned)nseg);
     hipLaunchKernelGGL((k_line_hsums<T>), g, dim3(256), 0, st, phi, lflag, nall, n, lw, ostride, istride, estride,
