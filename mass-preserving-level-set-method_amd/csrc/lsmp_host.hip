@@ -535,7 +535,8 @@ int reinit(lsmp_ctx *c, int btn, double timestop, int max_iter, bool init_s0, do
     int &hint = c->redis_hint[btn];
     if (queued) *queued = 0;
     while (launched < budget) {
-        const int k = std::min(launched == 0 && hint > 0 ? std::min(hint, AHEAD) : CHUNK, budget - launched);
+        const int ahead = launched == 0 && hint > 0 ? std::min(hint, AHEAD) : CHUNK;
+        const int k = defer ? budget : std::min(ahead, budget - launched);   // deferred: this batch is the whole run
         for (int q = 0; q < k; ++q) {
             T *cur = (T *)c->phi, *b = (T *)c->phiB, *cc = (T *)c->phiC;
             c->rset = (c->rset + 1) % 3;
