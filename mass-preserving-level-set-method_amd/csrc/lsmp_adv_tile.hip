@@ -291,7 +291,7 @@ __global__ __launch_bounds__(TW * 64) void k_adv_tile(T *phi, const T *__restric
                 phi[a] = Pv[i] + r * dt;
             } else if (STAGE == 2) {
                 L2[a] = r;
-                phi[a] = Pv[i] + (T(-3) * l1[i] + r) / T(4) * dt;
+                phi[a] = Pv[i] + fma(T(-3), l1[i], r) / T(4) * dt;
             } else {
                 phi[a] = Pv[i] + (-l1[i] - l2[i] + T(8) * r) / T(12) * dt;
             }
@@ -305,7 +305,7 @@ void launch_adv_tile(hipStream_t st, int mode, int stage, T *phi, const T *vel, 
                      const TubeMask &tm)
 {
     const int rs = adv_tile_row_slots(n);
-    const bool tube = lines != nullptr;   // the narrow band's lines, whose stage pass has the mask tm
+    const bool tube = lines != nullptr;   // the narrow band's lines: the stage pass has the mask tm, FP32 adv_exact
     const bool h4 = n <= 32 * 4 + 1 && !(tube && sizeof(T) == 4);   // half a wave per system and four rows a lane suffice
     const bool k4 = n <= 64 * 4 + 1;   // else a wave per system and four, or eight (up to 513 cells)
     // lines of 514..1025 cells: sixteen rows per lane, four lines per workgroup
@@ -324,15 +324,19 @@ void launch_adv_tile(hipStream_t st, int mode, int stage, T *phi, const T *vel, 
     } while (0)
 #define LSMP_TILET(M, S, TB)                                                                                   \
     do {                                                                                                       \
-        if (h4) LSMP_TILEK(M, S, 4, 32, TB, 8, 4);                                                             \
+        if (k16) LSMP_TILEK(M, S, 16, 64, (TB && M != 2), 4, 8);   /* (its stage pass has no mask) */            \
+        else if (h4) LSMP_TILEK(M, S, 4, 32, TB, 8, 4);                                                        \
         else if (k4) LSMP_TILEK(M, S, 4, 64, TB, 8, 4);                                                        \
         else LSMP_TILEK(M, S, 8, 64, TB, 8, 4);                                                                \
     } while (0)
 #define LSMP_TILE(M, S)                                                                                        \
     do {                                                                                                       \
-        if (k16) LSMP_TILEK(M, S, 16, 64, false, 4, 8);                                                        \
-        else if (tube) LSMP_TILET(M, S, true);                                                                 \
-        else LSMP_TILET(M, S, false);                                                                          \
+        if constexpr (M == 2 || adv_exact<T, true>()) {                                                        \
+            if (tube) LSMP_TILET(M, S, true);                                                                  \
+            else LSMP_TILET(M, S, false);                                                                      \
+        } else {                                                                                               \
+            LSMP_TILET(M, S, false);                                                                           \
+        }                                                                                                      \
     } while (0)
     if (mode == 0) LSMP_TILE(0, 0);
     else if (mode == 1) LSMP_TILE(1, 1);

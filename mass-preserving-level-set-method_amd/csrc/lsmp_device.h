@@ -300,7 +300,8 @@ LSMP_DEV void crweno_g_row_unit(float g0, float g1, float g2, float g3, float g4
 // FP32 in the narrow band keeps the rounding of the full reduction over normalised
 // rows: the tube's tiles are the ones with a cell |phi| < W, and beyond its edge phi
 // is +-W up to the rounding of the advection, so that other roundings would move
-// the tube's edge by a tile here and there (0.2 dx in the tile's flat cells).
+// the tube's edge by a tile here and there (0.2 dx in the tile's flat cells).  Every
+// solve a line can take does so (tiles, a wave per line, paired, twisted).
 template <typename T, bool NB> constexpr bool adv_exact() { return NB && sizeof(T) == 4; }
 template <typename T, bool NB>
 LSMP_DEV void crweno_row(T g0, T g1, T g2, T g3, T g4, T &A, T &B, T &C, T &S)

@@ -74,6 +74,7 @@ constexpr int AXB = 8;
 template <typename T> struct TwistDepth { static constexpr int C = 8, B = 4; };
 template <> struct TwistDepth<double> { static constexpr int C = 4, B = 4; };
 
+// TUBE: the narrow band's lines (MODE 2: with its mask)
 template <typename T, int MODE, int STAGE, bool TUBE>
 __global__ __launch_bounds__(256) void k_adv_twist(T *phi, const T *__restrict__ vel, T *R, T *L1, T *L2,
                                                     T *__restrict__ scr, int nlines, int n, int lw, long ostride,
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(256) void k_adv_twist(T *phi, const T *__restrict__
         const T x0 = mir ? w[5] : w[0], x1 = mir ? w[4] : w[1], x2 = mir ? w[3] : w[2];
         const T x3 = mir ? w[2] : w[3], x4 = mir ? w[1] : w[4];
         T Ag, Cg;
-        crweno_g_row_fast(x0, x1, x2, x3, x4, Ag, B, Cg, S);
+        crweno_row<T, TUBE>(x0, x1, x2, x3, x4, Ag, B, Cg, S);
         A = mir ? Cg : Ag;
         C = mir ? Ag : Cg;
     };
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(256) void k_adv_twist(T *phi, const T *__restrict__
 // workgroup barriers are uniform.
 constexpr int XW = 16;
 
-template <typename T>
+template <typename T, bool NB>
 __global__ __launch_bounds__(256) void k_adv_pair_x(const T *__restrict__ phi, const T *__restrict__ vel,
                                                      T *__restrict__ R, T *__restrict__ scr, int nlines, int n,
                                                      T dd)
@@ -375,7 +376,7 @@ __global__ __launch_bounds__(256) void k_adv_pair_x(const T *__restrict__ phi, c
         const T x0 = isf ? w[5] : w[0], x1 = isf ? w[4] : w[1], x2 = isf ? w[3] : w[2];
         const T x3 = isf ? w[2] : w[3], x4 = isf ? w[1] : w[4];
         T Ag, Cg;
-        crweno_g_row_fast(x0, x1, x2, x3, x4, Ag, B, Cg, S);
+        crweno_row<T, NB>(x0, x1, x2, x3, x4, Ag, B, Cg, S);
         A = isf ? Cg : Ag;
         C = isf ? Ag : Cg;
     };
@@ -553,7 +554,7 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
                 phi[a] = Pv[j] + r * dt;
             } else if (STAGE == 2) {
                 L2[a] = r;
-                phi[a] = Pv[j] + (T(-3) * l1[j] + r) / T(4) * dt;
+                phi[a] = Pv[j] + fma(T(-3), l1[j], r) / T(4) * dt;   // (l1 comes from another block: no contraction there)
             } else {
                 phi[a] = Pv[j] + (-l1[j] - l2[j] + T(8) * r) / T(12) * dt;
             }
@@ -570,7 +571,6 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
     T fl[KR + 6];
 #pragma unroll
     for (int t = 0; t < KR + 6; ++t) fl[t] = flux(lo - 2 + t);
-    const T fe[3] = {flux(n - 2), flux(n - 1), flux(n)};
     auto coeffs = [&](int j, T &A, T &B, T &C, T &S) {   // row lo + j
         const T x0 = isf ? fl[j + 5] : fl[j], x1 = isf ? fl[j + 4] : fl[j + 1], x2 = isf ? fl[j + 3] : fl[j + 2];
         const T x3 = isf ? fl[j + 2] : fl[j + 3], x4 = isf ? fl[j + 1] : fl[j + 4];
@@ -579,11 +579,25 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
         A = isf ? Cg : Ag;
         C = isf ? Ag : Cg;
     };
-    // boundary faces of this system, where a lane needs them: cells -2 .. 3, the
-    // clamped ones being cell 1, and cells n-2 .. n+3
+    // boundary faces of this system, where a lane needs them, from cells -2 .. 3 and
+    // n-2 .. n+3 (the clamped ones being cells 1 and n)
     T bc0 = T(0), bcN = T(0);
-    if (s == 0) bc0 = isf ? wenojs_f(fl[0], fl[1], fl[2], fl[3], fl[4]) : wenojs_g(fl[0], fl[0], fl[1], fl[2], fl[3]);
-    if (active && last) bcN = isf ? wenojs_f(fe[1], fe[2], fe[2], fe[2], fe[2]) : wenojs_g(fe[0], fe[1], fe[2], fe[2], fe[2]);
+    if constexpr (adv_exact<T, TUBE>()) {   // from fluxes of their own, which are contracted into the sums
+        auto face = [&](int c) {
+            T v[6];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) v[t] = flux(c + t);
+            return isf ? wenojs_f(v[1], v[2], v[3], v[4], v[5]) : wenojs_g(v[0], v[1], v[2], v[3], v[4]);
+        };
+        if (s == 0) bc0 = face(-2);
+        if (active && last) bcN = face(n - 2);
+    } else {
+        const T fe[3] = {flux(n - 2), flux(n - 1), flux(n)};
+        if (s == 0)
+            bc0 = isf ? wenojs_f(fl[0], fl[1], fl[2], fl[3], fl[4]) : wenojs_g(fl[0], fl[0], fl[1], fl[2], fl[3]);
+        if (active && last)
+            bcN = isf ? wenojs_f(fe[1], fe[2], fe[2], fe[2], fe[2]) : wenojs_g(fe[0], fe[1], fe[2], fe[2], fe[2]);
+    }
 
     // local sweep: X_i = d'_i + e'_i L - c'_i X_{i+1}; the row after the last
     // (j == nrow) is the interface row of a lane that has one
@@ -1695,7 +1709,8 @@ void launch_adv_pass(hipStream_t st, int dir, int mode, int stage, T *phi, const
     // its loads being one line per lane, and at 256^3 the paired x kernel is
     // as fast (FP64) or faster (FP32 182 against 220 us).  Listed lines (the
     // narrow band) take it up to PART_MAX_LISTED_ADV strided lines.
-    int nlines = lines ? nlist : nall;
+    const bool nb = lines != nullptr;   // the narrow band
+    int nlines = nb ? nlist : nall;
     // many lines: the tiled solve reads and writes each field once, coalesced;
     // lines of 514..1025 cells (2D 1024^2) take its long-line form whatever
     // their count, since the paired and twisted kernels would give them one
@@ -1708,7 +1723,7 @@ void launch_adv_pass(hipStream_t st, int dir, int mode, int stage, T *phi, const
     }
     const bool part = n >= 34 && n <= 32 * PKX + 1 &&
                       nlines <= (dir == 0 ? PART_MAX_LINES_X : lines ? PART_MAX_LISTED_ADV : PART_MAX_LINES_STRIDED);
-    if (mode == 0 && !part && lines) {   // the paired x kernel takes every line
+    if (mode == 0 && !part && nb) {   // the paired x kernel takes every line
         lines = nullptr;
         nlines = nall;
     }
@@ -1716,15 +1731,15 @@ void launch_adv_pass(hipStream_t st, int dir, int mode, int stage, T *phi, const
     const size_t threads = (size_t)((nlines + 31) / 32) * 64;       // two lanes per line (x)
     const size_t threads4 = (size_t)((nlines + 15) / 16) * 64;      // four lanes per line (y, z)
     const dim3 g((unsigned)((threads + 255) / 256)), g4((unsigned)((threads4 + 255) / 256)), b(256);
-    // listed lines (the narrow band's) exist in separate instantiations, with the mask in the stage pass
-    const bool tube = tm.fx != nullptr;
+    // the narrow band's lines exist in separate instantiations where those differ:
+    // in the stage pass, which has the mask, and in FP32 (adv_exact)
 #define LSMP_ADVK(M, S, TB)                                                                                     \
     hipLaunchKernelGGL((k_adv_twist<T, M, S, TB>), g4, b, 0, st, phi, vel, R, L1, L2, scr, nlines, n, lw, ostride, \
                        istride, estride, dd, dt, lines, tm)
 #define LSMP_ADV(M, S)                                                                                          \
     do {                                                                                                        \
-        if constexpr (M == 2) {                                                                                 \
-            if (tube) LSMP_ADVK(M, S, true);                                                                    \
+        if constexpr (M == 2 || adv_exact<T, true>()) {                                                         \
+            if (nb) LSMP_ADVK(M, S, true);                                                                      \
             else LSMP_ADVK(M, S, false);                                                                        \
         } else {                                                                                                \
             LSMP_ADVK(M, S, false);                                                                             \
@@ -1735,16 +1750,25 @@ void launch_adv_pass(hipStream_t st, int dir, int mode, int stage, T *phi, const
 #define LSMP_PARTK(M, S, KR, TB)                                                                              \
     hipLaunchKernelGGL((k_adv_part<T, M, S, KR, TB>), gp, b, 0, st, phi, vel, R, L1, L2, nlines, n, lw, ostride, \
                        istride, estride, dd, dt, lines, tm)
+#define LSMP_PARTT(M, S, TB)                                                                                  \
+    do {                                                                                                      \
+        if (part8) LSMP_PARTK(M, S, 8, TB);                                                                   \
+        else LSMP_PARTK(M, S, PKX, TB);                                                                       \
+    } while (0)
 #define LSMP_PART(M, S)                                                                                       \
     do {                                                                                                      \
-        if (part8 && lines) LSMP_PARTK(M, S, 8, true);                                                        \
-        else if (part8) LSMP_PARTK(M, S, 8, false);                                                           \
-        else if (lines) LSMP_PARTK(M, S, PKX, true);                                                          \
-        else LSMP_PARTK(M, S, PKX, false);                                                                    \
+        if constexpr (M == 2 || adv_exact<T, true>()) {                                                       \
+            if (nb) LSMP_PARTT(M, S, true);                                                                   \
+            else LSMP_PARTT(M, S, false);                                                                     \
+        } else {                                                                                              \
+            LSMP_PARTT(M, S, false);                                                                          \
+        }                                                                                                     \
     } while (0)
     if (mode == 0) {
         if (part) LSMP_PART(0, 0);
-        else hipLaunchKernelGGL((k_adv_pair_x<T>), g, b, 0, st, phi, vel, R, scr, nlines, n, dd);
+        else if (nb && adv_exact<T, true>())
+            hipLaunchKernelGGL((k_adv_pair_x<T, adv_exact<T, true>()>), g, b, 0, st, phi, vel, R, scr, nlines, n, dd);
+        else hipLaunchKernelGGL((k_adv_pair_x<T, false>), g, b, 0, st, phi, vel, R, scr, nlines, n, dd);
     } else if (part) {
         if (mode == 1) LSMP_PART(1, 1);
         else if (stage == 1) LSMP_PART(2, 1);
@@ -1757,6 +1781,7 @@ void launch_adv_pass(hipStream_t st, int dir, int mode, int stage, T *phi, const
 #undef LSMP_ADV
 #undef LSMP_ADVK
 #undef LSMP_PART
+#undef LSMP_PARTT
 #undef LSMP_PARTK
 }
 
