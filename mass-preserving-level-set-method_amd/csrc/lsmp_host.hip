@@ -645,7 +645,8 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
                                                   &nfixed)));
     }
     // the final pass's block sums, before anything writes them
-    if (nfixed + ccd_plan(dfin, ns[dfin], lst[dfin] ? nlst[dfin] : nfin, lst[dfin] != nullptr).blocks > c->nsums)
+    if (nfixed + ccd_plan(dfin, ns[dfin], lst[dfin] ? nlst[dfin] : nfin, lst[dfin] != nullptr, c->esz).blocks >
+        c->nsums)
         return LSMP_E_INVALID;
     double *psolve = c->partial + (size_t)3 * nfixed;
     // Iterations are queued ahead: as many as the last correction took (two to
@@ -1018,7 +1019,7 @@ int lsmp_init(const lsmp_params *params, lsmp_handle *out)
     size_t maxlines = 0;
     for (int d = 1; d < c->dim; ++d) maxlines = std::max(maxlines, c->ncell / (size_t)ns[d]);
     c->npartial = (int)std::max<size_t>(1024, (maxlines + 7) / 8 + LINE_SEGMENTS * ((maxlines + 255) / 256));
-    c->nsums = std::max((long)c->npartial, mass_sums(c->dim, c->nx, c->ny, c->nz));
+    c->nsums = std::max((long)c->npartial, mass_sums(c->dim, c->nx, c->ny, c->nz, c->esz));
     if (alloc((void **)&c->partial, (size_t)3 * c->nsums * sizeof(double))) return fail(LSMP_E_HIP);
     if (alloc((void **)&c->scal, SCAL_WORDS * sizeof(double))) return fail(LSMP_E_HIP);
     if (alloc((void **)&c->u64, 4 * sizeof(unsigned long long))) return fail(LSMP_E_HIP);

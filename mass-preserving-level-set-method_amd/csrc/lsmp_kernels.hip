@@ -1853,7 +1853,7 @@ void launch_ccd_pass(hipStream_t st, int dir, int dim, bool final_pass, const T 
     const long ostride = dir == 0 ? 0 : dir == 1 ? (long)nx * ny : (long)nx;
     const long istride = dir == 0 ? (long)nx : 1;
     const long estride = dir == 0 ? 1 : dir == 1 ? (long)nx : (long)nx * ny;
-    const CcdPlan plan = ccd_plan(dir, n, nlines, lines != nullptr);
+    const CcdPlan plan = ccd_plan(dir, n, nlines, lines != nullptr, sizeof(T));
     const dim3 g((unsigned)plan.blocks), b(256);
     const size_t tab = (size_t)13 * (n + 6) * sizeof(T);
     const bool lds = tab <= 64 * 1024;

@@ -3,13 +3,13 @@
 #include "../../mass-preserving-level-set-method_amd/csrc/lsmp_ccd_plan.h"
 
 extern "C" {
-int hc_ccd_plan(int dir, int n, long nlines, int listed, long *blocks)
+int hc_ccd_plan(int dir, int n, long nlines, int listed, int esz, long *blocks)
 {
-    const lsmp::CcdPlan p = lsmp::ccd_plan(dir, n, nlines, listed != 0);
+    const lsmp::CcdPlan p = lsmp::ccd_plan(dir, n, nlines, listed != 0, (size_t)esz);
     *blocks = p.blocks;
     return p.lanes;
 }
 int hc_hsum_segments(int n) { return lsmp::hsum_segments(n); }
 long hc_hsum_blocks(int n, long nlines) { return lsmp::hsum_blocks(n, nlines); }
-long hc_mass_sums(int dim, int nx, int ny, int nz) { return lsmp::mass_sums(dim, nx, ny, nz); }
+long hc_mass_sums(int dim, int nx, int ny, int nz, int esz) { return lsmp::mass_sums(dim, nx, ny, nz, (size_t)esz); }
 }
