@@ -115,13 +115,13 @@ __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__
     const int nx = ra.nx, ny = ra.ny, nz = ra.nz;
     // tiles in x-fastest order, renumbered so that each XCD takes a contiguous
     // run of them: the x and y halos of a tile are then mostly in its XCD's L2
-    const int gx = (int)gridDim.x, gy = (int)gridDim.y;
-    const int tile_id = xcd_renumber((int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x),
-                                     gx * gy * (int)gridDim.z);
+    // (one grid dimension: the planes have no launch bound)
+    const int gx = (nx + R3X - 1) / R3X, gy = (ny + R3Y - 1) / R3Y;
+    const int tile_id = xcd_renumber((int)blockIdx.x, (int)gridDim.x);
     const int bx = tile_id % gx, by = (tile_id / gx) % gy, bz = tile_id / (gx * gy);
     // whether the pseudo-time loop has stopped: looked at once the run-up's loads
     // are on their way, before anything is written
-    const bool lead = (blockIdx.x | blockIdx.y | blockIdx.z) == 0;
+    const bool lead = blockIdx.x == 0;
     auto stopped = [&]() { return STAGE == 1 ? redis_begin_step(ctl, step, lead) : ctl[1] != 0; };
     // narrow band: a workgroup with no cell of the tube keeps its cells.  Stage
     // 1 writes the step's output buffer and stage 2 the one stage 3 reads, so
@@ -510,7 +510,7 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
 {
     // the narrow band (tiles) marches RKC_NB planes per workgroup
     const int kc = tiles ? RKC_NB : stage_planes(nb_of(ra.nx, R3X) * nb_of(ra.ny, R3Y), ra.nz, sizeof(T) == 4);
-    const dim3 g(nb_of(ra.nx, R3X), nb_of(ra.ny, R3Y), nb_of(ra.nz, kc));
+    const dim3 g(nb_of(ra.nx, R3X) * nb_of(ra.ny, R3Y) * nb_of(ra.nz, kc));
 #define LSMP_R3(S, B)                                                                                          \
     do {                                                                                                       \
         if (!band)                                                                                             \
