@@ -94,7 +94,8 @@ LSMP_DEV void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 }  // namespace
 
-// NB: the narrow band (tiles), which keeps the roundings of redis_exact in FP32
+// NB: the narrow band in FP32, which keeps the roundings of redis_exact (in FP64
+// the tiles are all there is to it)
 template <typename T, int STAGE, int BTN, bool NB>
 __global__ __launch_bounds__(NT) void k_redis3d(const T *__restrict__ phi, T *__restrict__ phi_out,
                                                 const T *__restrict__ phi0, const T *__restrict__ S0, RedisArgs ra,
@@ -514,8 +515,9 @@ void launch_redis3d(hipStream_t st, int stage, int btn, const T *phi, T *phi_out
 #define LSMP_R3(S, B)                                                                                          \
     do {                                                                                                       \
         if (!band)                                                                                             \
-            hipLaunchKernelGGL((tiles ? &k_redis3d<T, S, B, true> : &k_redis3d<T, S, B, false>), g, dim3(NT), 0, st, \
-                               phi, phi_out, phi0, S0, ra, ctl, tiles, bd.f, bd.list, bd.count, kc, step);         \
+            hipLaunchKernelGGL((tiles ? &k_redis3d<T, S, B, redis_exact<T, true>()> : &k_redis3d<T, S, B, false>), g, \
+                               dim3(NT), 0, st, phi, phi_out, phi0, S0, ra, ctl, tiles, bd.f, bd.list, bd.count, kc, \
+                               step);                                                                          \
         else if (B == 1)                                                                                       \
             hipLaunchKernelGGL((k_redis3d_band<T, S>), dim3(BAND_GRID), dim3(NT), 0, st, phi, phi_out, phi0,   \
                                S0, ra, ctl, bd.f, bd.list, bd.count, bd.next, step);                                \
