@@ -517,12 +517,15 @@ __global__ __launch_bounds__(256) void k_adv_pair_x(const T *__restrict__ phi, c
 // by the latency of its chain at such sizes: the boundary faces come from cells
 // already loaded, what the pass updates is loaded during the reduction (200^2
 // advection 104 -> 90 us; before, with divisions in the reduction, two more rounds of loads
-// for the faces and a load per cell updated).
+// for the faces and a load per cell updated).  Sixteen rows a lane leave no registers
+// for that: FP64 took up to 386 and ran one wave per SIMD (60x60x300, z 71 us against 57
+// without any of this).  There the pass loads each cell as it stores it (FP32 but
+// for MODE 1), and the registers are held to two waves per SIMD (FP32 three): 48 us,
+// 3000x500 y 67 -> 56 (FP32 56 -> 43).
 template <typename T, int MODE, int STAGE, int KR, bool TUBE>
-__global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ vel, T *R, T *L1, T *L2,
-                                                   int nlines, int n, int lw, long ostride, long istride,
-                                                   long estride, T dd, T dt, const int *__restrict__ lines,
-                                                   TubeMask tm)
+__global__ __launch_bounds__(256, KR > 8 ? (sizeof(T) == 4 ? 3 : 2) : 1)
+void k_adv_part(T *phi, const T *__restrict__ vel, T *R, T *L1, T *L2, int nlines, int n, int lw, long ostride,
+                long istride, long estride, T dd, T dt, const int *__restrict__ lines, TubeMask tm)
 {
     const int tid = xcd_block() * blockDim.x + threadIdx.x;
     const int wline = tid >> 6, lane = tid & 63;
@@ -539,24 +542,27 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
     const size_t base = (size_t)(line / lw) * (size_t)ostride + (size_t)(line % lw) * (size_t)istride;
     const T inv_dd = T(1) / dd;
     auto at = [&](int c) -> size_t { return base + (size_t)clampi(c - 1, 0, n - 1) * (size_t)estride; };
-    // what the pass updates: R, phi, L1 and L2 of cells lo .. lo + KR
-    T Ro[KR + 1], Pv[KR + 1], l1[KR + 1], l2[KR + 1];
+    // what the pass updates: R, phi, L1 and L2 of cells lo .. lo + KR, loaded ahead or as they are needed
+    constexpr bool AHEAD = KR <= 8 || (sizeof(T) == 4 && MODE == 1);
+    constexpr int NA = AHEAD ? KR + 1 : 1;
+    T Ro[NA], Pv[NA], l1[NA], l2[NA];
     auto emit = [&](int j, T t1, T t2) {   // cell lo + j of the line
         const size_t a = at(lo + j);
+        const int q = AHEAD ? j : 0;
         if (MODE == 0) {
             R[a] = t1 + t2;
         } else if (MODE == 1) {
-            R[a] = (Ro[j] + t1) + t2;
-        } else if (!TUBE || tm.in(a)) {
-            const T r = (Ro[j] + t1) + t2;
+            R[a] = ((AHEAD ? Ro[q] : R[a]) + t1) + t2;
+        } else if (!TUBE || tm.in(line % lw, line / lw, clampi(lo + j - 1, 0, n - 1))) {   // (a z line)
+            const T r = ((AHEAD ? Ro[q] : R[a]) + t1) + t2, P = AHEAD ? Pv[q] : phi[a];
             if (STAGE == 1) {
                 L1[a] = r;
-                phi[a] = Pv[j] + r * dt;
+                phi[a] = P + r * dt;
             } else if (STAGE == 2) {
                 L2[a] = r;
-                phi[a] = Pv[j] + fma(T(-3), l1[j], r) / T(4) * dt;   // (l1 comes from another block: no contraction there)
+                phi[a] = P + fma(T(-3), AHEAD ? l1[q] : L1[a], r) / T(4) * dt;   // (loaded in another block: no contraction there)
             } else {
-                phi[a] = Pv[j] + (-l1[j] - l2[j] + T(8) * r) / T(12) * dt;
+                phi[a] = P + (-(AHEAD ? l1[q] : L1[a]) - (AHEAD ? l2[q] : L2[a]) + T(8) * r) / T(12) * dt;
             }
         }
     };
@@ -582,15 +588,20 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
     // boundary faces of this system, where a lane needs them, from cells -2 .. 3 and
     // n-2 .. n+3 (the clamped ones being cells 1 and n)
     T bc0 = T(0), bcN = T(0);
-    if constexpr (adv_exact<T, TUBE>()) {   // from fluxes of their own, which are contracted into the sums
+    if constexpr (adv_exact<T, TUBE>()) {
+        // loaded here, so that their fluxes are contracted into the sums; both ends
+        // of the line in one branch (80^3 narrow band advection 210 -> 191 us)
         auto face = [&](int c) {
             T v[6];
 #pragma unroll
             for (int t = 0; t < 6; ++t) v[t] = flux(c + t);
             return isf ? wenojs_f(v[1], v[2], v[3], v[4], v[5]) : wenojs_g(v[0], v[1], v[2], v[3], v[4]);
         };
-        if (s == 0) bc0 = face(-2);
-        if (active && last) bcN = face(n - 2);
+        if (s == 0 || (active && last)) {   // (no lane is both: two rows a lane at least)
+            const T v = face(s == 0 ? -2 : n - 2);
+            if (s == 0) bc0 = v;
+            else bcN = v;
+        }
     } else {
         const T fe[3] = {flux(n - 2), flux(n - 1), flux(n)};
         if (s == 0)
@@ -665,9 +676,9 @@ __global__ __launch_bounds__(256) void k_adv_part(T *phi, const T *__restrict__ 
             rc = T(0);
         }
     }
-    if (MODE != 0 && !isf) {   // on their way during the reduction
+    if (AHEAD && MODE != 0 && !isf) {   // on their way during the reduction
 #pragma unroll
-        for (int j = 0; j <= KR; ++j) {
+        for (int j = 0; j < NA; ++j) {
             const size_t a = at(lo + j);
             Ro[j] = R[a];
             if (MODE == 2) Pv[j] = phi[a];
