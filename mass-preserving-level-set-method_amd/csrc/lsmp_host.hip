@@ -610,11 +610,13 @@ template <typename T> int mass_fix(lsmp_ctx *c, double imass, double *mass_out, 
     const int dfin = c->dim == 3 ? 2 : 1;   // direction of the final pass (its sums)
     for (int d = 0; d < 3; ++d) c->last_lines[d] = -1;
     int nfixed = 0;                         // partials of the unlisted lines, constant over the iterations
-    // Band lines pay where solving every line would take the one-lane kernel
-    // (more than PART_MAX_LINES_STRIDED lines in a direction) and the listed
-    // lines fit the 32-lane one: 3D grids from about 65^3 with lines of at
-    // most 540 cells.  Elsewhere every line already goes through the 32-lane
-    // solve, or the one-lane solve of long lines gains nothing from fewer lanes.
+    // Band lines pay on 3D grids from about 65^3 (more than PART_MAX_LINES_STRIDED
+    // lines in a direction) with lines of at most 540 cells: the passes over the
+    // flags and the unlisted lines cost 20 us, the lists leave out most of the
+    // solves.  us per correction of four or five iterations, every line and
+    // listed: 48^3 178, 188 (FP32 198, 218), 64^3 187, 186 (168, 180), 72^3 221, 192
+    // (186, 183), 96^3 388, 253 (298, 221), 128^3 657, 386 (437, 281), 256^3 2849, 1265
+    // (1796, 821).  Longer lines are listed on demand only (lsmp_set_band_lines).
     const int ns[3] = {c->nx, c->ny, c->nz};
     const long nfin = (long)(c->ncell / (size_t)ns[dfin]);   // lines of the final pass
     bool pays = c->dim == 3;

@@ -480,17 +480,22 @@ constexpr unsigned BAND_GRID = 1024;
 // nz planes.  A workgroup's march is a serial chain (1.1 us a plane with one
 // workgroup on a CU, 2.6 us with four), so a grid that leaves the device
 // idle is cut into shorter ones: the shortest that still fit one round of
-// resident workgroups (1,024, four per CU).  Per pseudo-step, FP64 (FP32),
-// with 32 planes always and with this rule: 32^3 161 -> 48 us (137 -> 36),
-// 96^3 167 -> 78 (140 -> 57), 128^3 176 -> 109 (150 -> 77), 131x77x101
-// 161 -> 83 (137 -> 65).  Grids of several rounds take 8 planes where the
-// tail of the last round counts (192^3: 238 us, 246 with 16, 274 with 32) and
-// 16 from three rounds of 16 (256^3: 534 us, 550 with 8, 536 with 32), beyond
-// which the three planes of run-up per march cost less than they save.
+// resident workgroups (1,024, four per CU).  us per pseudo-step with marches of
+// 1, 2, 3, 4, 6, 8 and 16 planes (the rule's in brackets), FP64:
+//   64^3        [50]  46   48   49   54   60   86
+//   96^3         78   68   67  [65]  70   72   87
+//   131x77x101   98   83   79   81  [81]  83  107
+//   128^3       131  111  107  101  103 [101] 111
+//   160^3       218  172  163  154  152 [151] 153
+//   192^3       328  262  242  226  220 [217] 220
+//   256^3       668  529  493  468  442  430 [416]
+// Grids of several rounds take 8 planes where the tail of the last round counts and
+// 16 from three rounds of 16, beyond which the three planes of run-up per march
+// cost less than they save.
 //
 // FP32 holds twice the workgroups, so its marches are cut to two thousand, but
-// not below three planes: 131x77x101 55.0 -> 51.2 us per pseudo-step, 128^3
-// 68.5 -> 65.7, 96^3 47.0 with four or three planes and 49.5 with two.
+// not below three planes: 96^3 62, 53, [52], 52, 55, 58, 76; 131x77x101 76, 65, [62],
+// 63, 66, 67, 88; 128^3 94, 79, 75, [73], 75, 74, 86.
 static int stage_planes(unsigned tiles, int nz, bool fp32)
 {
     constexpr int ROUND = 1024;
