@@ -12,6 +12,8 @@ CASES = [
     (dict(nx=60, ny=20, nz=73, dim=3), 0), (dict(nx=60, ny=20, nz=75, dim=3), 0),
     (dict(nx=60, ny=20, nz=112, dim=3), 1), (dict(nx=60, ny=20, nz=115, dim=3), 1),
     (dict(nx=125, ny=240, nz=128, dim=3), 0), (dict(nx=126, ny=240, nz=128, dim=3), 0),
+    # 42,000 x lines of 130 cells, which have no limit
+    (dict(nx=130, ny=210, nz=200, dim=3), 0),
 ]
 
 
